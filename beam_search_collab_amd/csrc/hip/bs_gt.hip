@@ -3,12 +3,12 @@
 // from HDF5 files, script/unpack.py:56-81); this is the one dense contraction near the
 // search path, so it runs on the matrix cores.
 //
-//   gt_norms    |b_j|^2 in fp32 and max_j |b_j|^2
-//   gt_select   32 queries x 32 rows per v_mfma_f32_32x32x2f32 step: a_j = |b_j|^2 - 2 q.b_j
-//               (fp32), the 128 smallest (a_j, j) per (query, row split) kept in HBM with a
-//               per-query threshold in registers and an LDS append buffer; each split
-//               publishes its 128th value per query (an upper bound of the query's 128th
-//               value over all rows) and filters by the least bound published
+//   gt_split    every row scaled by a power of two and split into two fp16 planes (h + l = the
+//               fp32 value to 2^-24 of it) in the matrix cores' operand layout, and |b_j|^2
+//               (fp64 sum, rounded once)
+//   gt_select   32 x 32 tiles of a_j = |b_j|^2 - 2 q.b_j from v_mfma_f32_32x32x16_f16, three
+//               products of the planes; the 128 smallest (a_j, j) per (query, row split) kept
+//               in HBM with a per-query threshold in registers and an LDS append buffer
 //   gt_refine   merge the splits' lists, exact fp64 distances of the 128 candidates summed
 //               in dimension order (the host bs_groundtruth's arithmetic), order by
 //               (distance, id), and a certificate: every other row j has
@@ -39,208 +39,569 @@ using bsw::readlane64;
 using bsw::wave_sync;
 
 constexpr uint32_t C = 128;           // candidates kept per (query, split)
-constexpr uint32_t BUF = 128;         // LDS append slots per query
+constexpr uint32_t BUF = 64;          // LDS append slots per query
 constexpr uint32_t FLUSH = BUF - 32;  // a buffer is merged once it holds this many keys
-constexpr uint32_t LDS_WAVE = 32 * BUF * 8 + 128 * 8 + 72 * 8;  // append buffers, merge scratch
+constexpr uint32_t PUB = 64;          // splits whose published values bound a query's C-th value
+constexpr uint32_t REFRESH = 16;      // tiles between two reads of the published values
+
+constexpr uint32_t TS = 36;           // floats per lane of the values staged for an append (16-byte aligned)
+
+// LDS of a gt_select wavefront of QB x 32 queries: append buffers, 32 lanes' values, key counts
+constexpr uint32_t lds_wave(int qb) { return static_cast<uint32_t>(qb) * 32 * (BUF * 8 + 4) + 32 * TS * 4; }
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
-__global__ void __launch_bounds__(256) gt_norms(const float* vecs, uint64_t n, uint32_t dim, uint32_t dstride,
-                                                float* bn, uint32_t* bmax_bits) {
-    const uint64_t j = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    float s = 0.0f;
-    if (j < n) {
-        const float* r = vecs + j * dstride;
-        for (uint32_t i = 0; i < dim; ++i) s = __builtin_fmaf(r[i], r[i], s);
-        bn[j] = s;
+// The power of two that brings a row's largest magnitude into [2^14, 2^15), below fp16's
+// 65504 (1 for an empty row or one with an infinity or NaN; at most 2^100, so that it and its
+// reciprocal are normal numbers).
+__device__ __forceinline__ float row_scale(float largest) {
+    const int e = static_cast<int>(__float_as_uint(largest) >> 23);  // biased exponent, 0 for 0 and subnormals
+    if (largest == 0.0f || e == 255) return 1.0f;
+    return __uint_as_float(static_cast<uint32_t>(std::min(141 - e, 100) + 127) << 23);
+}
+
+// the smaller of sc and the scale of a query with this largest magnitude (an empty query and
+// one with an infinity or NaN do not count: their products are 0, infinite or NaN at any scale)
+__device__ __forceinline__ float query_scale(float largest, float sc) {
+    return largest == 0.0f || largest == __builtin_inff() ? sc : fminf(sc, row_scale(largest));
+}
+
+// x (already scaled) as NP fp16 planes: each keeps the next 11 significant bits, rounded to
+// nearest, so two planes hold x to 2^-24 |x| and three hold it exactly.  What falls below
+// fp16's range is less than 2^-29 of the row's largest value.  A value that is infinite or NaN
+// leaves a NaN, which makes every product with it a survivor.
+template <int NP>
+__device__ __forceinline__ void split_value(float x, _Float16 (&p)[NP]) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+        p[i] = static_cast<_Float16>(x);
+        x = x - static_cast<float>(p[i]);
     }
-    s = bsw::wave_max(s);  // s >= 0, so the float order is the bit order
-    if (lane_id() == 0) atomicMax(bmax_bits, __float_as_uint(s));
+}
+
+// Two planes; three up to 32 dimensions, where an fp32 chain rounds so few times that the
+// planes' 2^-24 would be the larger error (the matrix time is the smaller part there).
+constexpr int planes(int KC) { return KC <= 2 ? 3 : 2; }
+
+// Operand layout of v_mfma_f32_32x32x16_f16 (A and B alike): lane l holds row (column) l % 32
+// and 8 of the 16 dimensions, 8 (l / 32) .. + 7.  Both operands are filled by the same rule, so
+// the order of the dimensions inside the instruction does not matter.  A fragment is one
+// operand register set of the wavefront, 64 x 16 bytes; the base's fragments are stored
+// [tile of 32 rows][16 dimensions][plane], so a wavefront's load of one is 1 KB contiguous.
+//
+// Rows row0 .. row0 + m of the base, a wavefront per tile.  Memory bound (4 bytes read and 4
+// written per value).  The norm is summed in fp64 (one rounding).  meta[j] = (|b_j|^2, -2 over
+// the row's scale).
+template <int KC>
+__global__ void __launch_bounds__(256) gt_split(const float* vecs, uint64_t row0, uint64_t m, uint32_t dstride,
+                                                uint4* frag, float2* meta, uint32_t* bmax_bits) {
+    constexpr int NP = planes(KC);
+    const uint32_t lane = lane_id(), half = lane >> 5, l32 = lane & 31u;
+    const uint64_t tiles = (m + 31) / 32, step = static_cast<uint64_t>(gridDim.x) * 4;
+    float mx = 0.0f;
+    for (uint64_t t = static_cast<uint64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6); t < tiles; t += step) {
+        const uint64_t j = std::min<uint64_t>(t * 32 + l32, m - 1);  // the last tile's spare rows repeat its last one
+        const float* row = vecs + (row0 + j) * dstride;
+        f32x4 x[KC][2];
+#pragma unroll
+        for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {  // loads of columns past the row read column 0
+                const uint32_t d = 16u * kc + 8u * half + 4u * q;
+                x[kc][q] = *reinterpret_cast<const f32x4*>(row + (d < dstride ? d : 0u));
+            }
+        double s = 0.0;
+        float big = 0.0f;
+#pragma unroll
+        for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                if (16u * kc + 8u * half + 4u * q >= dstride) x[kc][q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float v = x[kc][q][i];
+                    big = fabsf(v) > big || v != v ? (v != v ? __builtin_inff() : fabsf(v)) : big;
+                    s += static_cast<double>(v) * static_cast<double>(v);
+                }
+            }
+        big = fmaxf(big, bsw::xor_lane_f<32>(big));
+        const float sc = row_scale(big);
+#pragma unroll
+        for (int kc = 0; kc < KC; ++kc) {
+            f16x8 p[NP];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                _Float16 v[NP];
+                split_value<NP>(x[kc][i / 4][i % 4] * sc, v);
+#pragma unroll
+                for (int q = 0; q < NP; ++q) p[q][i] = v[q];
+            }
+            uint4* f = frag + ((t * KC + kc) * NP) * 64 + lane;
+#pragma unroll
+            for (int q = 0; q < NP; ++q) f[q * 64] = __builtin_bit_cast(uint4, p[q]);
+        }
+        s += __longlong_as_double(static_cast<long long>(
+            bsw::xor_lane64<32>(static_cast<uint64_t>(__double_as_longlong(s)))));
+        const float nj = static_cast<float>(s);
+        if (half == 0) meta[t * 32 + l32] = make_float2(nj, -2.0f / sc);
+        mx = fmaxf(mx, nj);
+    }
+    mx = bsw::wave_max(mx);  // mx >= 0, so the float order is the bit order
+    if (lane == 0) atomicMax(bmax_bits, __float_as_uint(mx));
 }
 
 // D (32 x 32) element of accumulator register r in this lane: row (query) 8(r/4) + 4(lane/32)
-// + r%4, column (base row) lane % 32 -- the v_mfma_f32_32x32x2f32 output layout, checked by
-// bs_debug_mfma32.
+// + r%4, column (base row) lane % 32 -- the 32 x 32 output layout of the f32 and f16
+// instructions alike, checked by bs_debug_mfma32.
 __device__ __forceinline__ uint32_t acc_row(int r, uint32_t half) {
     return 8u * static_cast<uint32_t>(r / 4) + 4u * half + static_cast<uint32_t>(r % 4);
 }
 
-template <int KP>
-__global__ void __launch_bounds__(256) gt_select(const float* vecs, uint32_t dstride, const float* bn, uint64_t n,
-                                                 const float* queries, uint32_t dim, uint64_t nq, uint32_t nsplit,
-                                                 uint64_t split_rows, uint64_t* topc, uint32_t* tshare) {
-    constexpr int H = KP / 2;  // dimensions per lane half
+__device__ __forceinline__ float tau_of(uint32_t key_hi) {
+    return key_hi == ~0u ? __builtin_inff() : bsd::key_dist(static_cast<uint64_t>(key_hi) << 32);
+}
+
+// the C smallest of the sorted beam and the sorted list whose keys are given in reverse (rev[r]
+// of lane l = key C - 1 - (64 r + l)): the elementwise minimum is bitonic and holds exactly
+// them, seven steps sort it
+__device__ __forceinline__ void merge_lists(uint64_t (&beam)[2], const uint64_t (&rev)[2]) {
+#pragma unroll
+    for (int r = 0; r < 2; ++r) beam[r] = rev[r] < beam[r] ? rev[r] : beam[r];
+    const uint64_t x = beam[0], y = beam[1];
+    beam[0] = y < x ? y : x;
+    beam[1] = y < x ? x : y;
+#pragma unroll
+    for (int i = 5; i >= 0; --i) {
+        const uint32_t step = 1u << i;
+        const uint64_t lower = bsd::lanes_bit_clear(step);
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            const uint64_t p = bsw::xor_lane64_rt(beam[r], step);
+            beam[r] = bsw::lane_in(~(lower ^ ballot(p < beam[r]))) ? p : beam[r];
+        }
+    }
+}
+
+// v sorted over the 64 lanes, largest first
+__device__ __forceinline__ uint64_t sort_descending(uint64_t v) {
+#pragma unroll
+    for (int ki = 1; ki <= 6; ++ki)
+#pragma unroll
+        for (int si = ki - 1; si >= 0; --si) {
+            const uint64_t p = bsw::xor_lane64_rt(v, 1u << si);
+            const uint64_t keep_max = ~(bsd::lanes_bit_clear(1u << si) ^ bsd::lanes_bit_clear(1u << ki));
+            v = bsw::lane_in(keep_max ^ ballot(p < v)) ? p : v;
+        }
+    return v;
+}
+
+// A wavefront holds 32 QB queries as A operands (KC steps of 16 dimensions x 2 planes) and
+// streams its split's base tiles as B operands, each operand register reloaded for the next
+// tile as soon as this tile's products have read it.  a.b = (hl + lh) + hh: the small products
+// are summed first and the large ones on top, so the small ones' roundings are 2^-11 of the
+// large ones', and the dropped one (ll) is below 2^-24 |a||b|.  Against fp64
+// the rms error of q.b is 0.37-0.71 of the fp32 instructions' (mixture and unit-sphere data, dims
+// 16..256; at most 0.87 over wide-ranged data), because the chain rounds 8 times less often.
+// Three fp16 products of 16 dimensions take 96 matrix cycles, eight v_mfma_f32_32x32x2f32 512.
+// 500k x 128, 10k queries: 17.1 -> 5.7 ms with the filtering below (the products alone 3.8, at
+// the rate a large bf16 matrix product reaches on the card); with it but fp32 products 12.2.
+// Two query blocks per wavefront (dim <= 128) halve the base bytes per product.
+//
+// The matrix pipe and the vector unit work at the same time: while tile t's products run, tile
+// t - 1's 16 QB values per lane are formed and compared, two after each step's products (two
+// accumulator sets).  Only a tile with a survivor leaves that rhythm.
+//
+// Filtering: a query's candidates are the rows with a_j <= tau, tau = the least of
+//   - this split's C-th value so far,
+//   - any split's C-th value (tshare: published with an atomic minimum),
+//   - the largest over G = min(splits, PUB) splits of each one's ceil(C / G)-th value: those
+//     splits together hold at least C values that are no larger.
+// Each bounds the query's C-th value over all rows from above, so no row among the C smallest
+// is dropped.  The third keeps the survivors near C (1 + ln(n / C)) per query instead of that
+// per split (500k rows in 6 splits: 917 -> 490 keys per query and split, 220 with the priming
+// below).
+template <int KC, int QB>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+gt_select(const uint4* frag, const float2* meta, uint64_t row0, uint64_t m, const float* queries, uint32_t dim,
+          uint64_t nq, uint32_t nsplit, uint32_t split_tiles, uint32_t fresh, uint64_t* topc, uint32_t* tshare,
+          uint32_t* pub, float* qscale) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    const uint32_t lane = lane_id(), wave = threadIdx.x >> 6, half = lane >> 5, l32 = lane & 31u;
+    const uint32_t lane = lane_id(), wave = bsw::uniform(threadIdx.x >> 6), half = lane >> 5, l32 = lane & 31u;
+    constexpr uint32_t NQ = 32 * QB;
+    constexpr int NP = planes(KC);
     const uint64_t w = static_cast<uint64_t>(blockIdx.x) * 4 + wave;
-    const uint64_t nqb = (nq + 31) / 32;
+    const uint64_t nqb = (nq + NQ - 1) / NQ;
     if (w >= nqb * nsplit) return;
     // consecutive wavefronts take consecutive query blocks of the same row split, so the
     // wavefronts resident together stream the same base tiles and share them through L2
-    const uint64_t qb = w % nqb, s = w / nqb;
-    const uint64_t r0 = s * split_rows;
-    const uint64_t r1 = std::min<uint64_t>(n, r0 + split_rows);
+    const uint64_t qb = w % nqb;
+    const uint32_t s = static_cast<uint32_t>(w / nqb);
+    const uint32_t ntile = static_cast<uint32_t>((m + 31) / 32);
+    const uint32_t t0 = s * split_tiles, t1 = std::min(ntile, t0 + split_tiles);
+    const uint32_t G = std::min(nsplit, PUB), mth = (C + G - 1) / G;
 
-    char* my = smem + static_cast<size_t>(wave) * LDS_WAVE;
+    char* my = smem + static_cast<size_t>(wave) * lds_wave(QB);
     uint64_t* buf = reinterpret_cast<uint64_t*>(my);
-    uint64_t* mscr = reinterpret_cast<uint64_t*>(my + 32 * BUF * 8);
-    uint64_t* maux = mscr + 128;
+    float* vals = reinterpret_cast<float*>(my + NQ * BUF * 8);
+    uint32_t* cnt = reinterpret_cast<uint32_t*>(my + NQ * BUF * 8 + 32 * TS * 4);  // keys in each query's buffer
 
-    // A operand: lane (l32, half) holds query qb*32 + l32, dimensions half*H + t
-    float a[H];
+    // A operands: block b, lane (l32, half): query qb * NQ + 32 b + l32, dimensions 16 kc + 8 half + i
+    // All the wavefront's queries share one scale, the largest query's: a query 2^k smaller
+    // keeps 2^(k - 29) of its own largest value and above in 11-bit planes, and the certificate
+    // counts what is lost below (gt_refine).
+    f16x8 a[QB][KC][NP];
+    float qinv;  // 1 / the scale
     {
-        const uint64_t qi = qb * 32 + l32;
-        const float* qv = queries + std::min<uint64_t>(qi, nq - 1) * dim;
+        float x[QB][KC][8], sc = 0x1p100f;
 #pragma unroll
-        for (int t = 0; t < H; ++t) {  // all loads first (clamped), then the zeroing
-            const uint32_t d = half * H + static_cast<uint32_t>(t);
-            a[t] = qv[d < dim ? d : 0u];
-        }
+        for (int b = 0; b < QB; ++b) {
+            const uint64_t qi = qb * NQ + 32u * b + l32;
+            const float* qv = queries + std::min<uint64_t>(qi, nq - 1) * dim;
 #pragma unroll
-        for (int t = 0; t < H; ++t) {
-            const uint32_t d = half * H + static_cast<uint32_t>(t);
-            if (qi >= nq || d >= dim) a[t] = 0.0f;
+            for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {  // all loads first (clamped), then the zeroing
+                    const uint32_t d = 16u * kc + 8u * half + i;
+                    x[b][kc][i] = qv[d < dim ? d : 0u];
+                }
+            float big = 0.0f;
+#pragma unroll
+            for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const uint32_t d = 16u * kc + 8u * half + i;
+                    const float v = qi < nq && d < dim ? x[b][kc][i] : 0.0f;
+                    x[b][kc][i] = v;
+                    big = fabsf(v) > big || v != v ? (v != v ? __builtin_inff() : fabsf(v)) : big;
+                }
+            big = fmaxf(big, bsw::xor_lane_f<32>(big));
+            sc = query_scale(big, sc);
         }
+        sc = bsw::wave_min(sc);
+        qinv = 1.0f / sc;
+#pragma unroll
+        for (int b = 0; b < QB; ++b)
+#pragma unroll
+            for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    _Float16 v[NP];
+                    split_value<NP>(x[b][kc][i] * sc, v);
+#pragma unroll
+                    for (int p = 0; p < NP; ++p) a[b][kc][p][i] = v[p];
+                }
     }
-    // per accumulator register, the threshold of its query: the largest value its list
-    // keeps (a float compare passes a superset of the list's key order)
-    float tau[16];
+    if (s == 0 && lane == 0) qscale[qb] = qinv;
+    // tau: per accumulator register, the threshold of its query (a float compare passes a
+    // superset of the list's key order; none passes for a query past nq).  Lane i's tq is query
+    // i's.
+    float tq = qb * NQ + lane < nq && lane < NQ ? __builtin_inff() : -__builtin_inff();
+    float tau[QB][16];
+    uint32_t real = 0;  // the bits of `bits` (below) whose query exists
 #pragma unroll
-    for (int r = 0; r < 16; ++r) tau[r] = __builtin_inff();
-    // lane i < 32 holds the number of keys in query i's append buffer
-    uint32_t cnt = 0;
+    for (int e = 0; e < 16 * QB; ++e) real |= qb * NQ + 32u * (e / 16) + acc_row(e % 16, half) < nq ? 1u << e : 0u;
     // queries whose list has been written to HBM (each lane re-reads only what it wrote)
-    uint32_t written = 0;
+    uint64_t written = fresh ? 0ull : ~0ull;
 
-    // B operand: lane (l32, half) holds row tile + l32 (clamped), dimensions half*H + t
-    auto load_tile = [&](uint64_t tile, float4 (&b)[H / 4], float& bnj) __attribute__((always_inline)) {
-        const uint64_t j = std::min<uint64_t>(tile + l32, n - 1);
-        const float4* row = reinterpret_cast<const float4*>(vecs + j * dstride);
-        // chunks past the row read chunk 0 instead: the query operand is 0 in those
-        // dimensions, so they add nothing, and no load waits on a condition
+    auto spread_tau = [&]() __attribute__((always_inline)) {
 #pragma unroll
-        for (int c = 0; c < H / 4; ++c) {
-            const uint32_t c4 = half * (H / 4) + static_cast<uint32_t>(c);
-            b[c] = row[4u * c4 < dstride ? c4 : 0u];
-        }
-        bnj = bn[j];
+        for (int b = 0; b < QB; ++b)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                tau[b][r] = __int_as_float(__builtin_amdgcn_ds_bpermute(
+                    static_cast<int>((32u * b + acc_row(r, half)) << 2), __float_as_int(tq)));
+    };
+    // every query's threshold from what the splits have published
+    auto refresh = [&]() __attribute__((always_inline)) {
+        const uint64_t qi = std::min<uint64_t>(qb * NQ + (lane & (NQ - 1)), nq - 1);
+        uint32_t v = 0;
+        for (uint32_t g = 0; g < G; ++g)
+            v = std::max(v, __hip_atomic_load(&pub[static_cast<uint64_t>(g) * nq + qi], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        tq = fminf(tq, tau_of(std::min(v, tshare[qi])));
+        return v != ~0u;
     };
 
-    // merge every query buffer holding at least `need` keys into its top-C list
+    // merge every query buffer holding at least `need` keys into its top-C list; the next
+    // buffer's list is requested before this one's is merged
+    struct Row {
+        uint64_t k0, k1;
+        uint32_t sh, pb;
+    };
     auto compact = [&](uint32_t need) __attribute__((always_inline)) {
-        const uint32_t mycnt = lane < 32 ? cnt : 0u;
-        uint64_t todo = ballot(lane < 32 && mycnt >= need);
+        const uint32_t have = cnt[lane & (NQ - 1)];  // lane i: query i's
+        uint64_t todo = ballot(lane < NQ && have >= need && qb * NQ + lane < nq);
+        auto fetch = [&](uint32_t i, Row& x) __attribute__((always_inline)) {
+            const uint64_t qi = qb * NQ + i;
+            const uint64_t* top = topc + (qi * nsplit + s) * C;
+            x.sh = tshare[qi];
+            x.pb = lane < G ? pub[static_cast<uint64_t>(lane) * nq + qi] : 0u;
+            x.k0 = x.k1 = EMPTY_KEY;
+            if ((written >> i) & 1u) {
+                x.k0 = top[lane];
+                x.k1 = top[64 + lane];
+            }
+        };
+        if (!todo) return;
+        if (bsw::lane_in(todo)) cnt[lane] = 0u;
+        Row cur;
+        uint32_t i = static_cast<uint32_t>(__builtin_ctzll(todo));
+        fetch(i, cur);
         while (todo) {
-            const uint32_t i = static_cast<uint32_t>(__builtin_ctzll(todo));
             todo &= todo - 1;
-            const uint32_t c = readlane(mycnt, i);
-            const uint64_t qi = qb * 32 + i;
-            if (qi < nq) {
-                uint64_t* top = topc + (qi * nsplit + s) * C;
-                uint64_t beam[2] = {EMPTY_KEY, EMPTY_KEY};
-                const uint32_t shared = tshare[qi];  // issued with the list: one round trip
-                if ((written >> i) & 1u) {
-                    beam[0] = top[lane];
-                    beam[1] = top[64 + lane];
-                }
-                written |= 1u << i;
-                // one HBM round trip of the list per flush, then the buffer in runs of 64
-                bsd::BeamState st = bsd::beam_state<2>(beam);
-                for (uint32_t b0 = 0; b0 < c; b0 += 64) {
-                    uint64_t ck[1] = {b0 + lane < c ? buf[i * BUF + b0 + lane] : EMPTY_KEY};
-                    uint64_t cm[1] = {ballot(b0 + lane < c)};
-                    bsd::beam_merge<2, 1, true>(beam, ck, cm, C, mscr, maux, st);
-                }
-                top[lane] = beam[0];
-                top[64 + lane] = beam[1];
-                const uint64_t last = readlane64(beam[1], 63);
-                // this split's C-th value bounds the query's C-th value over all rows from
-                // above; publish it, and filter by the least bound any split has published
-                if (last != EMPTY_KEY && lane == 0) atomicMin(&tshare[qi], static_cast<uint32_t>(last >> 32));
-                const uint32_t tk = std::min(last == EMPTY_KEY ? ~0u : static_cast<uint32_t>(last >> 32), shared);
-                const float nt = tk == ~0u ? __builtin_inff() : bsd::key_dist(static_cast<uint64_t>(tk) << 32);
-                const uint32_t rr = 4u * (i / 8u) + (i % 4u), hh = (i / 4u) & 1u;
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    if (static_cast<uint32_t>(r) == rr && half == hh) tau[r] = nt;
+            Row nxt = {EMPTY_KEY, EMPTY_KEY, 0u, 0u};
+            const uint32_t ni = todo ? static_cast<uint32_t>(__builtin_ctzll(todo)) : i;
+            if (todo) fetch(ni, nxt);
+            const uint32_t c = readlane(have, i);
+            const uint64_t qi = qb * NQ + i;
+            uint64_t* top = topc + (qi * nsplit + s) * C;
+            uint64_t beam[2] = {cur.k0, cur.k1};
+            // the list's second half against the new keys, largest first, is already bitonic
+            const uint64_t rev[2] = {EMPTY_KEY, sort_descending(lane < c ? buf[i * BUF + lane] : EMPTY_KEY)};
+            merge_lists(beam, rev);
+            top[lane] = beam[0];
+            top[64 + lane] = beam[1];
+            written |= 1ull << i;
+            const uint32_t last = static_cast<uint32_t>(readlane64(beam[1], 63) >> 32);
+            const uint32_t mk = static_cast<uint32_t>(
+                readlane64(mth > 64u ? beam[1] : beam[0], (mth - 1) & 63u) >> 32);
+            if (lane == 0) {
+                if (last != ~0u) atomicMin(&tshare[qi], last);
+                if (s < G) atomicMin(&pub[static_cast<uint64_t>(s) * nq + qi], mk);  // primed values may be lower
             }
-            if (lane == i) cnt = 0;
-            wave_sync();
+            uint32_t pb = lane == s ? std::min(mk, cur.pb) : cur.pb;
+            pb = std::max(pb, bsw::xor_lane<1>(pb));
+            pb = std::max(pb, bsw::xor_lane<2>(pb));
+            pb = std::max(pb, bsw::partner<4>(pb));
+            pb = std::max(pb, bsw::partner<8>(pb));
+            const uint32_t all = std::max(std::max(readlane(pb, 0), readlane(pb, 16)),
+                                          std::max(readlane(pb, 32), readlane(pb, 48)));
+            const float nt = tau_of(std::min(std::min(last, cur.sh), all));
+            tq = lane == i ? nt : tq;
+            cur = nxt;
+            i = ni;
         }
+        spread_tau();
+        wave_sync();
     };
 
-    auto step = [&](uint64_t tile, const float4 (&b)[H / 4], float bnj) __attribute__((always_inline)) {
-        // one accumulator: a 32x32x2 f32 step occupies the matrix pipe as long as its
-        // result takes, so the dependent chain costs no extra issue slots
-        f32x16 acc = {};
+    // The survivors (bit 16 b + r of a lane's `bits`: its value of block b, register r) into
+    // their queries' buffers.  The values of 32 lanes at a time go to LDS, where each lane picks
+    // its survivors one by one; a slot is an LDS counter's.  (Appending from the registers, a
+    // branch and a ballot for each of the 32, took three times as long, and its code did not fit
+    // the instruction cache.)  Returns whether a buffer has reached FLUSH.
+    auto append = [&](uint32_t bits, const float (&av)[QB][16], uint32_t j) __attribute__((always_inline)) {
+        bool full = false;
+        uint64_t todo = ballot(bits != 0u);
+        while (todo) {
+            const uint32_t rank = bsw::lanes_below(todo);
+            const uint64_t now = todo & ballot(rank < 32u);
+            float* mine = vals + std::min(rank, 31u) * TS;
+            uint32_t left = 0;
+            if (bsw::lane_in(now)) {
 #pragma unroll
-        for (int c = 0; c < H / 4; ++c) {
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[4 * c + 0], b[c].x, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[4 * c + 1], b[c].y, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[4 * c + 2], b[c].z, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[4 * c + 3], b[c].w, acc, 0, 0, 0);
+                for (int b = 0; b < QB; ++b)
+#pragma unroll
+                    for (int r = 0; r < 16; r += 4)
+                        *reinterpret_cast<f32x4*>(mine + 16 * b + r) = f32x4{av[b][r], av[b][r + 1], av[b][r + 2], av[b][r + 3]};
+                left = bits;
+            }
+            wave_sync();
+            while (ballot(left != 0u)) {
+                if (left) {
+                    const uint32_t e = static_cast<uint32_t>(__builtin_ctz(left));
+                    left &= left - 1;
+                    const uint32_t q = (e & 16u) * 2u + (e & 12u) * 2u + 4u * half + (e & 3u);  // 32 b + acc_row(r, half)
+                    const uint32_t pos = __hip_atomic_fetch_add(&cnt[q], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+                    float x = mine[e];
+                    if (x != x) x = __builtin_nanf("");  // any NaN sorts last
+                    buf[q * BUF + pos] = (static_cast<uint64_t>(orderable(x)) << 32) | j;  // pos < BUF: < FLUSH before the tile
+                    full |= pos >= FLUSH - 1;
+                }
+            }
+            todo &= ~now;
+            wave_sync();
         }
-        const uint64_t j = tile + l32;
-        const bool whole = tile + 32 <= r1;  // wave-uniform: only a split's last tile is partial
-        // Accumulator register r holds, in each lane half h, the 32 rows of one query
-        // acc_row(r, h), so a register's survivors append to at most two buffers: their
-        // slots come from the ballot (mbcnt within the half), not from LDS atomics.  First
-        // every a_j and the survivors (independent, so they issue back to back), then the
-        // wave-uniform branches, only for groups of four registers holding a survivor.
-        float av[16];
-        uint32_t okb = 0;
-        const bool in = whole || j < r1;
+        return ballot(full) != 0;
+    };
+
+    f16x8 bp[KC][NP];
+    auto load_plane = [&](uint32_t tile, int kc, int p) __attribute__((always_inline)) {
+        bp[kc][p] = __builtin_bit_cast(f16x8, frag[((static_cast<uint64_t>(tile) * KC + kc) * NP + p) * 64 + lane]);
+    };
+    if (lane < NQ) cnt[lane] = 0u;
+    wave_sync();
+
+    // Tile t's products into accN (the next tile's operands requested as these are read), with
+    // the previous tile's values av formed from accO on the way; returns the lane's survivors
+    float av[QB][16];
+    auto step = [&](uint32_t next, f32x16 (&accN)[QB], const f32x16 (&accO)[QB], float2 mo) __attribute__((always_inline)) {
+        uint32_t bits = 0;
+        constexpr int SMALL = (NP == 3 ? 5 : 2) * QB, ALL = KC * (SMALL + QB);  // matrix instructions
+        // the values screened beside instructions [m0, m1) of the tile's ALL
+        auto screen = [&](int m0, int m1) __attribute__((always_inline)) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            av[r] = __builtin_fmaf(-2.0f, acc[r], bnj);
-            okb |= (in && av[r] <= tau[r]) ? 1u << r : 0u;
+            for (int e = 16 * QB * m0 / ALL; e < 16 * QB * m1 / ALL; ++e) {
+                const int b = e / 16, r = e % 16;
+                // a_j = |b_j|^2 - 2 acc / (row scale query scale): exact factors, one rounding
+                // (their product may underflow, so they are not combined)
+                av[b][r] = __builtin_fmaf(accO[b][r] * mo.y, qinv, mo.x);
+                bits |= !(av[b][r] > tau[b][r]) ? 1u << e : 0u;  // a NaN survives
+            }
+        };
+#define BSG_MFMA(kc, pa, pb, from)                                                                   \
+    _Pragma("unroll") for (int b = 0; b < QB; ++b) accN[b] =                                          \
+        __builtin_amdgcn_mfma_f32_32x32x16_f16(a[b][kc][pa], bp[kc][pb], from, 0, 0, 0);
+        const f32x16 zero = {};
+#pragma unroll
+        for (int kc = 0; kc < KC; ++kc) {
+            if (kc == 0) {
+                BSG_MFMA(kc, 0, NP - 1, zero)
+            } else {
+                BSG_MFMA(kc, 0, NP - 1, accN[b])
+            }
+            BSG_MFMA(kc, NP - 1, 0, accN[b])
+            if constexpr (NP == 3) {
+                BSG_MFMA(kc, 1, 1, accN[b])
+                BSG_MFMA(kc, 0, 1, accN[b])
+                BSG_MFMA(kc, 1, 0, accN[b])
+                load_plane(next, kc, 1);
+            }
+            load_plane(next, kc, NP - 1);
+            screen(kc * SMALL, (kc + 1) * SMALL);
+            // keep the reloads and the screening among the products: a matrix instruction, then
+            // vector ones in its shadow
+#pragma unroll
+            for (int i = 0; i < SMALL; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        const uint64_t any = ballot(okb != 0u);
-        bool appended = false;
-        if (any) {
-            appended = true;
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                if (!ballot(((okb >> (4 * g)) & 15u) != 0u)) continue;
+        for (int kc = 0; kc < KC; ++kc) {
+            BSG_MFMA(kc, 0, 0, accN[b])
+            load_plane(next, kc, 0);
+            screen(KC * SMALL + kc * QB, KC * SMALL + (kc + 1) * QB);
 #pragma unroll
-                for (int r = 4 * g; r < 4 * g + 4; ++r) {
-                    const bool ok = (okb >> r) & 1u;
-                    const uint64_t m = ballot(ok);
-                    if (!m) continue;
-                    const uint32_t m0 = static_cast<uint32_t>(m), m1 = static_cast<uint32_t>(m >> 32);
-                    const uint32_t i0 = acc_row(r, 0), i1 = acc_row(r, 1);
-                    const uint32_t c0 = readlane(cnt, i0), c1 = readlane(cnt, i1);  // < FLUSH: see below
-                    if (ok) {
-                        const uint32_t pos = half ? c1 + __builtin_amdgcn_mbcnt_hi(m1, 0u) : c0 + __builtin_amdgcn_mbcnt_lo(m0, 0u);
-                        const uint32_t i = half ? i1 : i0;
-                        buf[i * BUF + pos] = (static_cast<uint64_t>(orderable(av[r])) << 32) | static_cast<uint32_t>(j);
+            for (int i = 0; i < QB; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#undef BSG_MFMA
+        return bits;
+    };
+    // the survivors of `tile` (values av) appended, full buffers merged: every buffer holds <
+    // FLUSH keys before the next 32 rows arrive
+    auto keep = [&](uint32_t bits, uint32_t tile) __attribute__((always_inline)) {
+        const uint32_t at = tile * 32u + l32;
+        bits = at < m ? bits & real : 0u;  // the last tile may be partial
+        if (ballot(bits != 0u) && append(bits, av, static_cast<uint32_t>(row0) + at)) compact(FLUSH);
+    };
+    // Priming.  A pass over the split's first `prime` tiles keeps only each lane's least value per
+    // query (in tau): the mth smallest of a query's 32 lane minima is no less than the mth
+    // smallest value of those rows, so it can be published as this split's mth value before any
+    // list exists, and the lists then start at a threshold that admits about one row in 50
+    // instead of every row.
+    const uint32_t prime = fresh && nsplit > 1 && mth <= 32u && t1 > t0 ? std::min(64u, (t1 - t0) / 16u) : 0u;
+    auto publish_minima = [&]() __attribute__((always_inline)) {
+        float* st = reinterpret_cast<float*>(buf);  // no keys yet: NQ queries x TS floats
+#pragma unroll
+        for (int b = 0; b < QB; ++b)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) st[(32u * b + acc_row(r, half)) * TS + l32] = tau[b][r];
+        wave_sync();
+        float x[32];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const f32x4 v = *reinterpret_cast<const f32x4*>(st + (lane & (NQ - 1)) * TS + 4 * i);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) x[4 * i + k] = v[k];
+        }
+        wave_sync();
+        // ascending bitonic network over the lane's 32 values
+#pragma unroll
+        for (int ki = 1; ki <= 5; ++ki)
+#pragma unroll
+            for (int si = ki - 1; si >= 0; --si)
+#pragma unroll
+                for (int i = 0; i < 32; ++i)
+                    if (!(i & (1 << si))) {
+                        const int o = i | (1 << si);
+                        const float lo = fminf(x[i], x[o]), hi = fmaxf(x[i], x[o]);
+                        x[i] = (i & (1 << ki)) ? hi : lo;
+                        x[o] = (i & (1 << ki)) ? lo : hi;
                     }
-                    cnt += lane == i0 ? static_cast<uint32_t>(__builtin_popcount(m0)) : 0u;
-                    cnt += lane == i1 ? static_cast<uint32_t>(__builtin_popcount(m1)) : 0u;
-                }
+        float v = x[31];
+#pragma unroll
+        for (int i = 0; i < 31; ++i) v = mth == static_cast<uint32_t>(i + 1) ? x[i] : v;
+        if (s < G && lane < NQ && qb * NQ + lane < nq && v < __builtin_inff())
+            __hip_atomic_store(&pub[static_cast<uint64_t>(s) * nq + qb * NQ + lane], static_cast<uint32_t>(orderable(v)),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // the other splits reach this point at about the same time: read until all have
+        // published, at most 32 times (about 30 us; a split that is not resident yet never will)
+        for (int i = 0; i < 32; ++i)
+            if (ballot(!refresh()) == 0) break;
+        spread_tau();
+    };
+    if (t0 < t1) {
+#pragma unroll
+        for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+            for (int p = 0; p < NP; ++p) load_plane(t0, kc, p);
+        refresh();
+        spread_tau();
+        if (prime) {
+#pragma unroll
+            for (int b = 0; b < QB; ++b)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) tau[b][r] = __builtin_inff();
+        }
+        // step u takes the products of tile_of(u) -- the primed tiles, then all of them, then the
+        // last once more -- and the values of the one before
+        const uint32_t total = prime + (t1 - t0), lastt = t1 - 1;
+        auto tile_of = [&](uint32_t u) __attribute__((always_inline)) {
+            return std::min(u < prime ? t0 + u : t0 + (u - prime), lastt);
+        };
+        auto done = [&](uint32_t bits, uint32_t u) __attribute__((always_inline)) {  // step u's values are in av
+            if (u < prime) {
+#pragma unroll
+                for (int b = 0; b < QB; ++b)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) tau[b][r] = fminf(tau[b][r], av[b][r]);
+                if (u + 1 == prime) publish_minima();
+            } else {
+                keep(bits, tile_of(u));
+            }
+        };
+        // the pass before the first screens zeros and its result is dropped
+        f32x16 acc0[QB], acc1[QB];
+#pragma unroll
+        for (int b = 0; b < QB; ++b) acc0[b] = acc1[b] = f32x16{};
+        float2 m0 = meta[t0 * 32u + l32], m1;
+        step(tile_of(1), acc0, acc1, m0);
+        for (uint32_t u = 1;; u += 2) {
+            m1 = meta[tile_of(u) * 32u + l32];
+            uint32_t bits = step(tile_of(u + 1), acc1, acc0, m0);
+            done(bits, u - 1);
+            if (u >= total) break;
+            m0 = meta[tile_of(u + 1) * 32u + l32];
+            bits = step(tile_of(u + 2), acc0, acc1, m1);
+            done(bits, u);
+            if (u + 1 >= total) break;
+            if (u % REFRESH == 1 && u > prime) {  // u is odd
+                refresh();
+                spread_tau();
             }
         }
-        if (appended) {
-            wave_sync();
-            compact(FLUSH);  // every buffer holds < FLUSH keys before the next 32 rows arrive
-        }
-    };
-
-    float4 bA[H / 4], bB[H / 4];
-    float nA = 0.0f, nB = 0.0f;
-    load_tile(r0, bA, nA);
-    for (uint64_t tile = r0; tile < r1; tile += 64) {
-        load_tile(tile + 32, bB, nB);  // rows past the split are loaded (clamped) and ignored
-        __builtin_amdgcn_sched_barrier(0);  // keep the prefetch ahead of this tile's products
-        step(tile, bA, nA);
-        if (tile + 32 >= r1) break;
-        load_tile(tile + 64, bA, nA);
-        __builtin_amdgcn_sched_barrier(0);
-        step(tile + 32, bB, nB);
     }
     compact(1);
-    for (uint32_t i = 0; i < 32; ++i) {  // a list with no key at all is still written
-        const uint64_t qi = qb * 32 + i;
+    // a list with no key at all is still written
+    for (uint32_t i = 0; i < NQ; ++i) {
+        const uint64_t qi = qb * NQ + i;
         if (!((written >> i) & 1u) && qi < nq) {
             topc[(qi * nsplit + s) * C + lane] = EMPTY_KEY;
             topc[(qi * nsplit + s) * C + 64 + lane] = EMPTY_KEY;
@@ -248,57 +609,107 @@ __global__ void __launch_bounds__(256) gt_select(const float* vecs, uint32_t dst
     }
 }
 
-// one wavefront per query: merge the split lists, exact fp64 re-score, order, certify
-__global__ void __launch_bounds__(256) gt_refine(const float* vecs, uint32_t dstride, uint64_t n, const float* queries,
-                                                 uint32_t dim, uint64_t nq, uint32_t nsplit, const uint64_t* topc,
-                                                 uint32_t k, float bmax2, int32_t* out, uint8_t* unc,
-                                                 unsigned long long* n_unc) {
-    extern __shared__ __attribute__((aligned(16))) char smem[];
-    const uint32_t lane = lane_id(), wave = threadIdx.x >> 6;
-    const uint64_t qi = static_cast<uint64_t>(blockIdx.x) * 4 + wave;
-    if (qi >= nq) return;
-    uint64_t* mscr = reinterpret_cast<uint64_t*>(smem) + static_cast<size_t>(wave) * 200;
-    uint64_t* maux = mscr + 128;
+// One workgroup of NW wavefronts per query: the split lists merged (a wavefront takes every
+// NW-th, the NW results meet in LDS), the 128 candidates re-scored exactly in fp64, ordered,
+// certified.  The candidates' rows pass through LDS: loaded coalesced (16 lanes per 64
+// dimensions of a row), read back by the lane that sums the row's distance in dimension order.
+// Bound by the gather of 128 rows per query: 10k queries x 128 dims 1.16 -> 0.27 ms (13 lists
+// before, 6 after) against a wavefront per query that merged by ranks and whose lanes read
+// their rows a word at a time.
+constexpr uint32_t RF_TS = 64 + 4;  // floats per staged row: 16 lanes of a b128 phase hit 16 distinct 4-bank groups
+
+template <int NW>
+__global__ void __launch_bounds__(64 * NW) gt_refine(const float* vecs, uint32_t dstride, const float* queries,
+                                                     uint32_t dim, uint32_t nsplit, const uint64_t* topc, uint32_t k,
+                                                     const uint32_t* bmax_bits, const float* qscale, uint32_t NQ,
+                                                     int32_t* out, uint8_t* unc, unsigned long long* n_unc) {
+    static_assert(NW >= 4, "four wavefronts score the candidates");
+    __shared__ __attribute__((aligned(16))) uint64_t keys[NW][C];
+    __shared__ __attribute__((aligned(16))) float rows[4][32 * RF_TS];
+    __shared__ float q[256];
+    __shared__ double dist[C];
+    __shared__ uint32_t ids[C], rank2[C];
+    const uint32_t t = threadIdx.x, lane = lane_id(), wave = bsw::uniform(t >> 6);
+    const uint64_t qi = blockIdx.x;
+    const float* qv = queries + qi * dim;
+    for (uint32_t i = t; i < dim; i += 64 * NW) q[i] = qv[i];
 
     const uint64_t* lists = topc + qi * nsplit * C;
-    uint64_t beam[2] = {lists[lane], lists[64 + lane]};
-    bsd::BeamState st = bsd::beam_state<2>(beam);
-    for (uint32_t s = 1; s < nsplit; ++s) {
-        uint64_t ck[2] = {lists[s * C + lane], lists[s * C + 64 + lane]};
-        uint64_t cm[2] = {ballot(ck[0] != EMPTY_KEY), ballot(ck[1] != EMPTY_KEY)};
-        bsd::beam_merge<2, 2, false>(beam, ck, cm, C, mscr, maux, st);
+    uint64_t beam[2] = {EMPTY_KEY, EMPTY_KEY};
+    for (uint32_t s = wave; s < nsplit; s += NW) {
+        const uint64_t rev[2] = {lists[static_cast<uint64_t>(s) * C + C - 1 - lane], lists[static_cast<uint64_t>(s) * C + 63 - lane]};
+        merge_lists(beam, rev);
     }
-    const uint64_t kc = readlane64(beam[1], 63);  // the C-th approximate key
-
-    // exact distances, dimension order, fp64 (bs_groundtruth's l2d)
-    const float* qv = queries + qi * dim;
-    double dd[2];
-    uint32_t id[2];
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-        id[r] = beam[r] == EMPTY_KEY ? 0xFFFFFFFFu : static_cast<uint32_t>(beam[r]);
-        const float* row = vecs + static_cast<uint64_t>(id[r] == 0xFFFFFFFFu ? 0u : id[r]) * dstride;
-        double acc = 0.0;
-        for (uint32_t i = 0; i < dim; ++i) {
-            const double diff = __dsub_rn(static_cast<double>(qv[i]), static_cast<double>(row[i]));
-            acc = __dadd_rn(acc, __dmul_rn(diff, diff));
+    // pairs of results, halving: the upper wavefront leaves its list in reverse
+#pragma unroll 1
+    for (uint32_t h = NW / 2; h >= 1; h >>= 1) {
+        if (wave >= h && wave < 2 * h) {
+            keys[wave][C - 1 - lane] = beam[0];
+            keys[wave][63 - lane] = beam[1];
         }
-        dd[r] = id[r] == 0xFFFFFFFFu ? __builtin_inf() : acc;
+        __syncthreads();
+        if (wave < h) {
+            const uint64_t rev[2] = {keys[wave + h][lane], keys[wave + h][64 + lane]};
+            merge_lists(beam, rev);
+        }
     }
-    // rank of each candidate in (distance, id) order
-    uint32_t rank[2] = {0, 0};
-    for (uint32_t e = 0; e < C; ++e) {
-        const uint64_t vb = readlane64(static_cast<uint64_t>(__double_as_longlong(e < 64 ? dd[0] : dd[1])), e & 63u);
-        const uint32_t ve = readlane(e < 64 ? id[0] : id[1], e & 63u);
-        const double de = __longlong_as_double(static_cast<long long>(vb));
+    if (wave == 0) {
+        keys[0][lane] = beam[0];
+        keys[0][64 + lane] = beam[1];
+        ids[lane] = beam[0] == EMPTY_KEY ? 0xFFFFFFFFu : static_cast<uint32_t>(beam[0]);
+        ids[64 + lane] = beam[1] == EMPTY_KEY ? 0xFFFFFFFFu : static_cast<uint32_t>(beam[1]);
+    }
+    if (t < C) rank2[t] = 0u;
+    __syncthreads();
+    const uint64_t kc = keys[0][C - 1];  // the C-th approximate key
+
+    // exact distances, dimension order, fp64 (bs_groundtruth's l2d): wavefront w < 4 takes
+    // candidates 32 w .. 32 w + 31
+    if (wave < 4) {
+        float* tile = rows[wave];
+        const uint32_t lr = lane >> 4, lc = (lane & 15u) * 4;
+        double acc = 0.0;
+        for (uint32_t d0 = 0; d0 < dim; d0 += 64) {
+            f32x4 v[8];
 #pragma unroll
-        for (int r = 0; r < 2; ++r) rank[r] += (de < dd[r] || (de == dd[r] && ve < id[r])) ? 1u : 0u;
+            for (uint32_t i = 0; i < 8; ++i) {
+                const uint32_t id = ids[32 * wave + 4 * i + lr];
+                const float* row = vecs + static_cast<uint64_t>(id == 0xFFFFFFFFu ? 0u : id) * dstride;
+                v[i] = *reinterpret_cast<const f32x4*>(row + (d0 + lc < dstride ? d0 + lc : 0u));
+            }
+            wave_sync();  // the previous tile's reads are done before it is overwritten
+#pragma unroll
+            for (uint32_t i = 0; i < 8; ++i) *reinterpret_cast<f32x4*>(tile + (4 * i + lr) * RF_TS + lc) = v[i];
+            wave_sync();
+            const float* mine = tile + (lane & 31u) * RF_TS;
+            const uint32_t cols = dim - d0 < 64 ? dim - d0 : 64;
+            for (uint32_t i = 0; i < cols; ++i) {
+                const double diff = __dsub_rn(static_cast<double>(q[d0 + i]), static_cast<double>(mine[i]));
+                acc = __dadd_rn(acc, __dmul_rn(diff, diff));
+            }
+        }
+        if (lane < 32) dist[32 * wave + lane] = ids[32 * wave + lane] == 0xFFFFFFFFu ? __builtin_inf() : acc;
     }
+    __syncthreads();
+    // rank of each candidate in (distance, id) order: thread t counts candidate t % C against
+    // half of the others
+    if (t < 2 * C) {
+        const uint32_t c = t & (C - 1), e0 = (t / C) * (C / 2);
+        const double d = dist[c];
+        const uint32_t id = ids[c];
+        uint32_t rank = 0;
+        for (uint32_t e = e0; e < e0 + C / 2; ++e) rank += (dist[e] < d || (dist[e] == d && ids[e] < id)) ? 1u : 0u;
+        if (rank) atomicAdd(&rank2[c], rank);
+    }
+    __syncthreads();
+    if (wave != 0) return;
     // valid candidates take ranks 0..nvalid-1; the slots from nvalid to k get -1
     int32_t* o = out + qi * k;
+    const uint32_t id[2] = {ids[lane], ids[64 + lane]}, rank[2] = {rank2[lane], rank2[64 + lane]};
+    const double dd[2] = {dist[lane], dist[64 + lane]};
     const uint32_t nvalid = static_cast<uint32_t>(__builtin_popcountll(ballot(id[0] != 0xFFFFFFFFu)) +
                                                   __builtin_popcountll(ballot(id[1] != 0xFFFFFFFFu)));
-    for (uint32_t t = nvalid + lane; t < k; t += 64) o[t] = -1;
+    for (uint32_t e = nvalid + lane; e < k; e += 64) o[e] = -1;
 #pragma unroll
     for (int r = 0; r < 2; ++r)
         if (id[r] != 0xFFFFFFFFu && rank[r] < k) o[rank[r]] = static_cast<int32_t>(id[r]);
@@ -314,10 +725,22 @@ __global__ void __launch_bounds__(256) gt_refine(const float* vecs, uint32_t dst
                            readlane64(static_cast<uint64_t>(__double_as_longlong(dd[r])), __builtin_ctzll(m))));
         }
         double qn2 = 0.0;
-        for (uint32_t i = 0; i < dim; ++i) qn2 += static_cast<double>(qv[i]) * static_cast<double>(qv[i]);
+        for (uint32_t i = 0; i < dim; ++i) qn2 += static_cast<double>(q[i]) * static_cast<double>(q[i]);
         const double ac = static_cast<double>(bsd::key_dist(kc));
-        const double qb = __builtin_sqrt(qn2) + __builtin_sqrt(static_cast<double>(bmax2));
-        const double eps = 2.0 * (dim + 3) * 0x1p-24 * qb * qb;
+        const double bm = __builtin_sqrt(static_cast<double>(__uint_as_float(*bmax_bits)));
+        const double qb = __builtin_sqrt(qn2) + bm;
+        // q.b's error: the planes' 2^-24 of each factor and the dropped product, 3 2^-24 |q||b|;
+        // dim accumulations of exact products, dim 2^-24 |q||b| (twice that if the matrix unit
+        // truncates); what lies below fp16's range in the row, 2^-28 sqrt(dim) |q||b|.  (|q| +
+        // |b|)^2 >= 4 |q||b|, so 2 (dim + 3) 2^-24 (|q| + |b|)^2 covers twice their sum and the
+        // norms' roundings.  What lies below fp16's range in the query (2^-14 over the scale it
+        // shares with its neighbours, if the matrix unit flushes it) is 2^-14 qscale sqrt(dim)
+        // |b| at most.  A row whose largest value is below 2^-86 has the largest scale, 2^100: it
+        // loses 2^-114 per value.  2^-140: results below fp32's normal range.
+        const double sd = __builtin_sqrt(static_cast<double>(dim));
+        const double eps = 2.0 * (dim + 3) * 0x1p-24 * qb * qb +
+                           2.0 * 0x1p-14 * static_cast<double>(qscale[qi / NQ]) * sd * bm +
+                           2.0 * 0x1p-114 * sd * __builtin_sqrt(qn2) + 0x1p-140;
         ok = dk < ac + qn2 - eps;
     }
     if (lane == 0) {
@@ -348,17 +771,39 @@ int gfail(int code, const std::string& msg) {
         if (e_ != hipSuccess) return gfail(BS_EHIP, std::string(#call) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
-template <int KP>
-hipError_t launch_select(dim3 g, hipStream_t s, const float* vecs, uint32_t dstride, const float* bn, uint64_t n,
-                         const float* q, uint32_t dim, uint64_t nq, uint32_t nsplit, uint64_t split_rows,
-                         uint64_t* topc, uint32_t* tshare) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(bsg::gt_select<KP>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, 4 * bsg::LDS_WAVE);
+// one workgroup of the select: KC steps of 16 dimensions, QB query blocks of 32 per wavefront
+template <int KC, int QB>
+hipError_t launch_select(dim3 g, hipStream_t s, const uint4* frag, const float2* meta, uint64_t row0, uint64_t m,
+                         const float* q, uint32_t dim, uint64_t nq, uint32_t nsplit, uint32_t split_tiles,
+                         uint64_t* topc, uint32_t* tshare, uint32_t* pub, float* qscale) {
+    constexpr int lds = 4 * bsg::lds_wave(QB);
+    auto k = bsg::gt_select<KC, QB>;
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(bsg::gt_select<KP>, g, dim3(256), 4 * bsg::LDS_WAVE, s, vecs, dstride, bn, n, q, dim, nq,
-                       nsplit, split_rows, topc, tshare);
+    hipLaunchKernelGGL(k, g, dim3(256), lds, s, frag, meta, row0, m, q, dim, nq, nsplit, split_tiles,
+                       row0 == 0 ? 1u : 0u, topc, tshare, pub, qscale);
     return hipGetLastError();
 }
+
+// Row splits per query block: nqb * nsplit wavefronts run 4 per CU (a SIMD holds one), so the
+// count is the one that fills whole rounds of them best, few rounds and few splits first (a
+// split costs its query another list of 128 to fill, publish and merge).  At least 8 tiles
+// per split.
+uint64_t pick_splits(uint64_t nqb, uint64_t tiles, uint64_t slots) {
+    const uint64_t most = std::max<uint64_t>(1, std::min<uint64_t>({1024, tiles / 8, 3 * slots / nqb}));
+    uint64_t best = 1;
+    double score = -1e9;
+    for (uint64_t s = 1; s <= most; ++s) {
+        const uint64_t w = nqb * s, rounds = (w + slots - 1) / slots;
+        const double fill = static_cast<double>(w) / static_cast<double>(rounds * slots) - 0.15 * static_cast<double>(rounds);
+        if (fill > score + 1e-9) {
+            score = fill;
+            best = s;
+        }
+    }
+    return best;
+}
+
 }  // namespace
 
 extern "C" int bs_index_groundtruth_device(bs_index idx, const float* d_queries, uint64_t nq, uint32_t k,
@@ -377,63 +822,79 @@ extern "C" int bs_index_groundtruth_device(bs_index idx, const float* d_queries,
     if (nq == 0) return BS_OK;
     if (!d_queries || !d_out) return gfail(BS_EINVAL, "queries and output must be given");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int KP = dim <= 64 ? 64 : dim <= 128 ? 128 : dim <= 192 ? 192 : 256;
-    const uint64_t nqb = (nq + 31) / 32;
-    // about 4096 wavefronts in flight: split the rows among them (>= 32 rows each)
-    uint64_t nsplit = std::max<uint64_t>(1, std::min<uint64_t>(256, 4096 / nqb));
-    uint64_t split_rows = ((n + nsplit - 1) / nsplit + 31) / 32 * 32;
-    nsplit = (n + split_rows - 1) / split_rows;
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+        cus = 256;
+    // 16-dimension steps, and 64 queries per wavefront while their operands fit beside a tile's
+    const uint32_t KC = dim <= 32 ? 2 : dim <= 64 ? 4 : dim <= 96 ? 6 : dim <= 128 ? 8 : dim <= 192 ? 12 : 16;
+    const uint32_t NQ = KC <= 8 ? 64 : 32;
+    const uint64_t nqb = (nq + NQ - 1) / NQ;
+    // the fp16 planes are made for at most 1 GiB of rows at a time; the lists carry over
+    const uint64_t tile_bytes = static_cast<uint64_t>(KC) * static_cast<uint64_t>(bsg::planes(static_cast<int>(KC))) * 1024;
+    const uint64_t tiles = (n + 31) / 32, chunk = std::min<uint64_t>(tiles, (1ull << 30) / tile_bytes);
+    const uint64_t nsplit = pick_splits(nqb, chunk, 4ull * static_cast<uint64_t>(cus));
+    const uint64_t split_tiles = (chunk + nsplit - 1) / nsplit;
 
-    float* bn = nullptr;
-    uint32_t* bmax = nullptr;
-    uint64_t* topc = nullptr;
-    uint32_t* tshare = nullptr;
-    unsigned long long* nunc = nullptr;
-    auto release = [&]() {
-        if (bn) (void)hipFree(bn);
-        if (bmax) (void)hipFree(bmax);
-        if (topc) (void)hipFree(topc);
-        if (tshare) (void)hipFree(tshare);
-        if (nunc) (void)hipFree(nunc);
-    };
-    if (hipMalloc(&bn, n * sizeof(float)) != hipSuccess || hipMalloc(&bmax, 4) != hipSuccess ||
-        hipMalloc(&topc, nq * nsplit * bsg::C * 8) != hipSuccess || hipMalloc(&nunc, 8) != hipSuccess ||
-        hipMalloc(&tshare, nq * 4) != hipSuccess) {
-        release();
+    // one allocation: planes, norms, lists, published values, counters
+    auto al = [](uint64_t v) { return (v + 255) & ~255ull; };
+    const uint64_t o_bn = al(chunk * tile_bytes), o_top = o_bn + al(chunk * 32 * 8),
+                   o_share = o_top + al(nq * nsplit * bsg::C * 8),
+                   o_pub = o_share + nq * 4,  // tshare and pub start as all ones together
+                   o_cnt = al(o_pub + std::min<uint64_t>(nsplit, bsg::PUB) * nq * 4), o_qs = o_cnt + 256, need = o_qs + nqb * 4;
+    char* ws = nullptr;
+    if (hipMalloc(reinterpret_cast<void**>(&ws), need) != hipSuccess)
         return gfail(BS_ENOMEM, "hipMalloc of the ground-truth work buffers failed");
-    }
-    hipError_t e = hipMemsetAsync(bmax, 0, 4, s);
-    if (e == hipSuccess) e = hipMemsetAsync(nunc, 0, 8, s);
-    if (e == hipSuccess) e = hipMemsetAsync(tshare, 0xFF, nq * 4, s);  // no bound published yet
-    if (e == hipSuccess) {
-        hipLaunchKernelGGL(bsg::gt_norms, dim3(static_cast<uint32_t>((n + 255) / 256)), dim3(256), 0, s, vecs, n, dim,
-                           dstride, bn, bmax);
-        e = hipGetLastError();
-    }
-    uint32_t bmax_host = 0;
-    if (e == hipSuccess) e = hipMemcpyAsync(&bmax_host, bmax, 4, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    float bmax2 = 0.0f;
-    std::memcpy(&bmax2, &bmax_host, 4);
-    if (e == hipSuccess) {
-        const dim3 g(static_cast<uint32_t>((nqb * nsplit + 3) / 4));
-        switch (KP) {
-        case 64: e = launch_select<64>(g, s, vecs, dstride, bn, n, d_queries, dim, nq, nsplit, split_rows, topc, tshare); break;
-        case 128: e = launch_select<128>(g, s, vecs, dstride, bn, n, d_queries, dim, nq, nsplit, split_rows, topc, tshare); break;
-        case 192: e = launch_select<192>(g, s, vecs, dstride, bn, n, d_queries, dim, nq, nsplit, split_rows, topc, tshare); break;
-        default: e = launch_select<256>(g, s, vecs, dstride, bn, n, d_queries, dim, nq, nsplit, split_rows, topc, tshare); break;
+    uint4* frag = reinterpret_cast<uint4*>(ws);
+    float2* meta = reinterpret_cast<float2*>(ws + o_bn);
+    uint64_t* topc = reinterpret_cast<uint64_t*>(ws + o_top);
+    uint32_t* tshare = reinterpret_cast<uint32_t*>(ws + o_share);
+    uint32_t* pub = reinterpret_cast<uint32_t*>(ws + o_pub);
+    unsigned long long* nunc = reinterpret_cast<unsigned long long*>(ws + o_cnt);
+    uint32_t* bmax = reinterpret_cast<uint32_t*>(ws + o_cnt + 8);
+    float* qscale = reinterpret_cast<float*>(ws + o_qs);
+    hipError_t e = hipMemsetAsync(nunc, 0, 16, s);
+    if (e == hipSuccess) e = hipMemsetAsync(tshare, 0xFF, o_cnt - o_share, s);  // no bound published yet
+    const dim3 g(static_cast<uint32_t>((nqb * nsplit + 3) / 4));
+    for (uint64_t c0 = 0; e == hipSuccess && c0 < tiles; c0 += chunk) {
+        const uint64_t row0 = c0 * 32, m = std::min(chunk * 32, n - row0), mt = (m + 31) / 32;
+        const dim3 sg(static_cast<uint32_t>(std::min<uint64_t>((mt + 3) / 4, 8ull * cus)));
+        auto go = [&](auto kc, auto qb) {
+            constexpr int K = decltype(kc)::value;
+            hipLaunchKernelGGL(bsg::gt_split<K>, sg, dim3(256), 0, s, vecs, row0, m, dstride, frag, meta, bmax);
+            const hipError_t le = hipGetLastError();
+            if (le != hipSuccess) return le;
+            return launch_select<K, decltype(qb)::value>(g, s, frag, meta, row0, m, d_queries, dim, nq,
+                                                         static_cast<uint32_t>(nsplit),
+                                                         static_cast<uint32_t>(split_tiles), topc, tshare, pub, qscale);
+        };
+        std::integral_constant<int, 1> q1;
+        std::integral_constant<int, 2> q2;
+        switch (KC) {
+        case 2: e = go(std::integral_constant<int, 2>{}, q2); break;
+        case 4: e = go(std::integral_constant<int, 4>{}, q2); break;
+        case 6: e = go(std::integral_constant<int, 6>{}, q2); break;
+        case 8: e = go(std::integral_constant<int, 8>{}, q2); break;
+        case 12: e = go(std::integral_constant<int, 12>{}, q1); break;
+        default: e = go(std::integral_constant<int, 16>{}, q1); break;
         }
     }
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(bsg::gt_refine, dim3(static_cast<uint32_t>((nq + 3) / 4)), dim3(256), 4 * 200 * 8, s, vecs,
-                           dstride, n, d_queries, dim, nq, static_cast<uint32_t>(nsplit), topc, k,
-                           bmax2, d_out, d_uncertified, nunc);
+        // a wavefront merges a list in ~0.3 us: with many splits (few queries) 16 share them
+        if (nsplit > 32)
+            hipLaunchKernelGGL(bsg::gt_refine<16>, dim3(static_cast<uint32_t>(nq)), dim3(1024), 0, s, vecs, dstride,
+                               d_queries, dim, static_cast<uint32_t>(nsplit), topc, k, bmax, qscale,
+                               NQ, d_out, d_uncertified, nunc);
+        else
+            hipLaunchKernelGGL(bsg::gt_refine<4>, dim3(static_cast<uint32_t>(nq)), dim3(256), 0, s, vecs, dstride,
+                               d_queries, dim, static_cast<uint32_t>(nsplit), topc, k, bmax, qscale,
+                               NQ, d_out, d_uncertified, nunc);
         e = hipGetLastError();
     }
     unsigned long long nu = 0;
     if (e == hipSuccess) e = hipMemcpyAsync(&nu, nunc, 8, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
-    release();
+    (void)hipFree(ws);
     if (e != hipSuccess) return gfail(BS_EHIP, std::string("ground truth: ") + hipGetErrorString(e));
     if (n_uncertified) *n_uncertified = nu;
     return BS_OK;

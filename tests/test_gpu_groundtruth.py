@@ -59,3 +59,86 @@ def test_groundtruth_at_scale(gpu):
     cert = (raw != -2).all(1)
     assert cert.mean() >= 0.95
     assert np.array_equal(raw[cert], exact[cert])
+
+
+@pytest.mark.parametrize("n,nq,dim,k", [(1, 1, 16, 1), (31, 31, 32, 31), (33, 65, 33, 100), (129, 64, 64, 128),
+                                        (2047, 33, 65, 100), (4096, 63, 96, 100), (30011, 3, 97, 100),
+                                        (40000, 129, 128, 100), (30000, 31, 129, 10), (20001, 65, 192, 100),
+                                        (50000, 1, 193, 128), (40003, 70, 256, 100)])
+def test_groundtruth_operand_sizes(gpu, n, nq, dim, k):
+    """the edges of the row tiles, query blocks, 16-dimension steps and operand instances; enough
+    rows per split to prime the thresholds in the larger ones"""
+    base = host.gen_mixture(n, dim, 16, 0.0, 128.0, 12.0, 0.0, 21, 22)
+    q = host.gen_mixture(nq, dim, 16, 0.0, 128.0, 12.0, 0.0, 21, 23)
+    g = search.GPUGraph(base, np.zeros((n, 1), np.uint32))
+    raw = g.groundtruth(q, k, exact_fallback=False)
+    exact = host.groundtruth(base, q, k)
+    cert = (raw != -2).all(1)
+    if k <= 100:
+        assert cert.mean() >= 0.95
+    assert np.array_equal(raw[cert], exact[cert])
+
+
+def test_groundtruth_rows_sorted_by_distance(gpu):
+    """all the near rows in one split, the nearest last (every row replaces a kept one) and first"""
+    rng = np.random.default_rng(5)
+    base = rng.standard_normal((60000, 48)).astype(np.float32)
+    q = np.zeros((40, 48), np.float32) + rng.standard_normal((40, 48)).astype(np.float32) * np.float32(0.01)
+    order = np.argsort(-(base.astype(np.float64) ** 2).sum(1))
+    for rows in (order, order[::-1]):
+        b = np.ascontiguousarray(base[rows])
+        g = search.GPUGraph(b, np.zeros((60000, 1), np.uint32))
+        raw = g.groundtruth(q, 100, exact_fallback=False)
+        cert = (raw != -2).all(1)
+        assert cert.mean() >= 0.95
+        assert np.array_equal(raw[cert], host.groundtruth(b, q, 100)[cert])
+
+
+@pytest.mark.parametrize("scale", [2.0 ** -60, 2.0 ** -20, 1.0, 2.0 ** 20, 2.0 ** 50])
+def test_groundtruth_scales(gpu, scale):
+    """fp16 operands are scaled per row: any magnitude, and queries of one block that differ by
+    2^12 from each other, stay certified"""
+    base = (host.gen_normalized(9000, 100, 31) * np.float32(scale)).astype(np.float32)
+    base[::7] *= np.float32(2.0 ** -9)
+    q = (host.gen_normalized(96, 100, 32) * np.float32(scale)).astype(np.float32)
+    q[1::3] *= np.float32(2.0 ** -12)
+    g = search.GPUGraph(base, np.zeros((9000, 1), np.uint32))
+    raw = g.groundtruth(q, 10, exact_fallback=False)
+    exact = host.groundtruth(base, q, 10)
+    cert = (raw != -2).all(1)
+    assert cert[0::3].mean() >= 0.95  # the unscaled queries
+    assert np.array_equal(raw[cert], exact[cert])
+    assert np.array_equal(g.groundtruth(q, 10), exact)
+
+
+def test_groundtruth_infinite_and_huge_rows(gpu):
+    """rows whose products overflow are candidates (never dropped), and no query is certified past them"""
+    base = host.gen_normalized(3000, 40, 41)
+    base[5] = np.float32(3.0e38)
+    base[77, 3] = np.inf
+    base[900] = 0.0
+    q = host.gen_normalized(33, 40, 42)
+    q[7] = 0.0
+    g = search.GPUGraph(base, np.zeros((3000, 1), np.uint32))
+    raw = g.groundtruth(q, 20, exact_fallback=False)
+    exact = host.groundtruth(base, q, 20)
+    cert = (raw != -2).all(1)
+    assert np.array_equal(raw[cert], exact[cert])
+    assert np.array_equal(g.groundtruth(q, 20), exact)
+    few = np.ascontiguousarray(base[:100])  # every row is a candidate: exact without a certificate
+    g = search.GPUGraph(few, np.zeros((100, 1), np.uint32))
+    assert np.array_equal(g.groundtruth(q, 100), host.groundtruth(few, q, 100))
+
+
+def test_groundtruth_in_chunks(gpu):
+    """more rows than the operand planes hold at a time (1 GiB): the lists carry over"""
+    rng = np.random.default_rng(6)
+    n = 1_070_000
+    base = rng.standard_normal((n, 256), dtype=np.float32)
+    q = rng.standard_normal((5, 256), dtype=np.float32)
+    base[n - 3] = q[0]
+    base[11] = q[1]
+    g = search.GPUGraph(base, np.zeros((n, 1), np.uint32))
+    raw = g.groundtruth(q, 100, exact_fallback=False)
+    assert (raw != -2).all()
+    assert np.array_equal(raw, host.groundtruth(base, q, 100))
