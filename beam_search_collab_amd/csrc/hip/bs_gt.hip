@@ -206,7 +206,8 @@ __device__ __forceinline__ uint64_t sort_descending(uint64_t v) {
 // 16..256; at most 0.87 over wide-ranged data), because the chain rounds 8 times less often.
 // Three fp16 products of 16 dimensions take 96 matrix cycles, eight v_mfma_f32_32x32x2f32 512.
 // 500k x 128, 10k queries: 17.1 -> 5.7 ms with the filtering below (the products alone 3.8, at
-// the rate a large bf16 matrix product reaches on the card); with it but fp32 products 12.2.
+// the rate a large bf16 matrix product reaches on the card); from three bf16 planes
+// and six products 12.2 with the filtering of one split at a time.
 // Two query blocks per wavefront (dim <= 128) halve the base bytes per product.
 //
 // The matrix pipe and the vector unit work at the same time: while tile t's products run, tile

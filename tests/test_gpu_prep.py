@@ -153,3 +153,18 @@ def test_device_vamana_reference_file(gpu, name):
     d = tempfile.mkdtemp()
     host.write_graph(f"{d}/g.bin", edges)
     assert hashlib.sha256(open(f"{d}/g.bin", "rb").read()).hexdigest() == meta["graph_sha256"]
+
+
+@pytest.mark.parametrize("n,dim,degree,beam,alpha", [(700, 15, 8, 40, 1.2), (700, 16, 64, 200, 2.0), (900, 47, 100, 150, 1.5),
+                                                     (800, 80, 33, 65, 1.1), (600, 97, 128, 300, 2.0), (900, 112, 20, 130, 1.2),
+                                                     (700, 128, 63, 64, 1.0), (500, 129, 16, 90, 1.3), (400, 161, 70, 129, 2.0)])
+def test_device_vamana_prune_sizes(gpu, n, dim, degree, beam, alpha):
+    """every row-register instance of the prune and the one without, lists of one and of several
+    blocks of 64, up to the largest degree; a hub every point reaches (mirrored lists far over
+    the degree)"""
+    rng = np.random.default_rng(n + dim)
+    base = rng.standard_normal((n, dim)).astype(np.float32)
+    base[3] = 0.0
+    base[10:14] = base[20]  # repeated points
+    want = host.build_vamana(base, degree, beam, alpha, 77, exact=True, threads=0)
+    assert np.array_equal(search.build_vamana_device(base, degree, beam, alpha, 77), want)
