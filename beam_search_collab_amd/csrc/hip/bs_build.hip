@@ -12,8 +12,9 @@
 //                  in HBM, every candidate pushed in list order under the reference's
 //                  rule "size < width or dist < tail"), the expanded nodes appended to
 //                  the point's visit list;
-//   (sort)         the visit lists by (dist, node) (segmented radix sort);
-//   vb_prune       a wavefront per list: dedupe_and_prune (build_graph.cpp:156-208) --
+//   vb_prune       a wavefront per list: the list sorted by (dist, node) (in LDS; lists over 1024
+//                  keys by a segmented radix sort before), then dedupe_and_prune
+//                  (build_graph.cpp:156-208) --
 //                  skip the node itself and repeated ids, then two passes (alpha 1, then
 //                  alpha) keeping a candidate unless alpha * d(candidate, kept) <= its
 //                  distance for a kept node;
@@ -77,6 +78,8 @@ __device__ __forceinline__ float l2_seq(const float* a, const float* b, uint32_t
     return s;
 }
 
+using f32x4 = float __attribute__((ext_vector_type(4)));
+
 struct Graph {
     const float* vecs;  // n * dstride
     uint32_t dstride, dim, deg;
@@ -89,52 +92,131 @@ struct Graph {
 // key of element e of the register-major beam (e uniform)
 template <int TR>
 __device__ __forceinline__ uint64_t beam_at(const uint64_t (&beam)[TR], uint32_t e) {
-    const uint32_t r = e >> 6;
-    uint64_t row = beam[0];
-#pragma unroll
-    for (int k = 1; k < TR; ++k) row = (r == static_cast<uint32_t>(k)) ? beam[k] : row;
-    return readlane64(row, e & 63u);
+    return readlane64(bsd::beam_reg<TR>(beam, e >> 6), e & 63u);
+}
+
+// value of the lane below; lane 0 gets `first` (one DPP move)
+__device__ __forceinline__ uint32_t lane_below(uint32_t v, uint32_t first) {
+    constexpr int WAVE_SHR1 = 0x138;
+    return static_cast<uint32_t>(
+        __builtin_amdgcn_update_dpp(static_cast<int>(first), static_cast<int>(v), WAVE_SHR1, 0xF, 0xF, false));
 }
 
 // push of one candidate key (LSB 0 = unexpanded) into the sorted beam of sz <= cap keys:
 // sorted insert, then truncation to cap (build_graph.cpp:45-89 BeamQueue::push)
 template <int TR>
 __device__ __forceinline__ void beam_insert(uint64_t (&beam)[TR], uint32_t& sz, uint32_t cap, uint64_t ck) {
-    const uint32_t lane = lane_id();
-    uint32_t pos = 0;
-#pragma unroll
-    for (int r = 0; r < TR; ++r) pos += static_cast<uint32_t>(__builtin_popcountll(ballot(beam[r] < ck)));
-    uint64_t carry[TR];
-#pragma unroll
-    for (int r = 0; r < TR; ++r) carry[r] = r == 0 ? EMPTY_KEY : readlane64(beam[r - 1], 63);
+    uint64_t lt[TR], carry[TR];  // lt: lanes whose key stays
 #pragma unroll
     for (int r = 0; r < TR; ++r) {
-        const uint32_t e = static_cast<uint32_t>(r) * 64u + lane;
-        const uint32_t plo = prev_lane(static_cast<uint32_t>(beam[r]));
-        const uint32_t phi = prev_lane(static_cast<uint32_t>(beam[r] >> 32));
-        uint64_t prv = (static_cast<uint64_t>(phi) << 32) | plo;
-        if (lane == 0) prv = carry[r];
-        uint64_t v = e < pos ? beam[r] : (e == pos ? ck : prv);
-        beam[r] = e < cap ? v : EMPTY_KEY;
+        lt[r] = ballot(beam[r] < ck);
+        carry[r] = r == 0 ? EMPTY_KEY : readlane64(beam[r - 1], 63);
+    }
+#pragma unroll
+    for (int r = 0; r < TR; ++r) {
+        const bool here = r == 0 || lt[r - 1] == ~0ull;  // the slot, the lowest that does not stay, is not below
+        const uint64_t slot = here ? ~lt[r] & (lt[r] + 1) : 0ull;
+        const uint32_t plo = lane_below(static_cast<uint32_t>(beam[r]), static_cast<uint32_t>(carry[r]));
+        const uint32_t phi = lane_below(static_cast<uint32_t>(beam[r] >> 32), static_cast<uint32_t>(carry[r] >> 32));
+        uint64_t v = (static_cast<uint64_t>(phi) << 32) | plo;
+        v = lane_in(slot) ? ck : v;
+        v = lane_in(lt[r]) ? beam[r] : v;
+        if (64u * r + 64u > cap) v = 64u * r + lane_id() < cap ? v : EMPTY_KEY;
+        beam[r] = v;
     }
     sz = sz + 1 < cap ? sz + 1 : cap;
+}
+
+// the first unexpanded key (EMPTY_KEY if none), its register and lane (EMPTY's mark bit is set)
+template <int TR>
+__device__ __forceinline__ uint64_t first_open(const uint64_t (&beam)[TR], uint32_t& pr, uint32_t& pl) {
+    uint64_t mp = 0;
+    pr = TR;
+#pragma unroll
+    for (int r = TR - 1; r >= 0; --r) {
+        const uint64_t m = ballot((static_cast<uint32_t>(beam[r]) & 1u) == 0u);
+        pr = m != 0 ? static_cast<uint32_t>(r) : pr;
+        mp = m != 0 ? m : mp;
+    }
+    if (pr == static_cast<uint32_t>(TR)) return EMPTY_KEY;
+    pl = static_cast<uint32_t>(__builtin_ctzll(mp));
+    return readlane64(bsd::beam_reg<TR>(beam, pr), pl);
+}
+
+constexpr uint32_t VS_ROWS = 32;    // rows per tile of squared differences
+constexpr uint32_t VS_S = 64 + 4;   // floats per row of a tile: 16 lanes of a b128 phase hit 16 distinct 4-bank groups
+
+// Distances of n <= 64 rows (ids in LDS, in list order) to the target, as l2_seq sums them;
+// lane j gets row j's.  Up to 32 rows x 64 dimensions at a time: loaded coalesced (16 lanes per
+// row, 4 rows per load, all loads in flight together), squared where they land, and passed
+// through LDS to the lane that adds its row's 64 terms in dimension order.
+__device__ __forceinline__ float rows_dist(const Graph& G, const float* trow, const uint32_t* ids, uint32_t n,
+                                           float* tile, float* out) {
+    const uint32_t lane = lane_id(), lr = lane >> 4, lc = (lane & 15u) * 4;
+    for (uint32_t g0 = 0; g0 < n; g0 += VS_ROWS) {
+        const uint32_t m = std::min(VS_ROWS, n - g0);
+        uint32_t id[VS_ROWS / 4];
+#pragma unroll
+        for (uint32_t t = 0; t < VS_ROWS / 4; ++t) id[t] = ids[g0 + std::min(4 * t + lr, m - 1)];
+        float s = 0.0f;
+        for (uint32_t d0 = 0; d0 < G.dstride; d0 += 64) {
+            const uint32_t c = d0 + lc < G.dstride ? d0 + lc : 0u;  // columns past the row are not added
+            f32x4 x[VS_ROWS / 4];
+#pragma unroll
+            for (uint32_t t = 0; t < VS_ROWS / 4; ++t)
+                if (4 * t < m) x[t] = *reinterpret_cast<const f32x4*>(G.vecs + static_cast<uint64_t>(id[t]) * G.dstride + c);
+            const f32x4 y = *reinterpret_cast<const f32x4*>(trow + c);
+            wave_sync();  // the previous tile's reads are done before it is overwritten
+#pragma unroll
+            for (uint32_t t = 0; t < VS_ROWS / 4; ++t)
+                if (4 * t < m) {
+                    const f32x4 d = x[t] - y;
+                    *reinterpret_cast<f32x4*>(tile + (4 * t + lr) * VS_S + lc) = d * d;
+                }
+            wave_sync();
+            const float* mine = tile + (lane & (VS_ROWS - 1)) * VS_S;
+            const uint32_t cols = std::min(64u, G.dstride - d0);  // a multiple of 16
+            for (uint32_t k = 0; k < cols; k += 16) {
+#pragma unroll
+                for (uint32_t i = 0; i < 4; ++i) {
+                    const f32x4 p = *reinterpret_cast<const f32x4*>(mine + k + 4 * i);
+                    s = s + p.x;
+                    s = s + p.y;
+                    s = s + p.z;
+                    s = s + p.w;
+                }
+            }
+        }
+        if (lane < m) out[g0 + lane] = s;
+    }
+    wave_sync();
+    return lane < n ? out[lane] : 0.0f;
 }
 
 // The greedy search of one point (build_graph.cpp:284-312), a wavefront per point.
 // out: the expanded nodes as list keys in expansion order (at most outcap; *overflow set
 // beyond); vis: this search's visited bitmap (cleared by the host before the batch).
+// A step is a chain of dependent round trips: the node's list, the visited words, the rows.  The
+// list of the next open beam entry, the likeliest next node, is requested while the current
+// node's neighbours are looked at.  (Requesting every neighbour's row beside the visited words,
+// also those that turn out to be seen, was slower at any number of searches: 0.55 against 0.43 ms
+// below.)  50k x 128, degree 32, beam 128: 0.84 -> 0.43 ms per batch of 1000.
 template <int TR>
 __global__ void __launch_bounds__(256) vb_search(const Graph G, const uint32_t* order, uint64_t start, uint64_t count,
                                                  uint32_t L, uint64_t* outk, uint32_t* outn, uint32_t outcap,
                                                  uint32_t* vis, uint64_t vis_words, uint32_t* overflow) {
-    const uint32_t lane = lane_id();
-    const uint64_t j = static_cast<uint64_t>(blockIdx.x) * 4 + uniform(threadIdx.x >> 6);
+    __shared__ __attribute__((aligned(16))) float tiles[4][VS_ROWS * VS_S];
+    __shared__ uint32_t ids_s[4][64];
+    __shared__ float dist_s[4][64];
+    const uint32_t lane = lane_id(), w = uniform(threadIdx.x >> 6);
+    const uint64_t j = static_cast<uint64_t>(blockIdx.x) * 4 + w;
     if (j >= count) return;
     const uint32_t target = order[start + j];
     const uint32_t ep = order[0];
     const float* trow = G.vecs + static_cast<uint64_t>(target) * G.dstride;
     uint32_t* vb = vis + j * vis_words;
     uint64_t* out = outk + j * outcap;
+    uint32_t* ids = ids_s[w];
     uint64_t beam[TR];
 #pragma unroll
     for (int r = 0; r < TR; ++r) beam[r] = EMPTY_KEY;
@@ -144,50 +226,62 @@ __global__ void __launch_bounds__(256) vb_search(const Graph G, const uint32_t* 
         beam_insert<TR>(beam, sz, L, bsd::make_key(d0, ep));
         if (lane == 0) vb[ep >> 5] |= 1u << (ep & 31u);
     }
-    uint32_t nout = 0;
+    // entry `lane` of a node's list (an entry past its length is not used) and its length
+    const uint32_t le = std::min(lane, G.deg - 1);
+    uint32_t nout = 0, pre = INVALID, pre_cnt = 0, pre_nb = 0;
     for (;;) {
         // the first unexpanded entry: its key, then its mark
-        uint32_t pr = TR;
-        uint64_t mp = 0;
-#pragma unroll
-        for (int r = TR - 1; r >= 0; --r) {
-            const uint64_t m = ballot((static_cast<uint32_t>(beam[r]) & 1u) == 0u && beam[r] != EMPTY_KEY);
-            pr = m != 0 ? static_cast<uint32_t>(r) : pr;
-            mp = m != 0 ? m : mp;
-        }
-        if (pr == static_cast<uint32_t>(TR)) break;
-        const uint32_t pl = static_cast<uint32_t>(__builtin_ctzll(mp));
-        const uint64_t kp = beam_at<TR>(beam, pr * 64u + pl);
+        uint32_t pr, pl = 0;
+        const uint64_t kp = first_open<TR>(beam, pr, pl);
+        if (kp == EMPTY_KEY) break;
 #pragma unroll
         for (int r = 0; r < TR; ++r)
             if (pr == static_cast<uint32_t>(r)) beam[r] |= (lane == pl) ? 1ull : 0ull;
-        const uint32_t cur = bsd::key_id(kp);
+        const uint32_t cur = uniform(bsd::key_id(kp));
         if (nout == outcap) {
             if (lane == 0) atomicOr(overflow, 1u);
             break;
         }
         if (lane == 0) out[nout] = lkey(bsd::key_dist(kp), cur);
         ++nout;
+        uint32_t cnt = pre_cnt, nb0 = pre_nb;
+        if (cur != pre) {
+            cnt = G.lcnt[cur];
+            nb0 = G.lid[static_cast<uint64_t>(cur) * G.deg + le];
+        }
+        cnt = uniform(cnt);
         // neighbours in list order; a neighbour not visited before joins the frontier
-        const uint32_t cnt = G.lcnt[cur];
         for (uint32_t k0 = 0; k0 < cnt; k0 += 64) {
             const uint32_t k = k0 + lane;
-            uint32_t nb = INVALID;
-            bool fresh = false;
-            if (k < cnt) {
-                nb = G.lid[static_cast<uint64_t>(cur) * G.deg + k];
-                const uint32_t bit = 1u << (nb & 31u);
-                fresh = (atomicOr(&vb[nb >> 5], bit) & bit) == 0u;
+            uint32_t nb = nb0;
+            if (k0 > 0) nb = G.lid[static_cast<uint64_t>(cur) * G.deg + std::min(k, cnt - 1)];
+            uint32_t seen = 0;
+            const uint32_t bit = 1u << (nb & 31u);
+            if (k < cnt) seen = atomicOr(&vb[nb >> 5], bit);
+            if (k0 == 0) {
+                uint32_t nr, nl = 0;
+                const uint64_t nk = first_open<TR>(beam, nr, nl);
+                pre = INVALID;
+                if (nk != EMPTY_KEY) {
+                    pre = uniform(bsd::key_id(nk));
+                    pre_cnt = G.lcnt[pre];
+                    pre_nb = G.lid[static_cast<uint64_t>(pre) * G.deg + le];
+                }
             }
-            float d = 0.0f;
-            if (fresh) d = l2_seq(G.vecs + static_cast<uint64_t>(nb) * G.dstride, trow, G.dim);
-            const uint64_t ck = fresh ? bsd::make_key(d, nb) : EMPTY_KEY;
-            uint64_t m = ballot(fresh);
+            const uint64_t fm = ballot(k < cnt && (seen & bit) == 0u);
+            const uint32_t n = static_cast<uint32_t>(__builtin_popcountll(fm));
+            if (n == 0) continue;
+            if (lane_in(fm)) ids[lanes_below(fm)] = nb;
+            wave_sync();
+            const float d = rows_dist(G, trow, ids, n, tiles[w], dist_s[w]);
+            uint64_t m = n == 64u ? ~0ull : (1ull << n) - 1ull;
+            const uint32_t id = ids[lane < n ? lane : 0u];
+            const uint64_t ck = lane_in(m) ? bsd::make_key(d, id) : EMPTY_KEY;
             if (sz == L && m) {
                 // a full beam's last entry only moves closer, so a candidate at or beyond it
                 // now is refused at its turn as well: only the others go through the pushes
                 const float dl = bsd::key_dist(beam_at<TR>(beam, L - 1));
-                m &= ballot(fresh && d < dl);
+                m &= ballot(d < dl);
             }
             while (m) {
                 const uint32_t l = static_cast<uint32_t>(__builtin_ctzll(m));
@@ -198,6 +292,7 @@ __global__ void __launch_bounds__(256) vb_search(const Graph G, const uint32_t* 
                 if (!take) take = bsd::key_dist(c) < bsd::key_dist(beam_at<TR>(beam, sz - 1));
                 if (take) beam_insert<TR>(beam, sz, L, c);
             }
+            wave_sync();  // ids are read before the next block writes them
         }
     }
     if (lane == 0) outn[j] = nout;
@@ -205,7 +300,6 @@ __global__ void __launch_bounds__(256) vb_search(const Graph G, const uint32_t* 
 
 // A vector read through the scalar cache: its address is the same in every lane, so the values
 // arrive in scalar registers and the vector unit takes them as operands.
-using f32x4 = float __attribute__((ext_vector_type(4)));
 using const_row = const __attribute__((address_space(4))) f32x4*;
 __device__ __forceinline__ const_row uniform_row(const Graph& G, uint32_t id) {
     return reinterpret_cast<const_row>(reinterpret_cast<uintptr_t>(G.vecs + static_cast<uint64_t>(uniform(id)) * G.dstride));
@@ -347,6 +441,38 @@ __device__ __forceinline__ void prune_list(const Graph& G, uint64_t* keys, uint3
     if (lane == 0) G.lcnt[src] = kc;
 }
 
+constexpr uint32_t SORT_CAP = 1024;  // keys a wavefront sorts in its LDS slice
+
+// n <= SORT_CAP keys sorted ascending into S (LDS): up to 64 across the lanes, more by a bitonic
+// network in LDS over the next power of two, padded with EMPTY keys
+__device__ __forceinline__ void sort_list(const uint64_t* keys, uint32_t n, uint64_t* S) {
+    const uint32_t lane = lane_id();
+    if (n <= 64) {
+        const uint64_t v = bsd::sort_lanes(lane < n ? keys[lane] : EMPTY_KEY, n);
+        S[lane] = v;
+        wave_sync();
+        return;
+    }
+    uint32_t N = 128;
+    while (N < n) N <<= 1;
+    for (uint32_t i = lane; i < N; i += 64) S[i] = i < n ? keys[i] : EMPTY_KEY;
+    wave_sync();
+#pragma unroll 1
+    for (uint32_t k = 2; k <= N; k <<= 1) {
+#pragma unroll 1
+        for (uint32_t j = k >> 1; j >= 1; j >>= 1) {
+            for (uint32_t i = lane; i < N / 2; i += 64) {
+                const uint32_t a = ((i & ~(j - 1u)) << 1) | (i & (j - 1u));
+                const uint64_t x = S[a], y = S[a + j];
+                const bool sw = (a & k) == 0 ? (y < x) : (x < y);
+                S[a] = sw ? y : x;
+                S[a + j] = sw ? x : y;
+            }
+            wave_sync();
+        }
+    }
+}
+
 // m rows of dim floats to rows of dstride, zero past dim
 __global__ void __launch_bounds__(256) vb_pad_rows(const float* rows, uint64_t m, uint32_t dim, uint32_t dstride,
                                                    float* out) {
@@ -357,21 +483,44 @@ __global__ void __launch_bounds__(256) vb_pad_rows(const float* rows, uint64_t m
     out[t] = d < dim ? rows[i * dim + d] : 0.0f;
 }
 
-// the batch's visit lists: job j = (sorted keys at j * outcap, outn[j] keys, order[start + j])
-template <int D4>
+// the batch's visit lists: job j = (keys at j * outcap, outn[j] keys, order[start + j]).  SORT:
+// the lists are unsorted and at most SORT_CAP keys; else sorted in memory
+template <int D4, bool SORT>
 __global__ void __launch_bounds__(256) vb_prune_targets(const Graph G, uint64_t* keys, const uint32_t* outn,
                                                         uint32_t outcap, const uint32_t* order, uint64_t start,
                                                         uint64_t count, float alpha) {
     __shared__ uint64_t kept_s[4][128];
+    __shared__ uint64_t sort_s[SORT ? 4 : 1][SORT ? SORT_CAP : 1];
     const uint32_t w = uniform(threadIdx.x >> 6);
     const uint64_t j = static_cast<uint64_t>(blockIdx.x) * 4 + w;
     if (j >= count) return;
-    prune_list<D4>(G, keys + j * outcap, outn[j], order[start + j], alpha, kept_s[w]);
+    const uint32_t n = uniform(outn[j]), src = uniform(order[start + j]);
+    if constexpr (SORT) {
+        sort_list(keys + j * outcap, n, sort_s[w]);
+        prune_list<D4>(G, sort_s[w], n, src, alpha, kept_s[w]);
+    } else {
+        prune_list<D4>(G, keys + j * outcap, n, src, alpha, kept_s[w]);
+    }
 }
+
+// segment j of the visit lists for the sort in memory: [j * outcap, j * outcap + outn[j])
+__global__ void __launch_bounds__(256) vb_segments(const uint32_t* outn, uint32_t outcap, uint64_t count,
+                                                   uint64_t* begin, uint64_t* end) {
+    const uint64_t j = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (j >= count) return;
+    begin[j] = j * outcap;
+    end[j] = j * outcap + outn[j];
+}
+
+// what a batch's kernels count, read by the host once per batch
+struct Counters {
+    unsigned long long records, big_keys;  // mirrored edges, keys of the lists to prune
+    uint32_t overflow, heads, big, longest;  // searches over their list, targets, lists to prune and the longest
+};
 
 // mirrored edges: record (j, k) of the batch -> key (target << 32 | j * deg + k), or ~0
 __global__ void __launch_bounds__(256) vb_rev_keys(const Graph G, const uint32_t* order, uint64_t start,
-                                                   uint64_t count, uint64_t* rk, unsigned long long* nvalid) {
+                                                   uint64_t count, uint64_t* rk, Counters* ctr) {
     const uint64_t t = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
     if (t >= count * G.deg) return;
     const uint64_t j = t / G.deg;
@@ -380,7 +529,7 @@ __global__ void __launch_bounds__(256) vb_rev_keys(const Graph G, const uint32_t
     uint64_t key = ~0ull;
     if (k < G.lcnt[src]) {
         key = (static_cast<uint64_t>(G.lid[static_cast<uint64_t>(src) * G.deg + k]) << 32) | static_cast<uint32_t>(t);
-        atomicAdd(nvalid, 1ull);
+        atomicAdd(&ctr->records, 1ull);
     }
     rk[t] = key;
 }
@@ -404,10 +553,10 @@ __device__ __forceinline__ uint32_t scan_wave(uint32_t v, uint32_t& total) {
 // also registers a prune job (target, offset of its old + new keys in `big`, their number), its
 // index + 1 in the head's last word.  One atomic per wavefront and counter: with one per
 // head, in vb_rev_apply, that kernel took 214 us per batch of 1000 points, now 7.
-__global__ void __launch_bounds__(256) vb_rev_heads(const Graph G, const uint64_t* rk, uint64_t m, uint4* heads,
-                                                    unsigned int* nheads, unsigned long long* bigtotal,
-                                                    uint4* bigjobs, unsigned int* nbig) {
+__global__ void __launch_bounds__(256) vb_rev_heads(const Graph G, const uint64_t* rk, uint4* heads, uint4* bigjobs,
+                                                    Counters* ctr) {
     const uint32_t lane = lane_id();
+    const uint64_t m = ctr->records;
     const uint64_t i = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
     const uint32_t dst = i < m ? static_cast<uint32_t>(rk[i] >> 32) : INVALID;
     const bool head = i < m && (i == 0 || static_cast<uint32_t>(rk[i - 1] >> 32) != dst);
@@ -440,12 +589,13 @@ __global__ void __launch_bounds__(256) vb_rev_heads(const Graph G, const uint64_
     unsigned int h0 = 0, b0 = 0;
     unsigned long long off0 = 0;
     if (lane == 0) {
-        h0 = atomicAdd(nheads, static_cast<unsigned int>(__builtin_popcountll(hm)));
+        h0 = atomicAdd(&ctr->heads, static_cast<uint32_t>(__builtin_popcountll(hm)));
         if (bm) {
-            b0 = atomicAdd(nbig, static_cast<unsigned int>(__builtin_popcountll(bm)));
-            off0 = atomicAdd(bigtotal, static_cast<unsigned long long>(sum));
+            b0 = atomicAdd(&ctr->big, static_cast<uint32_t>(__builtin_popcountll(bm)));
+            off0 = atomicAdd(&ctr->big_keys, static_cast<unsigned long long>(sum));
         }
     }
+    if (isbig && tot > 64u) atomicMax(&ctr->longest, tot);
     h0 = readlane(h0, 0);
     b0 = readlane(b0, 0);
     const uint64_t off = readlane64(off0, 0) + before;
@@ -514,16 +664,23 @@ __global__ void __launch_bounds__(256) vb_big_offsets(const uint4* bigjobs, unsi
     end[i] = off + jb.w;
 }
 
-template <int D4>
+template <int D4, bool SORT>
 __global__ void __launch_bounds__(256) vb_prune_big(const Graph G, uint64_t* keys, const uint4* bigjobs,
                                                     unsigned int nbig, float alpha) {
     __shared__ uint64_t kept_s[4][128];
+    __shared__ uint64_t sort_s[SORT ? 4 : 1][SORT ? SORT_CAP : 1];
     const uint32_t w = uniform(threadIdx.x >> 6);
     const uint64_t i = static_cast<uint64_t>(blockIdx.x) * 4 + w;
     if (i >= nbig) return;
     const uint4 jb = bigjobs[i];
     const uint64_t off = (static_cast<uint64_t>(jb.z) << 32) | jb.y;
-    prune_list<D4>(G, keys + off, jb.w, jb.x, alpha, kept_s[w]);
+    const uint32_t n = uniform(jb.w), src = uniform(jb.x);
+    if constexpr (SORT) {
+        sort_list(keys + off, n, sort_s[w]);
+        prune_list<D4>(G, sort_s[w], n, src, alpha, kept_s[w]);
+    } else {
+        prune_list<D4>(G, keys + off, n, src, alpha, kept_s[w]);
+    }
 }
 
 // the final dedupe_and_prune of every node (build_graph.cpp:382-390): its list (at most
@@ -641,17 +798,17 @@ extern "C" int bs_build_vamana_device(const float* vecs, uint64_t n, uint32_t di
     const uint64_t vis_words = (n + 31) / 32;
     const uint64_t slots = std::max<uint64_t>(1, std::min<uint64_t>(max_batch, (2ull << 30) / (vis_words * 4)));
 
-    DevBuf d_vecs, d_lid, d_ld, d_lcnt, d_order, d_vis, d_outk, d_outs, d_outn, d_flag, d_rk, d_rks, d_heads, d_nh,
-        d_nvalid, d_big, d_bigs, d_bigtot, d_bigjobs, d_nbig, d_beg, d_end, d_segb, d_sege, d_edges, d_tmp;
+    DevBuf d_vecs, d_lid, d_ld, d_lcnt, d_order, d_vis, d_outk, d_outs, d_outn, d_rk, d_rks, d_heads, d_ctr, d_big, d_bigs,
+        d_bigjobs, d_beg, d_end, d_segb, d_sege, d_edges, d_tmp;
     auto alloc = [&](DevBuf& b, size_t bytes) { return hipMalloc(&b.p, std::max<size_t>(bytes, 8)) == hipSuccess; };
     const uint64_t mrec = max_batch * degree;
     const uint64_t bigcap = mrec * (static_cast<uint64_t>(degree) + 1);
     if (!alloc(d_vecs, n * dstride * 4ull) || !alloc(d_lid, n * degree * 4ull) || !alloc(d_ld, n * degree * 4ull) ||
         !alloc(d_lcnt, n * 4ull) || !alloc(d_order, n * 4ull) || !alloc(d_vis, slots * vis_words * 4ull) ||
         !alloc(d_outk, slots * outcap * 8ull) || !alloc(d_outs, slots * outcap * 8ull) || !alloc(d_outn, slots * 4ull) ||
-        !alloc(d_flag, 4) || !alloc(d_rk, mrec * 8ull) || !alloc(d_rks, mrec * 8ull) || !alloc(d_heads, mrec * 16ull) ||
-        !alloc(d_nh, 4) || !alloc(d_nvalid, 8) || !alloc(d_big, bigcap * 8ull) || !alloc(d_bigs, bigcap * 8ull) ||
-        !alloc(d_bigtot, 8) || !alloc(d_bigjobs, mrec * 16ull) || !alloc(d_nbig, 4) || !alloc(d_beg, mrec * 8ull) ||
+        !alloc(d_rk, mrec * 8ull) || !alloc(d_rks, mrec * 8ull) || !alloc(d_heads, mrec * 16ull) ||
+        !alloc(d_ctr, sizeof(bvb::Counters)) || !alloc(d_big, bigcap * 8ull) || !alloc(d_bigs, bigcap * 8ull) ||
+        !alloc(d_bigjobs, mrec * 16ull) || !alloc(d_beg, mrec * 8ull) ||
         !alloc(d_end, mrec * 8ull) || !alloc(d_segb, slots * 8ull) || !alloc(d_sege, slots * 8ull) ||
         !alloc(d_edges, n * degree * 4ull))
         return vfail(BS_ENOMEM, "hipMalloc of the graph-construction buffers failed");
@@ -676,12 +833,12 @@ extern "C" int bs_build_vamana_device(const float* vecs, uint64_t n, uint32_t di
     }
     if (e == hipSuccess) e = hipMemcpy(d_order.p, order.data(), n * 4ull, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemset(d_lcnt.p, 0, n * 4ull);
-    if (e == hipSuccess) e = hipMemset(d_flag.p, 0, 4);
     if (e != hipSuccess) return vfail(BS_EHIP, std::string("graph construction upload: ") + hipGetErrorString(e));
 
     bvb::Graph G{d_vecs.as<float>(), dstride, dim, degree, n, d_lid.as<uint32_t>(), d_ld.as<float>(),
                  d_lcnt.as<uint32_t>()};
     const uint32_t* ord = d_order.as<uint32_t>();
+    bvb::Counters* ctr = d_ctr.as<bvb::Counters>();
 
     if (slots * outcap > 0x7FFFFFFFull || bigcap > 0x7FFFFFFFull || mrec > 0xFFFFFFFFull)
         return vfail(BS_EINVAL, "batch too large for the device sorts (n or beam width too large)");
@@ -708,10 +865,11 @@ extern "C" int bs_build_vamana_device(const float* vecs, uint64_t n, uint32_t di
 
     uint64_t start = 1;
     double last_print = 0.0;
-    std::vector<uint64_t> segb(slots), sege(slots);
-    std::vector<uint32_t> outn(slots);
+    // visit lists short enough are sorted by the kernel that prunes them
+    const bool sort_here = outcap <= bvb::SORT_CAP;
     while (start < n) {
         const uint64_t end = std::min(std::min(start * 2, start + batch_bound), n);
+        e = hipMemsetAsync(ctr, 0, sizeof(bvb::Counters), nullptr);
         // 1. searches and visit-list prunes, `slots` points at a time
         for (uint64_t s0 = start; e == hipSuccess && s0 < end; s0 += slots) {
             const uint64_t cnt = std::min(slots, end - s0);
@@ -722,84 +880,77 @@ extern "C" int bs_build_vamana_device(const float* vecs, uint64_t n, uint32_t di
                 constexpr int T = decltype(trc)::value;
                 hipLaunchKernelGGL(bvb::vb_search<T>, wg, dim3(256), 0, nullptr, G, ord, s0, cnt, beam_width,
                                    d_outk.as<uint64_t>(), d_outn.as<uint32_t>(), outcap, d_vis.as<uint32_t>(),
-                                   vis_words, d_flag.as<uint32_t>());
+                                   vis_words, &ctr->overflow);
             });
-            if (e != hipSuccess) break;
-            uint32_t flag = 0;
-            e = hipMemcpy(outn.data(), d_outn.p, cnt * 4ull, hipMemcpyDeviceToHost);
-            if (e == hipSuccess) e = hipMemcpy(&flag, d_flag.p, 4, hipMemcpyDeviceToHost);
-            if (e != hipSuccess) break;
-            if (flag) return vfail(BS_EINVAL, "a search expanded more than " + std::to_string(outcap) + " nodes");
-            for (uint64_t j = 0; j < cnt; ++j) {
-                segb[j] = j * outcap;
-                sege[j] = j * outcap + outn[j];
+            if (e == hipSuccess && !sort_here) {
+                hipLaunchKernelGGL(bvb::vb_segments, dim3(static_cast<uint32_t>((cnt + 255) / 256)), dim3(256), 0, nullptr,
+                                   d_outn.as<uint32_t>(), outcap, cnt, d_segb.as<uint64_t>(), d_sege.as<uint64_t>());
+                e = hipGetLastError();
+                if (e == hipSuccess)
+                    e = hipcub::DeviceSegmentedRadixSort::SortKeys(d_tmp.p, tmp_bytes, d_outk.as<uint64_t>(),
+                                                                   d_outs.as<uint64_t>(), static_cast<int>(cnt * outcap),
+                                                                   static_cast<int>(cnt), d_segb.as<uint64_t>(),
+                                                                   d_sege.as<uint64_t>());
             }
-            e = hipMemcpy(d_segb.p, segb.data(), cnt * 8ull, hipMemcpyHostToDevice);
-            if (e == hipSuccess) e = hipMemcpy(d_sege.p, sege.data(), cnt * 8ull, hipMemcpyHostToDevice);
             if (e == hipSuccess)
-                e = hipcub::DeviceSegmentedRadixSort::SortKeys(d_tmp.p, tmp_bytes, d_outk.as<uint64_t>(),
-                                                               d_outs.as<uint64_t>(), static_cast<int>(cnt * outcap),
-                                                               static_cast<int>(cnt), d_segb.as<uint64_t>(),
-                                                               d_sege.as<uint64_t>());
-            if (e != hipSuccess) break;
-            e = launch_d4(dstride, [&](auto d4) {
-                constexpr int D = decltype(d4)::value;
-                hipLaunchKernelGGL(bvb::vb_prune_targets<D>, wg, dim3(256), 0, nullptr, G, d_outs.as<uint64_t>(),
-                                   d_outn.as<uint32_t>(), outcap, ord, s0, cnt, alpha);
-            });
+                e = launch_d4(dstride, [&](auto d4) {
+                    constexpr int D = decltype(d4)::value;
+                    auto go = [&](auto k, uint64_t* lists) {
+                        hipLaunchKernelGGL(k, wg, dim3(256), 0, nullptr, G, lists, d_outn.as<uint32_t>(), outcap, ord, s0,
+                                           cnt, alpha);
+                    };
+                    if (sort_here) go(bvb::vb_prune_targets<D, true>, d_outk.as<uint64_t>());
+                    else go(bvb::vb_prune_targets<D, false>, d_outs.as<uint64_t>());
+                });
         }
         if (e != hipSuccess) break;
         // 2. mirrored edges in batch order
         const uint64_t bcnt = end - start, m = bcnt * degree;
-        e = hipMemsetAsync(d_nvalid.p, 0, 8, nullptr);
-        if (e == hipSuccess) e = hipMemsetAsync(d_nh.p, 0, 4, nullptr);
-        if (e == hipSuccess) e = hipMemsetAsync(d_nbig.p, 0, 4, nullptr);
-        if (e == hipSuccess) e = hipMemsetAsync(d_bigtot.p, 0, 8, nullptr);
-        if (e != hipSuccess) break;
-        hipLaunchKernelGGL(bvb::vb_rev_keys, dim3(static_cast<uint32_t>((m + 255) / 256)), dim3(256), 0, nullptr, G,
-                           ord, start, bcnt, d_rk.as<uint64_t>(), d_nvalid.as<unsigned long long>());
+        const dim3 mg(static_cast<uint32_t>((m + 255) / 256));
+        hipLaunchKernelGGL(bvb::vb_rev_keys, mg, dim3(256), 0, nullptr, G, ord, start, bcnt, d_rk.as<uint64_t>(), ctr);
         e = hipGetLastError();
         if (e == hipSuccess)
             e = hipcub::DeviceRadixSort::SortKeys(d_tmp.p, tmp_bytes, d_rk.as<uint64_t>(), d_rks.as<uint64_t>(),
                                                   static_cast<int>(m));
-        unsigned long long mv = 0;
-        if (e == hipSuccess) e = hipMemcpy(&mv, d_nvalid.p, 8, hipMemcpyDeviceToHost);
+        if (e == hipSuccess) {
+            hipLaunchKernelGGL(bvb::vb_rev_heads, mg, dim3(256), 0, nullptr, G, d_rks.as<uint64_t>(), d_heads.as<uint4>(),
+                               d_bigjobs.as<uint4>(), ctr);
+            e = hipGetLastError();
+        }
+        // the batch's one wait for the device
+        bvb::Counters c = {};
+        if (e == hipSuccess) e = hipMemcpy(&c, ctr, sizeof(c), hipMemcpyDeviceToHost);
         if (e != hipSuccess) break;
-        if (mv) {
-            hipLaunchKernelGGL(bvb::vb_rev_heads, dim3(static_cast<uint32_t>((mv + 255) / 256)), dim3(256), 0, nullptr, G,
-                               d_rks.as<uint64_t>(), static_cast<uint64_t>(mv), d_heads.as<uint4>(),
-                               d_nh.as<unsigned int>(), d_bigtot.as<unsigned long long>(), d_bigjobs.as<uint4>(),
-                               d_nbig.as<unsigned int>());
-            unsigned int nh = 0, nbig = 0;
+        if (c.overflow) return vfail(BS_EINVAL, "a search expanded more than " + std::to_string(outcap) + " nodes");
+        if (c.heads) {
+            hipLaunchKernelGGL(bvb::vb_rev_apply, dim3((c.heads + 3) / 4), dim3(256), 0, nullptr, G, d_rks.as<uint64_t>(),
+                               d_heads.as<uint4>(), c.heads, ord, start, d_big.as<uint64_t>(), d_bigjobs.as<uint4>());
             e = hipGetLastError();
-            if (e == hipSuccess) e = hipMemcpy(&nh, d_nh.p, 4, hipMemcpyDeviceToHost);
-            if (e != hipSuccess) break;
-            hipLaunchKernelGGL(bvb::vb_rev_apply, dim3((nh + 3) / 4), dim3(256), 0, nullptr, G, d_rks.as<uint64_t>(),
-                               d_heads.as<uint4>(), nh, ord, start, d_big.as<uint64_t>(), d_bigjobs.as<uint4>());
-            e = hipGetLastError();
-            if (e == hipSuccess) e = hipMemcpy(&nbig, d_nbig.p, 4, hipMemcpyDeviceToHost);
-            if (e != hipSuccess) break;
-            if (nbig) {
-                unsigned long long tot = 0;
-                e = hipMemcpy(&tot, d_bigtot.p, 8, hipMemcpyDeviceToHost);
-                if (e != hipSuccess) break;
-                hipLaunchKernelGGL(bvb::vb_big_offsets, dim3((nbig + 255) / 256), dim3(256), 0, nullptr,
-                                   d_bigjobs.as<uint4>(), nbig, d_beg.as<uint64_t>(), d_end.as<uint64_t>());
+        }
+        if (e == hipSuccess && c.big) {
+            const bool here = c.longest <= bvb::SORT_CAP;
+            if (!here) {
+                hipLaunchKernelGGL(bvb::vb_big_offsets, dim3((c.big + 255) / 256), dim3(256), 0, nullptr,
+                                   d_bigjobs.as<uint4>(), c.big, d_beg.as<uint64_t>(), d_end.as<uint64_t>());
                 e = hipGetLastError();
                 if (e == hipSuccess)
                     e = hipcub::DeviceSegmentedRadixSort::SortKeys(d_tmp.p, tmp_bytes, d_big.as<uint64_t>(),
-                                                                   d_bigs.as<uint64_t>(), static_cast<int>(tot),
-                                                                   static_cast<int>(nbig), d_beg.as<uint64_t>(),
+                                                                   d_bigs.as<uint64_t>(), static_cast<int>(c.big_keys),
+                                                                   static_cast<int>(c.big), d_beg.as<uint64_t>(),
                                                                    d_end.as<uint64_t>());
-                if (e != hipSuccess) break;
+            }
+            if (e == hipSuccess)
                 e = launch_d4(dstride, [&](auto d4) {
                     constexpr int D = decltype(d4)::value;
-                    hipLaunchKernelGGL(bvb::vb_prune_big<D>, dim3((nbig + 3) / 4), dim3(256), 0, nullptr, G,
-                                       d_bigs.as<uint64_t>(), d_bigjobs.as<uint4>(), nbig, alpha);
+                    auto go = [&](auto k, uint64_t* lists) {
+                        hipLaunchKernelGGL(k, dim3((c.big + 3) / 4), dim3(256), 0, nullptr, G, lists, d_bigjobs.as<uint4>(),
+                                           c.big, alpha);
+                    };
+                    if (here) go(bvb::vb_prune_big<D, true>, d_big.as<uint64_t>());
+                    else go(bvb::vb_prune_big<D, false>, d_bigs.as<uint64_t>());
                 });
-                if (e != hipSuccess) break;
-            }
         }
+        if (e != hipSuccess) break;
         if (verbose) {
             e = hipDeviceSynchronize();
             const double el = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();

@@ -168,3 +168,14 @@ def test_device_vamana_prune_sizes(gpu, n, dim, degree, beam, alpha):
     base[10:14] = base[20]  # repeated points
     want = host.build_vamana(base, degree, beam, alpha, 77, exact=True, threads=0)
     assert np.array_equal(search.build_vamana_device(base, degree, beam, alpha, 77), want)
+
+
+def test_device_vamana_hub(gpu):
+    """a point nearest to all others: its mirrored list passes what a wavefront sorts in LDS
+    (1024 keys), so the lists of those batches are sorted in memory"""
+    rng = np.random.default_rng(9)
+    base = rng.standard_normal((56000, 40)).astype(np.float32)
+    base /= np.linalg.norm(base, axis=1, keepdims=True)
+    base[17] = 0.0
+    want = host.build_vamana(base, 8, 16, 1.2, 3, exact=True, threads=0)
+    assert np.array_equal(search.build_vamana_device(base, 8, 16, 1.2, 3), want)
