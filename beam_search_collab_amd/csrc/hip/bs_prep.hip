@@ -8,10 +8,11 @@
 //
 // build_rabitq (src/build_rabitq.cpp:59-99,138-264): the same two steps in double for the
 // codebook's medoid, every node's rotation WHT(signs * [v, 0...]) once, then a thread per
-// edge for the residual, its 1-bit code and the float parts of its factors, in the
-// reference's operation order; the three factor products, which the reference forms in
-// long double, are finished on the host.
+// edge for the residual, its 1-bit code and its factors, in the reference's operation order;
+// the three factor products, which the reference forms in long double, are made in integers
+// with the same roundings (bs_ext.hpp).
 #include "bs_hip.h"
+#include "bs_ext.hpp"
 #include "wave.hpp"
 
 #include <hip/hip_runtime.h>
@@ -331,51 +332,104 @@ __global__ void __launch_bounds__(256) rq_rotate(const float* vecs, uint32_t dst
 
 // Thread per edge (build_rabitq.cpp:217-256): residual = v_rot - u_rot over the first
 // dim components; sqr_r, the code bits, bin_sum, fac_x0 and fac_x1 accumulate in
-// dimension order as in the reference's loops.  out: (r_norm, fac_x0 / r_norm,
-// fac_x1 * fac_norm, bin_sum); an absent neighbour gets bin_sum = -1.
+// dimension order as in the reference's loops; then the factors (tx | fdq | fvq per node).
+// A wavefront's 64 neighbour rows pass through its LDS tile 32 dimensions (one code word) at a
+// time: loaded coalesced, 8 lanes per 128-byte piece of a row, 8 rows per load, read back by the
+// edge's lane.  Bound by the gather of 4 pdim bytes per edge: 200k x 128, degree 32, 3.3 GB
+// in 0.47 ms (2.52 when each lane walked its own row in 16-byte loads).
+// RAW: out gets (r_norm, fac_x0 / r_norm, fac_x1 * fac_norm, bin_sum; an absent neighbour
+// bin_sum = -1) instead of the factors; without it an edge whose parts are not finite sets *odd.
+constexpr uint32_t RE_S = 32 + 4;  // floats per row of a tile (9 16-byte pieces: no bank conflicts)
+
+template <bool RAW>
 __global__ void __launch_bounds__(256) rq_edges(const float* rot, const uint32_t* edges, uint64_t ne, uint32_t R,
                                                 uint32_t dim, uint32_t pdim, uint32_t wpp, float fac_norm,
-                                                uint32_t* codes, float4* out) {
-    const uint64_t e = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (e >= ne) return;
+                                                uint32_t* codes, float4* out, float* factors, uint32_t* odd) {
+    __shared__ __attribute__((aligned(16))) float tiles[4][64 * RE_S];
+    __shared__ uint32_t ids_s[4][64];
+    const uint32_t lane = lane_id(), w = uniform(threadIdx.x >> 6);
+    const uint64_t e0 = (static_cast<uint64_t>(blockIdx.x) * 4 + w) * 64;
+    if (e0 >= ne) return;
+    const uint64_t e = std::min<uint64_t>(e0 + lane, ne - 1);  // lanes past the end repeat the last edge
+    const bool mine = e0 + lane < ne;
     const uint32_t v = edges[e];
+    const bool absent = v == 0xFFFFFFFFu;
+    const uint64_t u = e / R;
+    float* tile = tiles[w];
+    uint32_t* ids = ids_s[w];
+    ids[lane] = absent ? 0u : v;
+    wave_sync();
+    const uint32_t lr = lane >> 3, lc = (lane & 7u) * 4;
+    uint32_t rows[8];
+#pragma unroll
+    for (uint32_t t = 0; t < 8; ++t) rows[t] = ids[8 * t + lr];
+    const f32x4* ur = reinterpret_cast<const f32x4*>(rot + u * pdim);
     uint32_t* cw = codes + e * wpp;
-    if (v == 0xFFFFFFFFu) {
-        for (uint32_t w = 0; w < wpp; ++w) cw[w] = 0u;
-        out[e] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(-1));
-        return;
-    }
-    const float4* ur = reinterpret_cast<const float4*>(rot + (e / R) * pdim);
-    const float4* vr = reinterpret_cast<const float4*>(rot + static_cast<uint64_t>(v) * pdim);
     float sqr = 0.0f, fx0 = 0.0f, fx1 = 0.0f;
     int bin_sum = 0;
-    uint32_t word = 0;
-    for (uint32_t d4 = 0; d4 * 4 < dim; ++d4) {
-        const float4 a = vr[d4], b = ur[d4];
-        const float av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
+    uint32_t word4[4] = {0, 0, 0, 0};
+    for (uint32_t k = 0; k < wpp; ++k) {
+        const uint32_t d0 = k * 32;
+        uint32_t word = 0;
+        if (d0 < dim) {
+            f32x4 x[8];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t d = d4 * 4 + j;
-            if (d < dim) {
-                const float res = av[j] - bv[j];
-                sqr = sqr + res * res;
-                const bool pos = res > 0.0f;
-                word |= pos ? (1u << (d & 31u)) : 0u;
-                bin_sum += pos ? 1 : 0;
-                const float sv = pos ? 1.0f : -1.0f;
-                fx0 = fx0 + res * sv * fac_norm;
-                fx1 = fx1 + bv[j] * sv;
+            for (uint32_t t = 0; t < 8; ++t)
+                x[t] = *reinterpret_cast<const f32x4*>(rot + static_cast<uint64_t>(rows[t]) * pdim + d0 + lc);
+            wave_sync();  // the previous tile's reads are done before it is overwritten
+#pragma unroll
+            for (uint32_t t = 0; t < 8; ++t) *reinterpret_cast<f32x4*>(tile + (8 * t + lr) * RE_S + lc) = x[t];
+            wave_sync();
+            const f32x4* vr = reinterpret_cast<const f32x4*>(tile + lane * RE_S);
+            auto four = [&](uint32_t q, uint32_t n) __attribute__((always_inline)) {
+                const f32x4 a = vr[q], b = ur[d0 / 4 + q];
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j) {
+                    if (j >= n) break;
+                    const float res = a[j] - b[j];
+                    sqr = sqr + res * res;
+                    const bool pos = res > 0.0f;
+                    word |= pos ? 1u << (4 * q + j) : 0u;
+                    fx0 = fx0 + __builtin_fabsf(res) * fac_norm;  // res * sign, exactly
+                    fx1 = fx1 + (pos ? b[j] : -b[j]);
+                }
+            };
+            if (d0 + 32 <= dim) {
+#pragma unroll
+                for (uint32_t q = 0; q < 8; ++q) four(q, 4);
+            } else {
+                for (uint32_t q = 0; d0 + 4 * q < dim; ++q) four(q, dim - d0 - 4 * q);
             }
-            if (d < dim && (d & 31u) == 31u) {
-                cw[d >> 5] = word;
-                word = 0;
-            }
+            if (absent) word = 0;
+            bin_sum += __builtin_popcount(word);
+        }
+        if (wpp >= 4) {  // a multiple of 4: one 16-byte store per four words
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) word4[j] = (k & 3u) == j ? word : word4[j];
+            if ((k & 3u) == 3u && mine)
+                *reinterpret_cast<uint4*>(cw + (k & ~3u)) = make_uint4(word4[0], word4[1], word4[2], word4[3]);
+        } else if (mine) {
+            cw[k] = word;
         }
     }
-    for (uint32_t w = (dim + 31) / 32; w < wpp; ++w) cw[w] = 0u;
-    if (dim & 31u) cw[dim >> 5] = word;
     const float r_norm = sqrtf(sqr) + 1e-10f;
-    out[e] = make_float4(r_norm, fx0 / r_norm, fx1 * fac_norm, __int_as_float(bin_sum));
+    const float x0 = fx0 / r_norm, x1 = fx1 * fac_norm;
+    if constexpr (RAW) {
+        if (mine) out[e] = absent ? make_float4(0.0f, 0.0f, 0.0f, __int_as_float(-1))
+                                  : make_float4(r_norm, x0, x1, __int_as_float(bin_sum));
+    } else {
+        float tx = FLT_MAX, dq = 0.0f, vq = 0.0f;
+        const bool fine = __builtin_isfinite(r_norm) && __builtin_isfinite(x0) && __builtin_isfinite(x1);
+        if (!absent && fine)
+            bsx::rabitq_factors(r_norm, x0, x1, fac_norm, static_cast<float>(2 * bin_sum - static_cast<int>(dim)), tx, dq, vq);
+        if (mine) {
+            float* f = factors + u * 3 * R + (e - u * R);
+            f[0] = tx;
+            f[R] = dq;
+            f[2 * R] = vq;
+            if (!absent && !fine) *odd = 1u;
+        }
+    }
 }
 
 }  // namespace bsp
@@ -464,6 +518,7 @@ extern "C" int bs_index_build_rabitq(bs_index idx, uint32_t seed, uint32_t* code
     float* d_rot = nullptr;
     uint32_t* d_codes = nullptr;
     float4* d_out = nullptr;
+    float* d_fac = nullptr;
     double* d_cent = nullptr;
     double* d_dist = nullptr;
     unsigned long long* d_best = nullptr;
@@ -473,22 +528,22 @@ extern "C" int bs_index_build_rabitq(bs_index idx, uint32_t seed, uint32_t* code
         if (d_rot) (void)hipFree(d_rot);
         if (d_codes) (void)hipFree(d_codes);
         if (d_out) (void)hipFree(d_out);
+        if (d_fac) (void)hipFree(d_fac);
         if (d_cent) (void)hipFree(d_cent);
         if (d_dist) (void)hipFree(d_dist);
         if (d_best) (void)hipFree(d_best);
         if (d_index) (void)hipFree(d_index);
     };
     if (hipMalloc(&d_signs, pdim * sizeof(float)) != hipSuccess || hipMalloc(&d_rot, n * pdim * sizeof(float)) != hipSuccess ||
-        hipMalloc(&d_codes, ne * wpp * sizeof(uint32_t)) != hipSuccess || hipMalloc(&d_out, ne * sizeof(float4)) != hipSuccess ||
+        hipMalloc(&d_codes, ne * wpp * sizeof(uint32_t)) != hipSuccess || hipMalloc(&d_fac, ne * 3 * sizeof(float)) != hipSuccess ||
         hipMalloc(&d_cent, dim * sizeof(double)) != hipSuccess || hipMalloc(&d_dist, n * sizeof(double)) != hipSuccess ||
-        hipMalloc(&d_best, sizeof(unsigned long long)) != hipSuccess || hipMalloc(&d_index, sizeof(uint32_t)) != hipSuccess) {
+        hipMalloc(&d_best, sizeof(unsigned long long)) != hipSuccess || hipMalloc(&d_index, 2 * sizeof(uint32_t)) != hipSuccess) {
         release();
         return pfail(BS_ENOMEM, "hipMalloc of the codebook work buffers failed");
     }
-    std::vector<float4> st(ne);
-    const uint32_t init_index = 0xFFFFFFFFu;
+    const uint32_t init_index[2] = {0xFFFFFFFFu, 0u};  // the medoid, the flag of non-finite edges
     hipError_t e = hipMemcpy(d_signs, signs_out, pdim * sizeof(float), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(d_index, &init_index, sizeof(init_index), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(d_index, init_index, sizeof(init_index), hipMemcpyHostToDevice);
     // medoid (find_medoid, build_rabitq.cpp:59-99) in double
     const size_t lds = bsp::EP_LDS;
     if (e == hipSuccess)
@@ -519,17 +574,34 @@ extern "C" int bs_index_build_rabitq(bs_index idx, uint32_t seed, uint32_t* code
         e = hipGetLastError();
     }
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(bsp::rq_edges, dim3(static_cast<uint32_t>((ne + 255) / 256)), dim3(256), 0, nullptr, d_rot,
-                           edges, ne, R, dim, pdim, wpp, fac_norm, d_codes, d_out);
+        hipLaunchKernelGGL(bsp::rq_edges<false>, dim3(static_cast<uint32_t>((ne + 255) / 256)), dim3(256), 0, nullptr, d_rot,
+                           edges, ne, R, dim, pdim, wpp, fac_norm, d_codes, nullptr, d_fac, d_index + 1);
         e = hipGetLastError();
     }
-    uint32_t medoid = 0;
-    if (e == hipSuccess) e = hipMemcpy(&medoid, d_index, sizeof(medoid), hipMemcpyDeviceToHost);
+    uint32_t index[2] = {0, 0};
+    if (e == hipSuccess) e = hipMemcpy(index, d_index, sizeof(index), hipMemcpyDeviceToHost);
     if (e == hipSuccess) e = hipMemcpy(codes_out, d_codes, ne * wpp * sizeof(uint32_t), hipMemcpyDeviceToHost);
-    if (e == hipSuccess) e = hipMemcpy(st.data(), d_out, ne * sizeof(float4), hipMemcpyDeviceToHost);
+    if (e == hipSuccess && !index[1]) e = hipMemcpy(factors_out, d_fac, ne * 3 * sizeof(float), hipMemcpyDeviceToHost);
+    // infinite or NaN vectors: the edges' float parts come to the host, which has the
+    // reference's long double for them
+    std::vector<float4> st;
+    if (e == hipSuccess && index[1]) {
+        (void)hipFree(d_fac);
+        d_fac = nullptr;
+        st.resize(ne);
+        if (hipMalloc(&d_out, ne * sizeof(float4)) != hipSuccess) {
+            release();
+            return pfail(BS_ENOMEM, "hipMalloc of the codebook work buffers failed");
+        }
+        hipLaunchKernelGGL(bsp::rq_edges<true>, dim3(static_cast<uint32_t>((ne + 255) / 256)), dim3(256), 0, nullptr, d_rot,
+                           edges, ne, R, dim, pdim, wpp, fac_norm, d_codes, d_out, nullptr, nullptr);
+        e = hipGetLastError();
+        if (e == hipSuccess) e = hipMemcpy(st.data(), d_out, ne * sizeof(float4), hipMemcpyDeviceToHost);
+    }
     release();
     if (e != hipSuccess) return pfail(BS_EHIP, std::string("rabitq codebook: ") + hipGetErrorString(e));
-    *entry_out = medoid == 0xFFFFFFFFu ? 0u : medoid;  // no row below DBL_MAX: row 0, as the reference
+    *entry_out = index[0] == 0xFFFFFFFFu ? 0u : index[0];  // no row below DBL_MAX: row 0, as the reference
+    if (st.empty()) return BS_OK;
 
     // the factor products in long double (build_rabitq.cpp:250-256), on the host threads
     auto finish = [&](uint64_t u0, uint64_t u1) {

@@ -175,9 +175,10 @@ int bs_index_entry_point(bs_index idx, uint32_t* entry);
  * residual of the rotated vectors, its 1-bit code and the factors (tx | fdq | fvq), entry =
  * medoid with a double centroid -- byte-identical to bs_build_rabitq (bs_host.h).  Host
  * outputs: codes n*degree*(pdim/32) u32, factors n*3*degree f32, signs pdim f32, entry.
- * The float work runs on the device; the factor products the reference forms in long
- * double are finished on the host.  Synchronous; allocates work buffers (rotations
- * n*pdim f32, codes, 16 B per edge).  dim > 16. */
+ * The factor products the reference forms in long double are made on the device in integers
+ * with the same roundings (edges of infinite or NaN vectors: on the host, in long double).
+ * Synchronous; allocates work buffers (rotations
+ * n*pdim f32, codes, 12 B per edge).  dim > 16. */
 int bs_index_build_rabitq(bs_index idx, uint32_t seed, uint32_t* codes, float* factors, float* signs,
                           uint32_t* entry);
 

@@ -179,3 +179,38 @@ def test_device_vamana_hub(gpu):
     base[17] = 0.0
     want = host.build_vamana(base, 8, 16, 1.2, 3, exact=True, threads=0)
     assert np.array_equal(search.build_vamana_device(base, 8, 16, 1.2, 3), want)
+
+
+@pytest.mark.parametrize("n,dim,degree", [(65, 17, 1), (300, 32, 3), (257, 33, 33), (130, 64, 64), (200, 96, 20),
+                                          (400, 127, 32), (150, 129, 100), (90, 700, 7)])
+def test_device_codebook_edge_sizes(gpu, n, dim, degree):
+    """code words and tiles at their edges, missing neighbours, residuals of zero (infinite
+    factors), far and near rows: the host builder's bytes"""
+    rng = np.random.default_rng(n + dim)
+    base = (rng.standard_normal((n, dim)) * rng.choice([1e-18, 1e-3, 1.0, 1e4], (n, 1))).astype(np.float32)
+    base[7] = base[3]
+    base[11] = 0.0
+    edges = rng.integers(0, n, (n, degree)).astype(np.uint32)
+    edges[rng.random((n, degree)) < 0.1] = 0xFFFFFFFF
+    edges[:, 0] = np.arange(n)  # the node itself
+    edges[3, -1] = 7
+    g = search.GPUGraph(base, edges)
+    got, want = g.build_rabitq(99), host.build_rabitq(base, edges, 99)
+    assert got[0] == want[0]
+    for a, b in zip(got[1:], want[1:]):
+        assert a.tobytes() == b.tobytes()
+
+
+def test_device_codebook_infinite_rows(gpu):
+    """an edge whose parts are not finite sends the factor products to the host"""
+    rng = np.random.default_rng(3)
+    base = rng.standard_normal((100, 40)).astype(np.float32)
+    base[9, 4] = np.inf
+    base[30] = np.float32(3e38)
+    edges = rng.integers(0, 100, (100, 12)).astype(np.uint32)
+    g = search.GPUGraph(base, edges)
+    got, want = g.build_rabitq(5), host.build_rabitq(base, edges, 5)
+    assert got[1].tobytes() == want[1].tobytes()
+    assert np.array_equal(np.isnan(got[2]), np.isnan(want[2]))
+    ok = ~np.isnan(want[2])
+    assert np.array_equal(got[2][ok], want[2][ok])
