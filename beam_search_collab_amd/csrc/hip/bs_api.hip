@@ -87,51 +87,16 @@ constexpr uint64_t ORDER_MIN_NQ = 4096;     // mode 1 orders launches of at leas
 // is resident 14 times per CU, not the 15 that 160 KB / 10848 B suggests)
 constexpr uint32_t LDS_GRANULE = 512;
 
-// Pivots for query scheduling: ORDER_P rows spread evenly over the index (all rows when
-// n is smaller), re-ordered by a greedy nearest-neighbour tour so that consecutive
-// labels are near in space.  Returns the transposed pivots and their squared norms.
-void make_pivots(const float* vecs, uint64_t n, uint32_t dim, std::vector<float>& pivT, std::vector<float>& pnorm) {
-    const uint32_t P = bso::ORDER_P;
-    const uint32_t m = static_cast<uint32_t>(std::min<uint64_t>(P, n));
-    std::vector<uint64_t> rows(m);
-    for (uint32_t i = 0; i < m; ++i) rows[i] = static_cast<uint64_t>(i) * n / m;
-    std::vector<uint32_t> tour;
-    std::vector<char> used(m, 0);
-    uint32_t cur = 0;
-    used[0] = 1;
-    tour.push_back(0);
-    while (tour.size() < m) {
-        const float* a = vecs + rows[cur] * dim;
-        double best = DBL_MAX;
-        uint32_t bi = 0;
-        for (uint32_t j = 0; j < m; ++j) {
-            if (used[j]) continue;
-            const float* b = vecs + rows[j] * dim;
-            double d = 0;
-            for (uint32_t k = 0; k < dim; ++k) {
-                const double t = static_cast<double>(a[k]) - b[k];
-                d += t * t;
-            }
-            if (d < best) {
-                best = d;
-                bi = j;
-            }
-        }
-        used[bi] = 1;
-        tour.push_back(bi);
-        cur = bi;
-    }
-    pivT.assign(static_cast<size_t>((dim + 15) & ~15u) * P, 0.0f);  // rows for whole blocks of 16
-    pnorm.assign(P, 1e30f);  // unused slots never win
-    for (uint32_t t = 0; t < m; ++t) {
-        const float* v = vecs + rows[tour[t]] * dim;
-        double nn = 0;
-        for (uint32_t k = 0; k < dim; ++k) {
-            pivT[static_cast<size_t>(k) * P + t] = v[k];
-            nn += static_cast<double>(v[k]) * v[k];
-        }
-        pnorm[t] = static_cast<float>(nn);
-    }
+// the first edge that is neither a node nor 0xFFFFFFFF, as an error (the kernels gather rows
+// without bounds checks); BS_OK if every edge is fine
+int edge_error(const uint32_t* edges, uint64_t i, uint64_t n) {
+    return fail(BS_EINVAL, "edge " + std::to_string(i) + " points to node " + std::to_string(edges[i]) +
+                               " >= n = " + std::to_string(n));
+}
+int check_edges_host(const uint32_t* edges, uint64_t cnt, uint64_t n) {
+    for (uint64_t i = 0; i < cnt; ++i)
+        if (edges[i] != 0xFFFFFFFFu && edges[i] >= n) return edge_error(edges, i, n);
+    return BS_OK;
 }
 // the device address of bs_search_device_noalloc's static workspace (defined below)
 int noalloc_workspace(int dev, uint32_t** out);
@@ -176,15 +141,14 @@ extern "C" int bs_index_create(const float* vecs, const uint32_t* edges, uint64_
     if (n == 0 || n > 0x7FFFFFFFull) return fail(BS_EINVAL, "need 0 < n < 2^31");
     if (dim == 0 || dim > 1024) return fail(BS_EINVAL, "dim must be in 1..1024");
     if (degree == 0 || degree > 256) return fail(BS_EINVAL, "degree must be in 1..256");
-    // every neighbour id must address a node (the kernels gather rows without bounds checks)
-    for (uint64_t i = 0, cnt = n * degree; i < cnt; ++i) {
-        const uint32_t e = edges[i];
-        if (e != 0xFFFFFFFFu && e >= n)
-            return fail(BS_EINVAL, "edge " + std::to_string(i) + " points to node " + std::to_string(e) +
-                                       " >= n = " + std::to_string(n));
-    }
+    // every neighbour id must address a node: checked on the device after the upload, here only
+    // where there is none
     int rc = check_device();
-    if (rc) return rc;
+    if (rc) {
+        const std::string why = g_err;
+        const int bad = check_edges_host(edges, n * degree, n);
+        return bad ? bad : fail(rc, why);
+    }
     int device = 0;
     HIP_TRY(hipGetDevice(&device));
     {
@@ -226,23 +190,38 @@ extern "C" int bs_index_create(const float* vecs, const uint32_t* edges, uint64_
     if (ix->dstride == dim) {
         e = hipMemcpy(ix->d_vecs, vecs, vbytes, hipMemcpyHostToDevice);
     } else {
-        e = hipMemset(ix->d_vecs, 0, vbytes);
-        if (e == hipSuccess)
-            e = hipMemcpy2D(ix->d_vecs, ix->dstride * sizeof(float), vecs, dim * sizeof(float), dim * sizeof(float),
-                            n, hipMemcpyHostToDevice);
+        // the rows as they are, up to 256 MiB at a time, spread to their padded places by a kernel
+        const uint64_t rows = std::min<uint64_t>(n, std::max<uint64_t>(1, (256ull << 20) / (dim * sizeof(float))));
+        float* stage = nullptr;
+        e = hipMalloc(&stage, rows * dim * sizeof(float));
+        for (uint64_t r0 = 0; e == hipSuccess && r0 < n; r0 += rows) {
+            const uint64_t m = std::min(rows, n - r0);
+            e = hipMemcpy(stage, vecs + r0 * dim, m * dim * sizeof(float), hipMemcpyHostToDevice);
+            if (e == hipSuccess)
+                e = bso::launch_pad_rows(stage, m, dim, ix->dstride, ix->d_vecs + r0 * ix->dstride, nullptr);
+        }
+        if (stage) (void)hipFree(stage);  // waits for the kernel
     }
     if (e == hipSuccess) e = hipMemcpy(ix->d_edges, edges, n * degree * sizeof(uint32_t), hipMemcpyHostToDevice);
+    unsigned long long bad = ~0ull;  // the first edge out of range
     if (e == hipSuccess) {
-        std::vector<float> pivT, pnorm;
-        make_pivots(vecs, n, dim, pivT, pnorm);
         const size_t ows = (2 * ORDER_CHUNK + 2 * bso::ORDER_P) * sizeof(uint32_t);
-        e = hipMalloc(&ix->d_pivT, pivT.size() * sizeof(float));
-        if (e == hipSuccess) e = hipMalloc(&ix->d_pnorm, pnorm.size() * sizeof(float));
+        const size_t pt = static_cast<size_t>((dim + 15) & ~15u) * bso::ORDER_P;  // rows for whole blocks of 16
+        e = hipMalloc(&ix->d_pivT, pt * sizeof(float));
+        if (e == hipSuccess) e = hipMalloc(&ix->d_pnorm, bso::ORDER_P * sizeof(float));
         if (e == hipSuccess) e = hipMalloc(&ix->d_ows, ows);
-        if (e == hipSuccess) e = hipMemcpy(ix->d_pivT, pivT.data(), pivT.size() * sizeof(float), hipMemcpyHostToDevice);
-        if (e == hipSuccess) e = hipMemcpy(ix->d_pnorm, pnorm.data(), pnorm.size() * sizeof(float), hipMemcpyHostToDevice);
-        if (e == hipSuccess) e = hipMemset(ix->d_ows, 0, ows);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&ix->ws_free, hipEventDisableTiming);
+        // d_ows holds the pivots' distances and their tour, and the edge check's answer, before
+        // it starts its life as the zeroed order workspace
+        if (e == hipSuccess) e = bso::launch_check_edges(ix->d_edges, n * degree, n, reinterpret_cast<unsigned long long*>(ix->d_ows), nullptr);
+        if (e == hipSuccess) e = hipMemcpy(&bad, ix->d_ows, sizeof(bad), hipMemcpyDeviceToHost);
+        if (e == hipSuccess && bad == ~0ull)
+            e = bso::launch_pivots(ix->d_vecs, ix->dstride, dim, n, ix->d_ows, ix->d_pivT, ix->d_pnorm, nullptr);
+        if (e == hipSuccess && bad == ~0ull) e = hipMemsetAsync(ix->d_ows, 0, ows, nullptr);
+    }
+    if (e == hipSuccess && bad != ~0ull) {
+        bs_index_destroy(ix);
+        return edge_error(edges, bad, n);
     }
     if (e != hipSuccess) {
         bs_index_destroy(ix);

@@ -28,6 +28,7 @@
 // per pair, so every comparison sees the reference's values.
 #include "bs_hip.h"
 #include "bs_device.hpp"
+#include "bs_order.hpp"
 
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
@@ -473,16 +474,6 @@ __device__ __forceinline__ void sort_list(const uint64_t* keys, uint32_t n, uint
     }
 }
 
-// m rows of dim floats to rows of dstride, zero past dim
-__global__ void __launch_bounds__(256) vb_pad_rows(const float* rows, uint64_t m, uint32_t dim, uint32_t dstride,
-                                                   float* out) {
-    const uint64_t t = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (t >= m * dstride) return;
-    const uint64_t i = t / dstride;
-    const uint32_t d = static_cast<uint32_t>(t - i * dstride);
-    out[t] = d < dim ? rows[i * dim + d] : 0.0f;
-}
-
 // the batch's visit lists: job j = (keys at j * outcap, outn[j] keys, order[start + j]).  SORT:
 // the lists are unsorted and at most SORT_CAP keys; else sorted in memory
 template <int D4, bool SORT>
@@ -825,9 +816,7 @@ extern "C" int bs_build_vamana_device(const float* vecs, uint64_t n, uint32_t di
             const uint64_t m = std::min(rows, n - r0);
             e = hipMemcpy(stage.p, vecs + r0 * dim, m * dim * 4ull, hipMemcpyHostToDevice);
             if (e != hipSuccess) break;
-            hipLaunchKernelGGL(bvb::vb_pad_rows, dim3(static_cast<uint32_t>((m * dstride + 255) / 256)), dim3(256), 0,
-                               nullptr, stage.as<float>(), m, dim, dstride, d_vecs.as<float>() + r0 * dstride);
-            e = hipGetLastError();
+            e = bso::launch_pad_rows(stage.as<float>(), m, dim, dstride, d_vecs.as<float>() + r0 * dstride, nullptr);
         }
         if (e == hipSuccess) e = hipDeviceSynchronize();  // the staging buffer is freed
     }

@@ -480,12 +480,162 @@ __global__ void __launch_bounds__(1024) label_cost(const uint32_t* labels, const
     }
 }
 
+// The least index of an edge that is neither below n nor 0xFFFFFFFF (*bad starts as all ones).
+// Bound by reading the edges once: 25 MB in ~15 us, where the host's loop took 2.5 ms.
+__global__ void __launch_bounds__(256) check_edges(const uint32_t* edges, uint64_t cnt, uint64_t n,
+                                                   unsigned long long* bad) {
+    unsigned long long first = ~0ull;
+    for (uint64_t i = (static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x) * 4; i < cnt;
+         i += static_cast<uint64_t>(gridDim.x) * 1024) {
+        uint4 v = make_uint4(0u, 0u, 0u, 0u);  // node 0 exists
+        if (i + 4 <= cnt) {
+            v = *reinterpret_cast<const uint4*>(edges + i);
+        } else {
+            v.x = edges[i];
+            if (i + 1 < cnt) v.y = edges[i + 1];
+            if (i + 2 < cnt) v.z = edges[i + 2];
+        }
+        const uint32_t e[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int j = 3; j >= 0; --j)
+            if (e[j] >= n && e[j] != 0xFFFFFFFFu && i + j < first) first = i + j;
+    }
+    if (first != ~0ull) atomicMin(bad, first);
+}
+
+hipError_t launch_check_edges(const uint32_t* edges, uint64_t cnt, uint64_t n, unsigned long long* bad, hipStream_t s) {
+    hipError_t e = hipMemsetAsync(bad, 0xFF, sizeof(*bad), s);
+    if (e != hipSuccess) return e;
+    const uint64_t blocks = (cnt + 1023) / 1024;
+    hipLaunchKernelGGL(check_edges, dim3(static_cast<uint32_t>(blocks < 2048 ? blocks : 2048)), dim3(256), 0, s, edges, cnt,
+                       n, bad);
+    return hipGetLastError();
+}
+
+// Pivots for query scheduling: m = min(ORDER_P, n) rows spread evenly over the index, in the
+// order of a greedy nearest-neighbour tour from the first (so that consecutive labels are near
+// in space).  The same tour as a host loop over double sums in dimension order.  (On the host
+// the 32640 distances took 4 ms at 128 dimensions; here 0.3 ms, most of it the tour's 255
+// dependent steps.)
+// A thread per pair: the squared distance as the bits of a non-negative double (all ones if it
+// is not below DBL_MAX, which the tour never takes).
+__global__ void __launch_bounds__(ORDER_P) pivot_dist(const float* vecs, uint32_t dstride, uint32_t dim, uint64_t n,
+                                                      uint32_t m, unsigned long long* dist) {
+    const uint32_t i = blockIdx.x, j = threadIdx.x;
+    if (j >= m) return;
+    const float* a = vecs + (static_cast<uint64_t>(i) * n / m) * dstride;
+    const float* b = vecs + (static_cast<uint64_t>(j) * n / m) * dstride;
+    double d = 0.0;
+    uint32_t k = 0;
+    for (; k + 4 <= dim; k += 4) {
+        const float4 x = *reinterpret_cast<const float4*>(a + k), y = *reinterpret_cast<const float4*>(b + k);
+        double t = static_cast<double>(x.x) - y.x;
+        d += t * t;
+        t = static_cast<double>(x.y) - y.y;
+        d += t * t;
+        t = static_cast<double>(x.z) - y.z;
+        d += t * t;
+        t = static_cast<double>(x.w) - y.w;
+        d += t * t;
+    }
+    for (; k < dim; ++k) {
+        const double t = static_cast<double>(a[k]) - b[k];
+        d += t * t;
+    }
+    dist[i * ORDER_P + j] = d < 1.7976931348623157e308 ? static_cast<unsigned long long>(__double_as_longlong(d)) : ~0ull;
+}
+
+// One workgroup: tour[t], the pivot (row number of the m) at place t.  Each step takes the
+// nearest unused pivot, the lowest of equals (pivot 0 if no distance is finite).
+__global__ void __launch_bounds__(ORDER_P) pivot_tour(uint32_t m, const unsigned long long* dist, uint32_t* tour) {
+    __shared__ unsigned long long key_s[2][4];
+    __shared__ uint32_t idx_s[2][4];
+    const uint32_t j = threadIdx.x, lane = lane_id(), w = uniform(threadIdx.x >> 6);
+    bool used = j == 0 || j >= m;
+    uint32_t cur = 0;
+    if (j == 0) tour[0] = 0;
+    for (uint32_t t = 1; t < m; ++t) {
+        const uint64_t k = used ? ~0ull : dist[cur * ORDER_P + j];
+        uint64_t v = k, o;
+        o = xor_lane64<1>(v); v = o < v ? o : v;
+        o = xor_lane64<2>(v); v = o < v ? o : v;
+        o = xor_lane64<4>(v); v = o < v ? o : v;
+        o = xor_lane64<8>(v); v = o < v ? o : v;
+        o = xor_lane64<16>(v); v = o < v ? o : v;
+        o = xor_lane64<32>(v); v = o < v ? o : v;
+        const uint64_t at = ballot(k == v);
+        const uint32_t h = t & 1u;  // two sets of slots: one barrier per step
+        if (lane == 0) {
+            key_s[h][w] = v;
+            idx_s[h][w] = 64 * w + static_cast<uint32_t>(__builtin_ctzll(at));
+        }
+        __syncthreads();
+        uint64_t best = key_s[h][0];
+        uint32_t bi = idx_s[h][0];
+#pragma unroll
+        for (int x = 1; x < 4; ++x)
+            if (key_s[h][x] < best) {
+                best = key_s[h][x];
+                bi = idx_s[h][x];
+            }
+        cur = uniform(best == ~0ull ? 0u : bi);
+        used = used || j == cur;
+        if (j == 0) tour[t] = cur;
+    }
+}
+
+// pivT (dim16 rows of ORDER_P, the rows past dim and the columns past m zero) and the pivots'
+// squared norms (1e30 past m: never the nearest)
+__global__ void __launch_bounds__(ORDER_P) pivot_rows(const float* vecs, uint32_t dstride, uint32_t dim, uint32_t dim16,
+                                                      uint64_t n, uint32_t m, const uint32_t* tour, float* pivT,
+                                                      float* pnorm) {
+    const uint32_t t = threadIdx.x;
+    const float* v = vecs + (static_cast<uint64_t>(t < m ? tour[t] : 0u) * n / m) * dstride;
+    for (uint32_t k = blockIdx.x; k < dim16; k += gridDim.x) pivT[static_cast<uint64_t>(k) * ORDER_P + t] = t < m && k < dim ? v[k] : 0.0f;
+    if (blockIdx.x != 0) return;
+    double nn = 0.0;
+    for (uint32_t k = 0; k < dim; ++k) nn += static_cast<double>(v[k]) * v[k];
+    pnorm[t] = t < m ? static_cast<float>(nn) : 1e30f;
+}
+
+// ws: ORDER_P * ORDER_P distances of 8 bytes and the tour
+hipError_t launch_pivots(const float* vecs, uint32_t dstride, uint32_t dim, uint64_t n, uint32_t* ws, float* pivT,
+                         float* pnorm, hipStream_t s) {
+    const uint32_t m = static_cast<uint32_t>(n < ORDER_P ? n : ORDER_P), dim16 = (dim + 15) & ~15u;
+    unsigned long long* dist = reinterpret_cast<unsigned long long*>(ws);
+    uint32_t* tour = ws + 2 * ORDER_P * ORDER_P;
+    hipLaunchKernelGGL(pivot_dist, dim3(m), dim3(ORDER_P), 0, s, vecs, dstride, dim, n, m, dist);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(pivot_tour, dim3(1), dim3(ORDER_P), 0, s, m, dist, tour);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(pivot_rows, dim3(dim16 < 64 ? dim16 : 64), dim3(ORDER_P), 0, s, vecs, dstride, dim, dim16, n, m, tour,
+                       pivT, pnorm);
+    return hipGetLastError();
+}
+
 __global__ void __launch_bounds__(256) gather_rows(const float* vecs, uint32_t dstride, uint32_t dim, uint64_t n,
                                                    uint32_t m, float* out) {
     const uint64_t e = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
     if (e >= static_cast<uint64_t>(m) * dim) return;
     const uint64_t i = e / dim, k = e - i * dim;
     out[e] = vecs[(i * n / m) * dstride + k];
+}
+
+__global__ void __launch_bounds__(256) pad_rows(const float* rows, uint64_t m, uint32_t dim, uint32_t dstride,
+                                                float* out) {
+    const uint64_t t = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (t >= m * dstride) return;
+    const uint64_t i = t / dstride;
+    const uint32_t d = static_cast<uint32_t>(t - i * dstride);
+    out[t] = d < dim ? rows[i * dim + d] : 0.0f;
+}
+
+hipError_t launch_pad_rows(const float* rows, uint64_t m, uint32_t dim, uint32_t dstride, float* out, hipStream_t s) {
+    hipLaunchKernelGGL(pad_rows, dim3(static_cast<uint32_t>((m * dstride + 255) / 256)), dim3(256), 0, s, rows, m, dim,
+                       dstride, out);
+    return hipGetLastError();
 }
 
 hipError_t launch_place(const OrderParams& o, hipStream_t s) {

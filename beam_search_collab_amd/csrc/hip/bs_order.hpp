@@ -58,6 +58,16 @@ hipError_t launch_label_cost(const uint32_t* labels, const uint32_t* per_query, 
 hipError_t launch_gather_rows(const float* vecs, uint32_t dstride, uint32_t dim, uint64_t n, uint32_t m, float* out,
                               hipStream_t s);
 
+// *bad = the least index of an edge that is neither below n nor 0xFFFFFFFF, or all ones
+hipError_t launch_check_edges(const uint32_t* edges, uint64_t cnt, uint64_t n, unsigned long long* bad, hipStream_t s);
+
+// the pivots (pivT, pnorm of OrderParams) of the rows; ws: 2 * ORDER_P * (ORDER_P + 1) words
+hipError_t launch_pivots(const float* vecs, uint32_t dstride, uint32_t dim, uint64_t n, uint32_t* ws, float* pivT,
+                         float* pnorm, hipStream_t s);
+
+// m rows of dim floats to rows of dstride, zero past dim
+hipError_t launch_pad_rows(const float* rows, uint64_t m, uint32_t dim, uint32_t dstride, float* out, hipStream_t s);
+
 // Launch map by predicted cost, longest first (nq >= 1): on entry key[q] holds query q's
 // cost signal as a float (larger = longer), on return its bucket; o.X and o.start are
 // ignored (one run).  Up to 65536 queries one workgroup does it all (cost_order_one);

@@ -519,3 +519,18 @@ def test_label_costs_calibration(gpu):
     tiny = dataset(40, 32, 8, 5)  # fewer rows than pivots: every label still has a cost
     ct = tiny["g"].label_costs()
     assert np.isfinite(ct).all() and (ct >= 1).all()
+
+
+@pytest.mark.parametrize("n,degree,where", [(5, 1, 0), (5, 1, 4), (7, 3, 20), (1000, 33, 17), (1000, 33, 32999),
+                                            (300000, 8, 2399999)])
+def test_index_rejects_first_bad_edge(gpu, n, degree, where):
+    """the device's edge check names the first edge out of range, at its quads' edges and past
+    one grid; 0xFFFFFFFF stays allowed"""
+    base = np.zeros((n, 4), np.float32)
+    edges = np.zeros((n, degree), np.uint32)
+    edges.reshape(-1)[::3] = 0xFFFFFFFF
+    search.GPUGraph(base, edges).close()
+    edges.reshape(-1)[where:] = n + 7
+    edges.reshape(-1)[where] = n
+    with pytest.raises(ValueError, match=f"edge {where} points to node {n} "):
+        search.GPUGraph(base, edges)
