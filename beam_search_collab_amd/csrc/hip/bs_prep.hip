@@ -28,6 +28,7 @@
 int bs_internal_vecs(bs_index idx, const float** vecs, uint32_t* dstride);
 int bs_internal_edges(bs_index idx, const uint32_t** edges);
 void bs_internal_set_error(const std::string& msg);
+hipError_t bs_internal_download(bs_index idx, void* dst, const void* src, size_t bytes);
 int bs_internal_exception();
 
 namespace bsp {
@@ -580,8 +581,8 @@ extern "C" int bs_index_build_rabitq(bs_index idx, uint32_t seed, uint32_t* code
     }
     uint32_t index[2] = {0, 0};
     if (e == hipSuccess) e = hipMemcpy(index, d_index, sizeof(index), hipMemcpyDeviceToHost);
-    if (e == hipSuccess) e = hipMemcpy(codes_out, d_codes, ne * wpp * sizeof(uint32_t), hipMemcpyDeviceToHost);
-    if (e == hipSuccess && !index[1]) e = hipMemcpy(factors_out, d_fac, ne * 3 * sizeof(float), hipMemcpyDeviceToHost);
+    if (e == hipSuccess) e = bs_internal_download(idx, codes_out, d_codes, ne * wpp * sizeof(uint32_t));
+    if (e == hipSuccess && !index[1]) e = bs_internal_download(idx, factors_out, d_fac, ne * 3 * sizeof(float));
     // infinite or NaN vectors: the edges' float parts come to the host, which has the
     // reference's long double for them
     std::vector<float4> st;
