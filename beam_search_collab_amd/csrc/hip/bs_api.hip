@@ -450,11 +450,15 @@ int make_plan(bs_index ix, const bs_search_cfg* cfg, uint64_t nq, Plan& pl) {
     if (cap > (1u << 22)) return fail(BS_EINVAL, "filter_capacity must be <= 2^22");
 
     pl.mode = mode;
+    // Base-family beams of 1025..1536 keys get 24 registers: every merge, pick and re-fill walks
+    // them all (32 registers took 100k x 75, 777 queries, topk 1500 9.73 ms against 8.36; 50k x
+    // 64 bwarp1, 2000 queries, topk 1100 4.80 against 3.94; 100k x 128, 10k queries, topk 1100 58.4
+    // against 51.3).
     // RaBitQ beams of 513..640 and 641..768 keys get 10 and 12 registers (the recall@10 0.95
     // point of config C is topk 640: 1M x 128, 10k queries, 6.31 ms with 12 registers)
     pl.TR = T <= 64 ? 1 : T <= 128 ? 2 : T <= 256 ? 4 : T <= 512 ? 8
           : (T <= 640 && mode == BS_RABITQ) ? 10 : (T <= 768 && mode == BS_RABITQ) ? 12
-          : T <= 1024 ? 16 : T <= 2048 ? 32 : 64;
+          : T <= 1024 ? 16 : (T <= 1536 && mode != BS_RABITQ) ? 24 : T <= 2048 ? 32 : 64;
     pl.CR = ix->degree <= 64 ? 1 : ix->degree <= 128 ? 2 : 4;
     // RaBitQ with narrow codes (dim <= 128): one chunk per lane (bsd::l2_shape_lanes)
     const bool narrow_rq = mode == BS_RABITQ && ix->wpp <= 4;

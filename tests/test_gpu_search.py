@@ -534,3 +534,21 @@ def test_index_rejects_first_bad_edge(gpu, n, degree, where):
     edges.reshape(-1)[where] = n
     with pytest.raises(ValueError, match=f"edge {where} points to node {n} "):
         search.GPUGraph(base, edges)
+
+
+@pytest.mark.parametrize("topk", [1024, 1025, 1100, 1473, 1535, 1536, 1537])
+@pytest.mark.parametrize("mode,degree", [("base", 24), ("warp2", 70), ("bwarp1", 33)])
+def test_beams_of_24_registers(gpu, topk, mode, degree):
+    """base-family beams of 1025..1536 keys (24 registers) and their neighbours of 16 and 32"""
+    base = host.gen_mixture(4000, 50, 8, 0.0, 128.0, 20.0, 0.0, 5, 6)
+    q = host.gen_mixture(9, 50, 8, 0.0, 128.0, 20.0, 0.0, 5, 7)
+    rng = np.random.default_rng(topk + degree)
+    edges = rng.integers(0, 4000, (4000, degree)).astype(np.uint32)
+    g = search.GPUGraph(base, edges)
+    oi = po.OracleIndex(base, edges)
+    omode = po.BASE_BLOOM if mode.startswith("bwarp") else po.BASE_HASH
+    cfg = GPUBaseSearchCfg(topk, 4096, 11, 900, 40)
+    ids, d, _ = g.search(q, 1000, mode, cfg, with_dists=True)
+    oids, od, _ = oi.search(q, 1000, omode, topk, 11, 900, 4096, 40)
+    assert np.array_equal(ids, oids)
+    assert d.tobytes() == od.tobytes()
