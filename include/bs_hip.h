@@ -66,8 +66,8 @@ typedef struct {
 
 /* Limits against the reference: degree 1..256 and dim 1..1024 as gpu_cli (gpu_cli.cu:208-233,
  * 340-347).  topk_size 1..4096 (any value, not only multiples of 32): the beam is held in the
- * wavefront's registers, 64 keys per register, in 1..16 registers up to 1024 keys and in 32 or
- * 64 above (the RaBitQ expanded set in the wavefront's LDS slice); the reference's
+ * wavefront's registers, 64 keys per register, in 1..16 registers up to 1024 keys and in 24, 32
+ * or 64 above (the RaBitQ expanded set in the wavefront's LDS slice); the reference's
  * SharedBitonicTopK (topk_shared.cuh:272-331) takes multiples of 32 in shared memory, bounded by
  * the shared memory per block.  Beams above 4096 are refused with BS_EINVAL.  With topk_size >=
  * filter_capacity a base search admits no new nodes once its table is full, as the reference's
@@ -87,7 +87,7 @@ typedef struct {
 
 /* Upload a graph: vecs n*dim f32, edges n*degree u32 (ids < n or 0xFFFFFFFF).
  * Replaces GPUGraph(const CPUGraph&) (gpu_graph.cuh:81-146).  Validates every edge on
- * the host.  dim 1..1024, degree 1..256 (the reference gpu_cli's range), n < 2^31.  Also
+ * the device.  dim 1..1024, degree 1..256 (the reference gpu_cli's range), n < 2^31.  Also
  * prepares the query scheduling: 256 pivot rows, and the expected search cost per pivot
  * region (about 7 ms at 1M x 128: the entry point and a base search of 16384 index rows;
  * without it, which a failure there leaves, the scheduling uses the plain label order). */
@@ -177,8 +177,7 @@ int bs_index_entry_point(bs_index idx, uint32_t* entry);
  * outputs: codes n*degree*(pdim/32) u32, factors n*3*degree f32, signs pdim f32, entry.
  * The factor products the reference forms in long double are made on the device in integers
  * with the same roundings (edges of infinite or NaN vectors: on the host, in long double).
- * Synchronous; allocates work buffers (rotations
- * n*pdim f32, codes, 12 B per edge).  dim > 16. */
+ * Synchronous; allocates work buffers (rotations n*pdim f32, codes, 12 B per edge).  dim > 16. */
 int bs_index_build_rabitq(bs_index idx, uint32_t seed, uint32_t* codes, float* factors, float* signs,
                           uint32_t* entry);
 
@@ -187,8 +186,8 @@ int bs_index_build_rabitq(bs_index idx, uint32_t seed, uint32_t* codes, float* f
  * distances, dedupe_and_prune and mirrored-edge order, so edges_out (host, n*degree u32,
  * rows padded with node 0) equals the reference's graph (bs_build_vamana with exact != 0,
  * bs_host.h).  vecs: host n*dim f32.  degree 1..128, beam_width 1..1024, alpha >= 1.
- * Synchronous; allocates its work buffers (the visited bitmaps of up to 2 GiB, lists,
- * visit lists and sort space).  Fails with BS_EINVAL if a search expands more than
+ * Synchronous; allocates its work buffers (the rows padded to 16 floats, visited bitmaps of up
+ * to 2 GiB, lists, visit lists and sort space).  Fails with BS_EINVAL if a search expands more than
  * max(1024, 4*beam_width) nodes.  verbose != 0 prints progress to stderr. */
 int bs_build_vamana_device(const float* vecs, uint64_t n, uint32_t dim, uint32_t degree, uint32_t beam_width,
                            float alpha, uint32_t seed, uint32_t* edges_out, int verbose);
@@ -204,7 +203,8 @@ const char* bs_last_error(void);
  * HDF5 files, script/unpack.py:56-81) ---------------------------------------------------
  * The k nearest rows of the index (k <= 128, dim <= 256) to each of nq queries by exact
  * distance: fp64 squared differences summed in dimension order, ties by id -- the order of
- * bs_groundtruth (bs_host.h).  Candidates come from fp32 matrix-core dot products; each
+ * bs_groundtruth (bs_host.h).  Candidates come from matrix-core dot products of the fp32
+ * values split into fp16 planes (their error no larger than an fp32 chain's); each
  * query carries a certificate that no row outside its candidates can be among the k nearest.
  * out: nq*k int32 (-1 where fewer than k rows exist).  uncertified: nq bytes (1 = no
  * certificate: recompute that query, e.g. with bs_groundtruth) or NULL; n_uncertified
