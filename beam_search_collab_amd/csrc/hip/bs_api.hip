@@ -7,7 +7,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <cfloat>
 #include <cstdio>
 #include <cstring>
 #include <exception>
@@ -76,8 +75,10 @@ struct bs_index_s {
     hipEvent_t ws_free = nullptr;
     // expected cost per label for the base-family label order (calibrate_labels), or null
     float* d_lcost = nullptr;
-    // streams of the large copies to the host (download), made by the first of them
+    // streams of the large copies to the host (download), made by the first of them; one copy of
+    // an index uses them at a time
     hipStream_t copy[4] = {nullptr, nullptr, nullptr, nullptr};
+    std::mutex copy_mutex;
     // device staging of bs_search (host buffers): grows to the largest call, reused after
     void* d_stage = nullptr;
     size_t stage_bytes = 0;
@@ -100,6 +101,7 @@ hipError_t download(bs_index ix, void* dst, const void* src, size_t bytes) {
     constexpr int T = 4;
     const hipMemcpyKind kind = hipMemcpyDeviceToHost;
     if (bytes < (16u << 20)) return hipMemcpy(dst, src, bytes, kind);
+    const std::lock_guard<std::mutex> lock(ix->copy_mutex);  // callers on several threads
     for (hipStream_t& s : ix->copy)
         if (!s && hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) {
             s = nullptr;

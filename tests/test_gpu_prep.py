@@ -214,3 +214,23 @@ def test_device_codebook_infinite_rows(gpu):
     assert np.array_equal(np.isnan(got[2]), np.isnan(want[2]))
     ok = ~np.isnan(want[2])
     assert np.array_equal(got[2][ok], want[2][ok])
+
+
+def test_codebook_from_two_threads(gpu):
+    """two threads ask one index for its codebook (20 MB of codes: the copies to the host go by
+    several streams, made by whichever comes first): each gets the result of a single call"""
+    from concurrent.futures import ThreadPoolExecutor
+    n, dim, degree = 40_000, 100, 32
+    base = host.gen_mixture(n, dim, 8, 0.0, 128.0, 12.0, 0.0, 3, 4)
+    edges = np.random.default_rng(5).integers(0, n, (n, degree), dtype=np.uint32)
+    g = search.GPUGraph(base, edges)
+    try:
+        with ThreadPoolExecutor(2) as ex:
+            got = list(ex.map(lambda _: g.build_rabitq(11), range(2)))
+        want = g.build_rabitq(11)
+        for r in got:
+            assert r[0] == want[0]
+            for x, y in zip(r[1:], want[1:]):
+                assert x.tobytes() == y.tobytes()
+    finally:
+        g.close()
