@@ -689,7 +689,14 @@ __global__ void __launch_bounds__(64 * NW) gt_refine(const float* vecs, uint32_t
                 acc = __dadd_rn(acc, __dmul_rn(diff, diff));
             }
         }
-        if (lane < 32) dist[32 * wave + lane] = ids[32 * wave + lane] == 0xFFFFFFFFu ? __builtin_inf() : acc;
+        if (lane < 32) {
+            // no neighbour: an empty slot, or a row whose distance is a NaN (the select keeps every
+            // row with a NaN value, which may stand for an infinity); a NaN has no rank
+            const uint32_t c = 32 * wave + lane;
+            const bool none = ids[c] == 0xFFFFFFFFu || acc != acc;
+            dist[c] = none ? __builtin_inf() : acc;
+            if (none) ids[c] = 0xFFFFFFFFu;
+        }
     }
     __syncthreads();
     // rank of each candidate in (distance, id) order: thread t counts candidate t % C against
@@ -718,10 +725,10 @@ __global__ void __launch_bounds__(64 * NW) gt_refine(const float* vecs, uint32_t
     // certificate
     bool ok = true;
     if (kc != EMPTY_KEY && k <= C) {
-        double dk = 0.0;
+        double dk = __builtin_inf();
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
-            const uint64_t m = ballot(rank[r] == k - 1);
+            const uint64_t m = ballot(id[r] != 0xFFFFFFFFu && rank[r] == k - 1);
             if (m) dk = __longlong_as_double(static_cast<long long>(
                            readlane64(static_cast<uint64_t>(__double_as_longlong(dd[r])), __builtin_ctzll(m))));
         }

@@ -142,3 +142,27 @@ def test_groundtruth_in_chunks(gpu):
     raw = g.groundtruth(q, 100, exact_fallback=False)
     assert (raw != -2).all()
     assert np.array_equal(raw, host.groundtruth(base, q, 100))
+
+
+@pytest.mark.parametrize("n", [100, 128, 3000])
+def test_groundtruth_nan_rows(gpu, n):
+    """a row with a NaN is nobody's neighbour: the others keep their places, with -1 past the last
+    of them, and a query with a NaN has no neighbours"""
+    base = host.gen_normalized(n, 24, 51)
+    base[0, 3] = np.nan
+    base[57] = np.nan
+    q = host.gen_normalized(40, 24, 52)
+    q[2, 5] = np.nan
+    rows = np.setdiff1d(np.arange(n), [0, 57])
+    g = search.GPUGraph(base, np.zeros((n, 1), np.uint32))
+    good = np.arange(40) != 2
+    for k in (1, 10, 100):
+        raw = g.groundtruth(q, k, exact_fallback=False)
+        want = host.groundtruth(np.ascontiguousarray(base[rows]), q, k)
+        want = np.where(want < 0, -1, rows[np.maximum(want, 0)])
+        cert = (raw != -2).all(1) & good
+        if n < 128:  # fewer rows than candidates: exact without a certificate
+            assert cert[good].all() and (raw[2] == -1).all()
+        elif n > 128:  # (at 128 the last candidate is a row with a NaN: no certificate)
+            assert cert[good].mean() >= 0.95
+        assert np.array_equal(raw[cert], want[cert])
