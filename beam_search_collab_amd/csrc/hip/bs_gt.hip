@@ -3,10 +3,10 @@
 // from HDF5 files, script/unpack.py:56-81); this is the one dense contraction near the
 // search path, so it runs on the matrix cores.
 //
-//   gt_split    every row scaled by a power of two and split into two fp16 planes (h + l = the
-//               fp32 value to 2^-24 of it) in the matrix cores' operand layout, and |b_j|^2
-//               (fp64 sum, rounded once)
-//   gt_select   32 x 32 tiles of a_j = |b_j|^2 - 2 q.b_j from v_mfma_f32_32x32x16_f16, three
+//   gt_split    every row scaled by a power of two and split into three fp16 planes (h + m + l =
+//               the fp32 value) in the matrix cores' operand layout, and |b_j|^2 (fp64 sum,
+//               rounded once)
+//   gt_select   32 x 32 tiles of a_j = |b_j|^2 - 2 q.b_j from v_mfma_f32_32x32x16_f16, six
 //               products of the planes; the 128 smallest (a_j, j) per (query, row split) kept
 //               in HBM with a per-query threshold in registers and an LDS append buffer
 //   gt_refine   merge the splits' lists, exact fp64 distances of the 128 candidates summed
@@ -23,6 +23,8 @@
 #include <algorithm>
 #include <cstring>
 #include <string>
+#include <type_traits>
+#include <vector>
 
 int bs_internal_vecs(bs_index idx, const float** vecs, uint32_t* dstride);
 void bs_internal_set_error(const std::string& msg);
@@ -68,11 +70,19 @@ __device__ __forceinline__ float query_scale(float largest, float sc) {
     return largest == 0.0f || largest == __builtin_inff() ? sc : fminf(sc, row_scale(largest));
 }
 
-// x (already scaled) as NP fp16 planes: each keeps the next 11 significant bits, rounded to
-// nearest, so two planes hold x to 2^-24 |x| and three hold it exactly.  What falls below
-// fp16's range is less than 2^-29 of the row's largest value.  A value that is infinite or NaN
-// leaves a NaN, which makes every product with it a survivor.
-template <int NP>
+constexpr int NP = 3;  // fp16 planes of a value: h, m, l
+
+// steps of 16 dimensions that a base tile's m and l planes are loaded ahead (a divisor of KC): as
+// many as the registers hold beside the queries' planes.  10k queries, 200k x 256: 4 steps 8.9 ms,
+// 8 (10 registers spilled) 9.4, 16 26.7; 5k, 200k x 200: 4 steps 4.7, 6 5.0; 10k, 500k x 128: 2
+// steps 10.0, 4 9.5, 8 (6 spilled) 13.1; 200k x 96: 3 and 6 steps 4.3
+constexpr int ahead(int KC) { return KC == 6 ? 3 : KC >= 8 ? 4 : KC; }
+
+// x (already scaled) as fp16 planes: each keeps the next 11 significant bits, rounded to nearest.
+// h leaves at most 2^-11 |x|, m at most the last of the 24 bits, 2^-23 |x|, and l holds that one.
+// What falls below fp16's range is less than 2^-27 of the row's largest value (if the matrix unit
+// takes fp16 subnormals as zero; else 2^-39).  A value that is infinite or NaN leaves a NaN, which
+// makes every product with it a survivor.
 __device__ __forceinline__ void split_value(float x, _Float16 (&p)[NP]) {
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
@@ -81,23 +91,18 @@ __device__ __forceinline__ void split_value(float x, _Float16 (&p)[NP]) {
     }
 }
 
-// Two planes; three up to 32 dimensions, where an fp32 chain rounds so few times that the
-// planes' 2^-24 would be the larger error (the matrix time is the smaller part there).
-constexpr int planes(int KC) { return KC <= 2 ? 3 : 2; }
-
 // Operand layout of v_mfma_f32_32x32x16_f16 (A and B alike): lane l holds row (column) l % 32
 // and 8 of the 16 dimensions, 8 (l / 32) .. + 7.  Both operands are filled by the same rule, so
 // the order of the dimensions inside the instruction does not matter.  A fragment is one
 // operand register set of the wavefront, 64 x 16 bytes; the base's fragments are stored
 // [tile of 32 rows][16 dimensions][plane], so a wavefront's load of one is 1 KB contiguous.
 //
-// Rows row0 .. row0 + m of the base, a wavefront per tile.  Memory bound (4 bytes read and 4
+// Rows row0 .. row0 + m of the base, a wavefront per tile.  Memory bound (4 bytes read and 6
 // written per value).  The norm is summed in fp64 (one rounding).  meta[j] = (|b_j|^2, -2 over
 // the row's scale).
 template <int KC>
 __global__ void __launch_bounds__(256) gt_split(const float* vecs, uint64_t row0, uint64_t m, uint32_t dstride,
                                                 uint4* frag, float2* meta, uint32_t* bmax_bits) {
-    constexpr int NP = planes(KC);
     const uint32_t lane = lane_id(), half = lane >> 5, l32 = lane & 31u;
     const uint64_t tiles = (m + 31) / 32, step = static_cast<uint64_t>(gridDim.x) * 4;
     float mx = 0.0f;
@@ -134,7 +139,7 @@ __global__ void __launch_bounds__(256) gt_split(const float* vecs, uint64_t row0
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 _Float16 v[NP];
-                split_value<NP>(x[kc][i / 4][i % 4] * sc, v);
+                split_value(x[kc][i / 4][i % 4] * sc, v);
 #pragma unroll
                 for (int q = 0; q < NP; ++q) p[q][i] = v[q];
             }
@@ -197,17 +202,67 @@ __device__ __forceinline__ uint64_t sort_descending(uint64_t v) {
     return v;
 }
 
-// A wavefront holds 32 QB queries as A operands (KC steps of 16 dimensions x 2 planes) and
-// streams its split's base tiles as B operands, each operand register reloaded for the next
-// tile as soon as this tile's products have read it.  a.b = (hl + lh) + hh: the small products
-// are summed first and the large ones on top, so the small ones' roundings are 2^-11 of the
-// large ones', and the dropped one (ll) is below 2^-24 |a||b|.  Against fp64
-// the rms error of q.b is 0.37-0.71 of the fp32 instructions' (mixture and unit-sphere data, dims
-// 16..256; at most 0.87 over wide-ranged data), because the chain rounds 8 times less often.
-// Three fp16 products of 16 dimensions take 96 matrix cycles, eight v_mfma_f32_32x32x2f32 512.
-// 500k x 128, 10k queries: 17.1 -> 5.7 ms with the filtering below (the products alone 3.8, at
-// the rate a large bf16 matrix product reaches on the card); from three bf16 planes
-// and six products 12.2 with the filtering of one split at a time.
+// A operands of a wavefront: block b, lane (l32, half): query q0 + 32 b + l32, dimensions
+// 16 kc + 8 half + i; returns 1 / the scale.
+// All the wavefront's queries share one scale, the largest query's: a query 2^k smaller
+// keeps 2^(k - 29) of its own largest value and above in 11-bit planes, and the certificate
+// counts what is lost below (gt_refine).
+template <int KC, int QB>
+__device__ __forceinline__ float load_queries(const float* queries, uint32_t dim, uint64_t nq, uint64_t q0,
+                                              f16x8 (&a)[QB][KC][NP]) {
+    const uint32_t lane = lane_id(), half = lane >> 5, l32 = lane & 31u;
+    float x[QB][KC][8], sc = 0x1p100f;
+#pragma unroll
+    for (int b = 0; b < QB; ++b) {
+        const uint64_t qi = q0 + 32u * b + l32;
+        const float* qv = queries + std::min<uint64_t>(qi, nq - 1) * dim;
+#pragma unroll
+        for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {  // all loads first (clamped), then the zeroing
+                const uint32_t d = 16u * kc + 8u * half + i;
+                x[b][kc][i] = qv[d < dim ? d : 0u];
+            }
+        float big = 0.0f;
+#pragma unroll
+        for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t d = 16u * kc + 8u * half + i;
+                const float v = qi < nq && d < dim ? x[b][kc][i] : 0.0f;
+                x[b][kc][i] = v;
+                big = fabsf(v) > big || v != v ? (v != v ? __builtin_inff() : fabsf(v)) : big;
+            }
+        big = fmaxf(big, bsw::xor_lane_f<32>(big));
+        sc = query_scale(big, sc);
+    }
+    sc = bsw::wave_min(sc);
+#pragma unroll
+    for (int b = 0; b < QB; ++b)
+#pragma unroll
+        for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                _Float16 v[NP];
+                split_value(x[b][kc][i] * sc, v);
+#pragma unroll
+                for (int p = 0; p < NP; ++p) a[b][kc][p][i] = v[p];
+            }
+    return 1.0f / sc;
+}
+
+// A wavefront holds 32 QB queries as A operands (KC steps of 16 dimensions x 3 planes) and
+// streams its split's base tiles as B operands, each operand register reloaded as soon as the
+// products have read it.  a.b = (hl + lh + mm + hm + mh) + hh: the small products are summed first
+// and the large ones on top, so the small ones' roundings are 2^-11 of the large ones', and
+// the dropped ones (ml, lm, ll) are below 2^-32 |a||b|: the fp32 operands with all their bits.
+// Against fp64 the rms error of q.b is 0.36-0.56 of the fp32 instructions' over mixture and
+// unit-sphere data of 16..256 dimensions and 0.12-0.79 over wide-ranged data of 32 and more and
+// values that differ in their last 12 bits, because the chain rounds 8 times less often; where one or
+// two products are most of the sum and both round once, 1.0-1.27 (the matrix unit's rounding).  Two planes and three products
+// hold 22 to 24 of the 24 bits: 1.9-2.9 there and up to 1.27 on wide-ranged data.
+// Six fp16 products of 16 dimensions take 192 matrix cycles, eight v_mfma_f32_32x32x2f32 512.
+// 500k x 128, 10k queries: 17.1 -> 8.3 ms with the filtering below.
 // Two query blocks per wavefront (dim <= 128) halve the base bytes per product.
 //
 // The matrix pipe and the vector unit work at the same time: while tile t's products run, tile
@@ -231,7 +286,6 @@ gt_select(const uint4* frag, const float2* meta, uint64_t row0, uint64_t m, cons
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const uint32_t lane = lane_id(), wave = bsw::uniform(threadIdx.x >> 6), half = lane >> 5, l32 = lane & 31u;
     constexpr uint32_t NQ = 32 * QB;
-    constexpr int NP = planes(KC);
     const uint64_t w = static_cast<uint64_t>(blockIdx.x) * 4 + wave;
     const uint64_t nqb = (nq + NQ - 1) / NQ;
     if (w >= nqb * nsplit) return;
@@ -248,52 +302,8 @@ gt_select(const uint4* frag, const float2* meta, uint64_t row0, uint64_t m, cons
     float* vals = reinterpret_cast<float*>(my + NQ * BUF * 8);
     uint32_t* cnt = reinterpret_cast<uint32_t*>(my + NQ * BUF * 8 + 32 * TS * 4);  // keys in each query's buffer
 
-    // A operands: block b, lane (l32, half): query qb * NQ + 32 b + l32, dimensions 16 kc + 8 half + i
-    // All the wavefront's queries share one scale, the largest query's: a query 2^k smaller
-    // keeps 2^(k - 29) of its own largest value and above in 11-bit planes, and the certificate
-    // counts what is lost below (gt_refine).
     f16x8 a[QB][KC][NP];
-    float qinv;  // 1 / the scale
-    {
-        float x[QB][KC][8], sc = 0x1p100f;
-#pragma unroll
-        for (int b = 0; b < QB; ++b) {
-            const uint64_t qi = qb * NQ + 32u * b + l32;
-            const float* qv = queries + std::min<uint64_t>(qi, nq - 1) * dim;
-#pragma unroll
-            for (int kc = 0; kc < KC; ++kc)
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {  // all loads first (clamped), then the zeroing
-                    const uint32_t d = 16u * kc + 8u * half + i;
-                    x[b][kc][i] = qv[d < dim ? d : 0u];
-                }
-            float big = 0.0f;
-#pragma unroll
-            for (int kc = 0; kc < KC; ++kc)
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const uint32_t d = 16u * kc + 8u * half + i;
-                    const float v = qi < nq && d < dim ? x[b][kc][i] : 0.0f;
-                    x[b][kc][i] = v;
-                    big = fabsf(v) > big || v != v ? (v != v ? __builtin_inff() : fabsf(v)) : big;
-                }
-            big = fmaxf(big, bsw::xor_lane_f<32>(big));
-            sc = query_scale(big, sc);
-        }
-        sc = bsw::wave_min(sc);
-        qinv = 1.0f / sc;
-#pragma unroll
-        for (int b = 0; b < QB; ++b)
-#pragma unroll
-            for (int kc = 0; kc < KC; ++kc)
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    _Float16 v[NP];
-                    split_value<NP>(x[b][kc][i] * sc, v);
-#pragma unroll
-                    for (int p = 0; p < NP; ++p) a[b][kc][p][i] = v[p];
-                }
-    }
+    const float qinv = load_queries<KC, QB>(queries, dim, nq, qb * NQ, a);
     if (s == 0 && lane == 0) qscale[qb] = qinv;
     // tau: per accumulator register, the threshold of its query (a float compare passes a
     // superset of the list's key order; none passes for a query past nq).  Lane i's tq is query
@@ -427,9 +437,11 @@ gt_select(const uint4* frag, const float2* meta, uint64_t row0, uint64_t m, cons
         return ballot(full) != 0;
     };
 
-    f16x8 bp[KC][NP];
-    auto load_plane = [&](uint32_t tile, int kc, int p) __attribute__((always_inline)) {
-        bp[kc][p] = __builtin_bit_cast(f16x8, frag[((static_cast<uint64_t>(tile) * KC + kc) * NP + p) * 64 + lane]);
+    // B operands: the h planes of the whole next tile, the m and l planes of the next D steps
+    constexpr int D = ahead(KC);
+    f16x8 bh[KC], bml[D][2];
+    auto frag_at = [&](uint32_t tile, int kc, int p) __attribute__((always_inline)) {
+        return __builtin_bit_cast(f16x8, frag[((static_cast<uint64_t>(tile) * KC + kc) * NP + p) * 64 + lane]);
     };
     if (lane < NQ) cnt[lane] = 0u;
     wave_sync();
@@ -437,9 +449,9 @@ gt_select(const uint4* frag, const float2* meta, uint64_t row0, uint64_t m, cons
     // Tile t's products into accN (the next tile's operands requested as these are read), with
     // the previous tile's values av formed from accO on the way; returns the lane's survivors
     float av[QB][16];
-    auto step = [&](uint32_t next, f32x16 (&accN)[QB], const f32x16 (&accO)[QB], float2 mo) __attribute__((always_inline)) {
+    auto step = [&](uint32_t tile, uint32_t next, f32x16 (&accN)[QB], const f32x16 (&accO)[QB], float2 mo) __attribute__((always_inline)) {
         uint32_t bits = 0;
-        constexpr int SMALL = (NP == 3 ? 5 : 2) * QB, ALL = KC * (SMALL + QB);  // matrix instructions
+        constexpr int SMALL = 5 * QB, ALL = KC * (SMALL + QB);  // matrix instructions
         // the values screened beside instructions [m0, m1) of the tile's ALL
         auto screen = [&](int m0, int m1) __attribute__((always_inline)) {
 #pragma unroll
@@ -451,25 +463,25 @@ gt_select(const uint4* frag, const float2* meta, uint64_t row0, uint64_t m, cons
                 bits |= !(av[b][r] > tau[b][r]) ? 1u << e : 0u;  // a NaN survives
             }
         };
-#define BSG_MFMA(kc, pa, pb, from)                                                                   \
+#define BSG_MFMA(kc, pa, y, from)                                                                    \
     _Pragma("unroll") for (int b = 0; b < QB; ++b) accN[b] =                                          \
-        __builtin_amdgcn_mfma_f32_32x32x16_f16(a[b][kc][pa], bp[kc][pb], from, 0, 0, 0);
+        __builtin_amdgcn_mfma_f32_32x32x16_f16(a[b][kc][pa], y, from, 0, 0, 0);
         const f32x16 zero = {};
 #pragma unroll
         for (int kc = 0; kc < KC; ++kc) {
+            const f16x8 m = bml[kc % D][0], l = bml[kc % D][1];
             if (kc == 0) {
-                BSG_MFMA(kc, 0, NP - 1, zero)
+                BSG_MFMA(kc, 0, l, zero)
             } else {
-                BSG_MFMA(kc, 0, NP - 1, accN[b])
+                BSG_MFMA(kc, 0, l, accN[b])
             }
-            BSG_MFMA(kc, NP - 1, 0, accN[b])
-            if constexpr (NP == 3) {
-                BSG_MFMA(kc, 1, 1, accN[b])
-                BSG_MFMA(kc, 0, 1, accN[b])
-                BSG_MFMA(kc, 1, 0, accN[b])
-                load_plane(next, kc, 1);
-            }
-            load_plane(next, kc, NP - 1);
+            BSG_MFMA(kc, 2, bh[kc], accN[b])
+            BSG_MFMA(kc, 1, m, accN[b])
+            BSG_MFMA(kc, 0, m, accN[b])
+            BSG_MFMA(kc, 1, bh[kc], accN[b])
+            const bool wraps = kc + D >= KC;
+            bml[kc % D][0] = frag_at(wraps ? next : tile, (kc + D) % KC, 1);
+            bml[kc % D][1] = frag_at(wraps ? next : tile, (kc + D) % KC, 2);
             screen(kc * SMALL, (kc + 1) * SMALL);
             // keep the reloads and the screening among the products: a matrix instruction, then
             // vector ones in its shadow
@@ -482,8 +494,8 @@ gt_select(const uint4* frag, const float2* meta, uint64_t row0, uint64_t m, cons
         }
 #pragma unroll
         for (int kc = 0; kc < KC; ++kc) {
-            BSG_MFMA(kc, 0, 0, accN[b])
-            load_plane(next, kc, 0);
+            BSG_MFMA(kc, 0, bh[kc], accN[b])
+            bh[kc] = frag_at(next, kc, 0);
             screen(KC * SMALL + kc * QB, KC * SMALL + (kc + 1) * QB);
 #pragma unroll
             for (int i = 0; i < QB; ++i) {
@@ -550,9 +562,13 @@ gt_select(const uint4* frag, const float2* meta, uint64_t row0, uint64_t m, cons
     };
     if (t0 < t1) {
 #pragma unroll
-        for (int kc = 0; kc < KC; ++kc)
-#pragma unroll
-            for (int p = 0; p < NP; ++p) load_plane(t0, kc, p);
+        for (int kc = 0; kc < KC; ++kc) {
+            bh[kc] = frag_at(t0, kc, 0);
+            if (kc < D) {
+                bml[kc][0] = frag_at(t0, kc, 1);
+                bml[kc][1] = frag_at(t0, kc, 2);
+            }
+        }
         refresh();
         spread_tau();
         if (prime) {
@@ -583,14 +599,14 @@ gt_select(const uint4* frag, const float2* meta, uint64_t row0, uint64_t m, cons
 #pragma unroll
         for (int b = 0; b < QB; ++b) acc0[b] = acc1[b] = f32x16{};
         float2 m0 = meta[t0 * 32u + l32], m1;
-        step(tile_of(1), acc0, acc1, m0);
+        step(t0, tile_of(1), acc0, acc1, m0);
         for (uint32_t u = 1;; u += 2) {
             m1 = meta[tile_of(u) * 32u + l32];
-            uint32_t bits = step(tile_of(u + 1), acc1, acc0, m0);
+            uint32_t bits = step(tile_of(u), tile_of(u + 1), acc1, acc0, m0);
             done(bits, u - 1);
             if (u >= total) break;
             m0 = meta[tile_of(u + 1) * 32u + l32];
-            bits = step(tile_of(u + 2), acc0, acc1, m1);
+            bits = step(tile_of(u + 1), tile_of(u + 2), acc0, acc1, m1);
             done(bits, u);
             if (u + 1 >= total) break;
             if (u % REFRESH == 1 && u > prime) {  // u is odd
@@ -737,24 +753,70 @@ __global__ void __launch_bounds__(64 * NW) gt_refine(const float* vecs, uint32_t
         const double ac = static_cast<double>(bsd::key_dist(kc));
         const double bm = __builtin_sqrt(static_cast<double>(__uint_as_float(*bmax_bits)));
         const double qb = __builtin_sqrt(qn2) + bm;
-        // q.b's error: the planes' 2^-24 of each factor and the dropped product, 3 2^-24 |q||b|;
-        // dim accumulations of exact products, dim 2^-24 |q||b| (twice that if the matrix unit
-        // truncates); what lies below fp16's range in the row, 2^-28 sqrt(dim) |q||b|.  (|q| +
-        // |b|)^2 >= 4 |q||b|, so 2 (dim + 3) 2^-24 (|q| + |b|)^2 covers twice their sum and the
-        // norms' roundings.  What lies below fp16's range in the query (2^-14 over the scale it
-        // shares with its neighbours, if the matrix unit flushes it) is 2^-14 qscale sqrt(dim)
-        // |b| at most.  A row whose largest value is below 2^-86 has the largest scale, 2^100: it
-        // loses 2^-114 per value.  2^-140: results below fp32's normal range.
+        // q.b's error, in 2^-24 |q||b|: dim roundings of the sum of the large products (dim; twice
+        // that if the matrix unit truncates), 5 dim roundings of partial sums of the small ones,
+        // each 2^-9 of it at most (0.02 dim), the dropped products (below 0.01), what lies below
+        // fp16's range in the row (2^-27 sqrt(dim): below sqrt(dim) / 8).  a_j doubles it; |b_j|^2
+        // and a_j are rounded once each.  (|q| + |b|)^2 >= 4 |q||b|, so 2 (dim + 3) 2^-24 (|q| +
+        // |b|)^2 grants 8 dim + 24 of 4.1 dim + sqrt(dim) / 4 + 2, and 6 |b|^2 of 2.  What lies
+        // below fp16's range in the query (2^-13 over the scale it shares with its neighbours) is
+        // 2^-13 qscale sqrt(dim) |b| at most.  A row whose largest value is below 2^-86 has the
+        // largest scale, 2^100: it loses 2^-113 per value.  2^-140: results below fp32's normal
+        // range.
         const double sd = __builtin_sqrt(static_cast<double>(dim));
         const double eps = 2.0 * (dim + 3) * 0x1p-24 * qb * qb +
-                           2.0 * 0x1p-14 * static_cast<double>(qscale[qi / NQ]) * sd * bm +
-                           2.0 * 0x1p-114 * sd * __builtin_sqrt(qn2) + 0x1p-140;
+                           2.0 * 0x1p-13 * static_cast<double>(qscale[qi / NQ]) * sd * bm +
+                           2.0 * 0x1p-113 * sd * __builtin_sqrt(qn2) + 0x1p-140;
         ok = dk < ac + qn2 - eps;
     }
     if (lane == 0) {
         if (unc) unc[qi] = ok ? 0 : 1;
         if (!ok) atomicAdd(n_unc, 1ull);
     }
+}
+
+// The dot products as gt_select forms them: 32 queries against every row (out: 32 x 32 tiles),
+// a wavefront per tile.  For the check of their rounding.
+template <int KC>
+__global__ void __launch_bounds__(64) dbg_products(const uint4* frag, const float2* meta, const float* queries,
+                                                   uint32_t dim, float* out) {
+    const uint32_t lane = lane_id(), half = lane >> 5, l32 = lane & 31u, t = blockIdx.x;
+    f16x8 a[1][KC][NP];
+    const float qinv = load_queries<KC, 1>(queries, dim, 32, 0, a);
+    auto b = [&](int kc, int p) __attribute__((always_inline)) {
+        return __builtin_bit_cast(f16x8, frag[((static_cast<uint64_t>(t) * KC + kc) * NP + p) * 64 + lane]);
+    };
+    f32x16 acc = {};
+    auto mul = [&](int kc, int pa, int pb) __attribute__((always_inline)) {
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0][kc][pa], b(kc, pb), acc, 0, 0, 0);
+    };
+    for (int kc = 0; kc < KC; ++kc) {
+        mul(kc, 0, 2);
+        mul(kc, 2, 0);
+        mul(kc, 1, 1);
+        mul(kc, 0, 1);
+        mul(kc, 1, 0);
+    }
+    for (int kc = 0; kc < KC; ++kc) mul(kc, 0, 0);
+    const float binv = -0.5f * meta[t * 32u + l32].y;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) out[(static_cast<uint64_t>(acc_row(r, half)) * gridDim.x + t) * 32 + l32] = acc[r] * binv * qinv;
+}
+
+// the same products from the fp32 instruction (lane half h: dimensions KC 8 h ..), one chain
+template <int KC>
+__global__ void __launch_bounds__(64) dbg_products_f32(const float* vecs, uint32_t dstride, const float* queries,
+                                                       uint32_t dim, float* out) {
+    const uint32_t lane = lane_id(), half = lane >> 5, l32 = lane & 31u, t = blockIdx.x;
+    f32x16 acc = {};
+    for (uint32_t i = 0; i < KC * 8; ++i) {
+        const uint32_t d = half * KC * 8 + i;
+        const float x = d < dim ? queries[l32 * dim + d] : 0.0f;
+        const float y = d < dim ? vecs[(static_cast<uint64_t>(t) * 32 + l32) * dstride + d] : 0.0f;
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) out[(static_cast<uint64_t>(acc_row(r, half)) * gridDim.x + t) * 32 + l32] = acc[r];
 }
 
 // v_mfma_f32_32x32x2f32 layout check: A 32x2, B 2x32 given row-major; D 32x32 row-major
@@ -791,6 +853,22 @@ hipError_t launch_select(dim3 g, hipStream_t s, const uint4* frag, const float2*
     hipLaunchKernelGGL(k, g, dim3(256), lds, s, frag, meta, row0, m, q, dim, nq, nsplit, split_tiles,
                        row0 == 0 ? 1u : 0u, topc, tshare, pub, qscale);
     return hipGetLastError();
+}
+
+// steps of 16 dimensions of the instance that takes rows of dim, and f(steps, query blocks) for it
+uint32_t steps_of(uint32_t dim) { return dim <= 32 ? 2 : dim <= 64 ? 4 : dim <= 96 ? 6 : dim <= 128 ? 8 : dim <= 192 ? 12 : 16; }
+template <typename F>
+hipError_t with_steps(uint32_t KC, F&& f) {
+    std::integral_constant<int, 1> q1;
+    std::integral_constant<int, 2> q2;
+    switch (KC) {
+    case 2: return f(std::integral_constant<int, 2>{}, q2);
+    case 4: return f(std::integral_constant<int, 4>{}, q2);
+    case 6: return f(std::integral_constant<int, 6>{}, q2);
+    case 8: return f(std::integral_constant<int, 8>{}, q2);
+    case 12: return f(std::integral_constant<int, 12>{}, q1);
+    default: return f(std::integral_constant<int, 16>{}, q1);
+    }
 }
 
 // Row splits per query block: nqb * nsplit wavefronts run 4 per CU (a SIMD holds one), so the
@@ -835,11 +913,11 @@ extern "C" int bs_index_groundtruth_device(bs_index idx, const float* d_queries,
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
         cus = 256;
     // 16-dimension steps, and 64 queries per wavefront while their operands fit beside a tile's
-    const uint32_t KC = dim <= 32 ? 2 : dim <= 64 ? 4 : dim <= 96 ? 6 : dim <= 128 ? 8 : dim <= 192 ? 12 : 16;
+    const uint32_t KC = steps_of(dim);
     const uint32_t NQ = KC <= 8 ? 64 : 32;
     const uint64_t nqb = (nq + NQ - 1) / NQ;
     // the fp16 planes are made for at most 1 GiB of rows at a time; the lists carry over
-    const uint64_t tile_bytes = static_cast<uint64_t>(KC) * static_cast<uint64_t>(bsg::planes(static_cast<int>(KC))) * 1024;
+    const uint64_t tile_bytes = static_cast<uint64_t>(KC) * bsg::NP * 1024;
     const uint64_t tiles = (n + 31) / 32, chunk = std::min<uint64_t>(tiles, (1ull << 30) / tile_bytes);
     const uint64_t nsplit = pick_splits(nqb, chunk, 4ull * static_cast<uint64_t>(cus));
     const uint64_t split_tiles = (chunk + nsplit - 1) / nsplit;
@@ -876,16 +954,7 @@ extern "C" int bs_index_groundtruth_device(bs_index idx, const float* d_queries,
                                                          static_cast<uint32_t>(nsplit),
                                                          static_cast<uint32_t>(split_tiles), topc, tshare, pub, qscale);
         };
-        std::integral_constant<int, 1> q1;
-        std::integral_constant<int, 2> q2;
-        switch (KC) {
-        case 2: e = go(std::integral_constant<int, 2>{}, q2); break;
-        case 4: e = go(std::integral_constant<int, 4>{}, q2); break;
-        case 6: e = go(std::integral_constant<int, 6>{}, q2); break;
-        case 8: e = go(std::integral_constant<int, 8>{}, q2); break;
-        case 12: e = go(std::integral_constant<int, 12>{}, q1); break;
-        default: e = go(std::integral_constant<int, 16>{}, q1); break;
-        }
+        e = with_steps(KC, go);
     }
     if (e == hipSuccess) {
         // a wavefront merges a list in ~0.3 us: with many splits (few queries) 16 share them
@@ -945,6 +1014,50 @@ extern "C" int bs_index_groundtruth(bs_index idx, const float* queries, uint64_t
     }
     release();
     return rc;
+} catch (...) {
+    return bs_internal_exception();
+}
+
+extern "C" int bs_debug_gt_products(const float* rows, uint32_t n, const float* queries, uint32_t dim, int fp32,
+                                    float* out) try {
+    if (!rows || !queries || !out) return gfail(BS_EINVAL, "null argument");
+    if (n == 0 || n % 32 != 0 || n > (1u << 20)) return gfail(BS_EINVAL, "n must be a multiple of 32 up to 2^20");
+    if (dim == 0 || dim > 256) return gfail(BS_EINVAL, "dim must be in 1..256");
+    const uint32_t dstride = (dim + 3) & ~3u, KC = steps_of(dim);
+    std::vector<float> padded(static_cast<size_t>(n) * dstride, 0.0f);
+    for (uint32_t j = 0; j < n; ++j)
+        std::memcpy(&padded[static_cast<size_t>(j) * dstride], rows + static_cast<size_t>(j) * dim, dim * sizeof(float));
+    const size_t b_rows = padded.size() * 4, b_q = 32ull * dim * 4, b_out = 32ull * n * 4, b_meta = n * 8ull,
+                 b_frag = static_cast<size_t>(n / 32) * KC * bsg::NP * 1024;
+    char* ws = nullptr;
+    auto al = [](size_t v) { return (v + 255) & ~static_cast<size_t>(255); };
+    if (hipMalloc(reinterpret_cast<void**>(&ws), al(b_rows) + al(b_q) + al(b_out) + al(b_meta) + al(b_frag) + 4) != hipSuccess)
+        return gfail(BS_ENOMEM, "hipMalloc failed");
+    float* dr = reinterpret_cast<float*>(ws);
+    float* dq = reinterpret_cast<float*>(ws + al(b_rows));
+    float* dout = reinterpret_cast<float*>(ws + al(b_rows) + al(b_q));
+    float2* meta = reinterpret_cast<float2*>(ws + al(b_rows) + al(b_q) + al(b_out));
+    uint4* frag = reinterpret_cast<uint4*>(ws + al(b_rows) + al(b_q) + al(b_out) + al(b_meta));
+    uint32_t* bmax = reinterpret_cast<uint32_t*>(ws + al(b_rows) + al(b_q) + al(b_out) + al(b_meta) + al(b_frag));
+    hipError_t e = hipMemcpy(dr, padded.data(), b_rows, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(dq, queries, b_q, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemset(bmax, 0, 4);
+    if (e == hipSuccess)
+        e = with_steps(KC, [&](auto kc, auto) {
+            constexpr int K = decltype(kc)::value;
+            if (fp32) {
+                hipLaunchKernelGGL(bsg::dbg_products_f32<K>, dim3(n / 32), dim3(64), 0, nullptr, dr, dstride, dq, dim, dout);
+            } else {
+                hipLaunchKernelGGL(bsg::gt_split<K>, dim3((n / 32 + 3) / 4), dim3(256), 0, nullptr, dr, uint64_t{0}, uint64_t{n},
+                                   dstride, frag, meta, bmax);
+                hipLaunchKernelGGL(bsg::dbg_products<K>, dim3(n / 32), dim3(64), 0, nullptr, frag, meta, dq, dim, dout);
+            }
+            return hipGetLastError();
+        });
+    if (e == hipSuccess) e = hipMemcpy(out, dout, b_out, hipMemcpyDeviceToHost);
+    (void)hipFree(ws);
+    if (e != hipSuccess) return gfail(BS_EHIP, std::string("products check: ") + hipGetErrorString(e));
+    return BS_OK;
 } catch (...) {
     return bs_internal_exception();
 }

@@ -324,6 +324,16 @@ def debug_mfma32(A, B):
     return D
 
 
+def debug_gt_products(rows, queries, fp32=False):
+    """q.b of 32 queries and n rows as the ground-truth candidates are selected by (bs_debug_gt_products)"""
+    rows = np.ascontiguousarray(rows, dtype=np.float32)
+    queries = np.ascontiguousarray(queries, dtype=np.float32).reshape(32, rows.shape[1])
+    out = np.empty((32, rows.shape[0]), dtype=np.float32)
+    _check(_lib.hip().bs_debug_gt_products(_ptr(rows), rows.shape[0], _ptr(queries), rows.shape[1], int(fp32), _ptr(out)),
+           "bs_debug_gt_products")
+    return out
+
+
 def debug_filter(bloom, capacity, keys, qkeys):
     keys = np.ascontiguousarray(keys, dtype=np.uint32)
     qkeys = np.ascontiguousarray(qkeys, dtype=np.uint32)

@@ -204,8 +204,9 @@ const char* bs_last_error(void);
  * The k nearest rows of the index (k <= 128, dim <= 256) to each of nq queries by exact
  * distance: fp64 squared differences summed in dimension order, ties by id -- the order of
  * bs_groundtruth (bs_host.h).  Candidates come from matrix-core dot products of the fp32
- * values split into fp16 planes (their error no larger than an fp32 chain's); each
- * query carries a certificate that no row outside its candidates can be among the k nearest.
+ * values, split into three fp16 planes that hold all their bits (rms error 0.36-0.56 of an fp32
+ * chain's over clustered and normalised vectors; bs_debug_gt_products); each query carries a
+ * certificate that no row outside its candidates can be among the k nearest.
  * out: nq*k int32 (-1 where fewer than k rows exist).  uncertified: nq bytes (1 = no
  * certificate: recompute that query, e.g. with bs_groundtruth) or NULL; n_uncertified
  * (nullable) gets their number.  Synchronous; allocates device work buffers. */
@@ -267,6 +268,11 @@ int bs_debug_cost_order(const float* signal, uint64_t n, uint32_t* qmap, uint32_
  * reference (its launches run query i in block i). */
 int bs_debug_label_order(const uint32_t* labels, const float* lcost, uint64_t n, uint32_t g, uint32_t X,
                          uint32_t* qmap);
+
+/* The dot products q.b that select ground-truth candidates, 32 queries against n rows (a
+ * multiple of 32, at most 2^20; dim 1..256): out 32 x n, as the matrix cores give them.  fp32 != 0:
+ * one chain of v_mfma_f32_32x32x2f32 instead, to compare the rounding with. */
+int bs_debug_gt_products(const float* rows, uint32_t n, const float* queries, uint32_t dim, int fp32, float* out);
 
 /* One v_mfma_f32_32x32x2f32 product: A 32x2 and B 2x32 row-major in, D = A B 32x32
  * row-major out, read back through the accumulator layout the ground-truth kernel uses. */

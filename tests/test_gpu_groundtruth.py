@@ -166,3 +166,38 @@ def test_groundtruth_nan_rows(gpu, n):
         elif n > 128:  # (at 128 the last candidate is a row with a NaN: no certificate)
             assert cert[good].mean() >= 0.95
         assert np.array_equal(raw[cert], want[cert])
+
+
+def _product_data(kind, n, dim, rng):
+    if kind == "sphere":
+        x = rng.standard_normal((n, dim))
+        return x / np.linalg.norm(x, axis=1, keepdims=True)
+    if kind == "mixture":
+        c = np.random.default_rng(8).random((16, dim)) * 128
+        return np.maximum(c[rng.integers(0, 16, n)] + 12 * rng.standard_normal((n, dim)), 0)
+    if kind == "wide":  # magnitudes over 24 binades in one row
+        return rng.standard_normal((n, dim)) * 2.0 ** rng.integers(-12, 12, (n, dim))
+    if kind == "near_one":  # only the low half of the significand differs
+        return 1 + rng.integers(0, 4096, (n, dim)) * 2.0 ** -23
+    return rng.standard_normal((n, dim))
+
+
+@pytest.mark.parametrize("dim", [16, 33, 34, 64, 97, 128, 200, 256])
+def test_groundtruth_products_precision(gpu, dim):
+    """the dot products that select the candidates lose nothing against an fp32 chain: their rms
+    error against fp64 is no larger, and a single product is rounded once (at most 2^-23 of it).
+    Wide-ranged rows count from 33 dimensions: of 16 such products one is most of the sum, so both
+    round about once, as the single product does"""
+    rng = np.random.default_rng(dim)
+    for kind in ("gauss", "mixture", "sphere", "near_one") + (("wide",) if dim > 16 else ()):
+        b = _product_data(kind, 2048, dim, rng).astype(np.float32)
+        q = _product_data(kind, 32, dim, rng).astype(np.float32)
+        exact = q.astype(np.float64) @ b.astype(np.float64).T
+        planes = search.debug_gt_products(b, q) - exact
+        chain = search.debug_gt_products(b, q, fp32=True) - exact
+        assert np.sqrt((planes ** 2).mean()) <= np.sqrt((chain ** 2).mean()), kind
+    b = np.zeros((2048, dim), np.float32)
+    b[:, dim - 1] = 1 + rng.random(2048)
+    q = (1 + rng.random((32, dim))).astype(np.float32)
+    exact = q.astype(np.float64) @ b.astype(np.float64).T
+    assert (np.abs(search.debug_gt_products(b, q) - exact) <= 2.0 ** -23 * np.abs(exact)).all()
