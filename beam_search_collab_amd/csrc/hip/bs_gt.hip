@@ -55,20 +55,14 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
-// The power of two that brings a row's largest magnitude into [2^14, 2^15), below fp16's
-// 65504 (1 for an empty row or one with an infinity or NaN; at most 2^100, so that it and its
-// reciprocal are normal numbers).
-__device__ __forceinline__ float row_scale(float largest) {
+// The exponent of the power of two that brings a vector's largest magnitude into [2^14, 2^15),
+// below fp16's 65504 (0 for an empty vector or one with an infinity or NaN; -113..100, so that
+// the power and its reciprocal are normal numbers).
+__device__ __forceinline__ int scale_exp(float largest) {
     const int e = static_cast<int>(__float_as_uint(largest) >> 23);  // biased exponent, 0 for 0 and subnormals
-    if (largest == 0.0f || e == 255) return 1.0f;
-    return __uint_as_float(static_cast<uint32_t>(std::min(141 - e, 100) + 127) << 23);
+    return largest == 0.0f || e == 255 ? 0 : std::min(141 - e, 100);
 }
-
-// the smaller of sc and the scale of a query with this largest magnitude (an empty query and
-// one with an infinity or NaN do not count: their products are 0, infinite or NaN at any scale)
-__device__ __forceinline__ float query_scale(float largest, float sc) {
-    return largest == 0.0f || largest == __builtin_inff() ? sc : fminf(sc, row_scale(largest));
-}
+__device__ __forceinline__ float exp2i(int e) { return __uint_as_float(static_cast<uint32_t>(e + 127) << 23); }
 
 constexpr int NP = 3;  // fp16 planes of a value: h, m, l
 
@@ -132,7 +126,7 @@ __global__ void __launch_bounds__(256) gt_split(const float* vecs, uint64_t row0
                 }
             }
         big = fmaxf(big, bsw::xor_lane_f<32>(big));
-        const float sc = row_scale(big);
+        const float sc = exp2i(scale_exp(big));
 #pragma unroll
         for (int kc = 0; kc < KC; ++kc) {
             f16x8 p[NP];
@@ -203,15 +197,13 @@ __device__ __forceinline__ uint64_t sort_descending(uint64_t v) {
 }
 
 // A operands of a wavefront: block b, lane (l32, half): query q0 + 32 b + l32, dimensions
-// 16 kc + 8 half + i; returns 1 / the scale.
-// All the wavefront's queries share one scale, the largest query's: a query 2^k smaller
-// keeps 2^(k - 29) of its own largest value and above in 11-bit planes, and the certificate
-// counts what is lost below (gt_refine).
+// 16 kc + 8 half + i, scaled by 2^-qe[b].  Each query has its own scale, as each row has, so what
+// a query loses below fp16's range does not depend on its neighbours.
 template <int KC, int QB>
-__device__ __forceinline__ float load_queries(const float* queries, uint32_t dim, uint64_t nq, uint64_t q0,
-                                              f16x8 (&a)[QB][KC][NP]) {
+__device__ __forceinline__ void load_queries(const float* queries, uint32_t dim, uint64_t nq, uint64_t q0,
+                                             f16x8 (&a)[QB][KC][NP], int (&qe)[QB]) {
     const uint32_t lane = lane_id(), half = lane >> 5, l32 = lane & 31u;
-    float x[QB][KC][8], sc = 0x1p100f;
+    float x[QB][KC][8];
 #pragma unroll
     for (int b = 0; b < QB; ++b) {
         const uint64_t qi = q0 + 32u * b + l32;
@@ -234,11 +226,9 @@ __device__ __forceinline__ float load_queries(const float* queries, uint32_t dim
                 big = fabsf(v) > big || v != v ? (v != v ? __builtin_inff() : fabsf(v)) : big;
             }
         big = fmaxf(big, bsw::xor_lane_f<32>(big));
-        sc = query_scale(big, sc);
-    }
-    sc = bsw::wave_min(sc);
-#pragma unroll
-    for (int b = 0; b < QB; ++b)
+        const int e = scale_exp(big);
+        const float sc = exp2i(e);
+        qe[b] = -e;
 #pragma unroll
         for (int kc = 0; kc < KC; ++kc)
 #pragma unroll
@@ -248,7 +238,7 @@ __device__ __forceinline__ float load_queries(const float* queries, uint32_t dim
 #pragma unroll
                 for (int p = 0; p < NP; ++p) a[b][kc][p][i] = v[p];
             }
-    return 1.0f / sc;
+    }
 }
 
 // A wavefront holds 32 QB queries as A operands (KC steps of 16 dimensions x 3 planes) and
@@ -262,7 +252,7 @@ __device__ __forceinline__ float load_queries(const float* queries, uint32_t dim
 // two products are most of the sum and both round once, 1.0-1.27 (the matrix unit's rounding).  Two planes and three products
 // hold 22 to 24 of the 24 bits: 1.9-2.9 there and up to 1.27 on wide-ranged data.
 // Six fp16 products of 16 dimensions take 192 matrix cycles, eight v_mfma_f32_32x32x2f32 512.
-// 500k x 128, 10k queries: 17.1 -> 8.3 ms with the filtering below.
+// 500k x 128, 10k queries: 17.1 -> 8.7 ms with the filtering below.
 // Two query blocks per wavefront (dim <= 128) halve the base bytes per product.
 //
 // The matrix pipe and the vector unit work at the same time: while tile t's products run, tile
@@ -282,7 +272,7 @@ template <int KC, int QB>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 gt_select(const uint4* frag, const float2* meta, uint64_t row0, uint64_t m, const float* queries, uint32_t dim,
           uint64_t nq, uint32_t nsplit, uint32_t split_tiles, uint32_t fresh, uint64_t* topc, uint32_t* tshare,
-          uint32_t* pub, float* qscale) {
+          uint32_t* pub) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const uint32_t lane = lane_id(), wave = bsw::uniform(threadIdx.x >> 6), half = lane >> 5, l32 = lane & 31u;
     constexpr uint32_t NQ = 32 * QB;
@@ -303,8 +293,17 @@ gt_select(const uint4* frag, const float2* meta, uint64_t row0, uint64_t m, cons
     uint32_t* cnt = reinterpret_cast<uint32_t*>(my + NQ * BUF * 8 + 32 * TS * 4);  // keys in each query's buffer
 
     f16x8 a[QB][KC][NP];
-    const float qinv = load_queries<KC, QB>(queries, dim, nq, qb * NQ, a);
-    if (s == 0 && lane == 0) qscale[qb] = qinv;
+    int qe[QB];
+    load_queries<KC, QB>(queries, dim, nq, qb * NQ, a, qe);
+    // the exponents by accumulator register, a byte each (a register each, 16 QB, does not fit: 10.3
+    // ms for 10k queries, 500k x 128; in bytes 9.85; one scale for the wavefront's queries 9.5):
+    // byte r % 4 of qep[b][r / 4] is that of query 32 b + acc_row(r, half)
+    int qep[QB][4] = {};
+#pragma unroll
+    for (int b = 0; b < QB; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            qep[b][r / 4] |= (__builtin_amdgcn_ds_bpermute(static_cast<int>(acc_row(r, half) << 2), qe[b]) & 0xFF) << (8 * (r % 4));
     // tau: per accumulator register, the threshold of its query (a float compare passes a
     // superset of the list's key order; none passes for a query past nq).  Lane i's tq is query
     // i's.
@@ -451,6 +450,11 @@ gt_select(const uint4* frag, const float2* meta, uint64_t row0, uint64_t m, cons
     float av[QB][16];
     auto step = [&](uint32_t tile, uint32_t next, f32x16 (&accN)[QB], const f32x16 (&accO)[QB], float2 mo) __attribute__((always_inline)) {
         uint32_t bits = 0;
+        // keeps the bytes packed: taken apart before the loop they are the 16 QB registers again
+#pragma unroll
+        for (int b = 0; b < QB; ++b)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) asm volatile("" : "+v"(qep[b][g]));
         constexpr int SMALL = 5 * QB, ALL = KC * (SMALL + QB);  // matrix instructions
         // the values screened beside instructions [m0, m1) of the tile's ALL
         auto screen = [&](int m0, int m1) __attribute__((always_inline)) {
@@ -458,8 +462,8 @@ gt_select(const uint4* frag, const float2* meta, uint64_t row0, uint64_t m, cons
             for (int e = 16 * QB * m0 / ALL; e < 16 * QB * m1 / ALL; ++e) {
                 const int b = e / 16, r = e % 16;
                 // a_j = |b_j|^2 - 2 acc / (row scale query scale): exact factors, one rounding
-                // (their product may underflow, so they are not combined)
-                av[b][r] = __builtin_fmaf(accO[b][r] * mo.y, qinv, mo.x);
+                const int e8 = static_cast<int>(static_cast<uint32_t>(qep[b][r / 4]) << (24 - 8 * (r % 4))) >> 24;
+                av[b][r] = __builtin_amdgcn_ldexpf(accO[b][r] * mo.y, e8) + mo.x;
                 bits |= !(av[b][r] > tau[b][r]) ? 1u << e : 0u;  // a NaN survives
             }
         };
@@ -638,7 +642,7 @@ constexpr uint32_t RF_TS = 64 + 4;  // floats per staged row: 16 lanes of a b128
 template <int NW>
 __global__ void __launch_bounds__(64 * NW) gt_refine(const float* vecs, uint32_t dstride, const float* queries,
                                                      uint32_t dim, uint32_t nsplit, const uint64_t* topc, uint32_t k,
-                                                     const uint32_t* bmax_bits, const float* qscale, uint32_t NQ,
+                                                     const uint32_t* bmax_bits,
                                                      int32_t* out, uint8_t* unc, unsigned long long* n_unc) {
     static_assert(NW >= 4, "four wavefronts score the candidates");
     __shared__ __attribute__((aligned(16))) uint64_t keys[NW][C];
@@ -756,17 +760,13 @@ __global__ void __launch_bounds__(64 * NW) gt_refine(const float* vecs, uint32_t
         // q.b's error, in 2^-24 |q||b|: dim roundings of the sum of the large products (dim; twice
         // that if the matrix unit truncates), 5 dim roundings of partial sums of the small ones,
         // each 2^-9 of it at most (0.02 dim), the dropped products (below 0.01), what lies below
-        // fp16's range in the row (2^-27 sqrt(dim): below sqrt(dim) / 8).  a_j doubles it; |b_j|^2
-        // and a_j are rounded once each.  (|q| + |b|)^2 >= 4 |q||b|, so 2 (dim + 3) 2^-24 (|q| +
-        // |b|)^2 grants 8 dim + 24 of 4.1 dim + sqrt(dim) / 4 + 2, and 6 |b|^2 of 2.  What lies
-        // below fp16's range in the query (2^-13 over the scale it shares with its neighbours) is
-        // 2^-13 qscale sqrt(dim) |b| at most.  A row whose largest value is below 2^-86 has the
-        // largest scale, 2^100: it loses 2^-113 per value.  2^-140: results below fp32's normal
-        // range.
-        const double sd = __builtin_sqrt(static_cast<double>(dim));
+        // fp16's range in the row and in the query (2^-27 sqrt(dim) each: below sqrt(dim) / 4
+        // together).  a_j doubles it; |b_j|^2 and a_j are rounded once each.  (|q| + |b|)^2 >=
+        // 4 |q||b|, so 2 (dim + 3) 2^-24 (|q| + |b|)^2 grants 8 dim + 24 of 4.1 dim + sqrt(dim) / 2
+        // + 2, and 6 |b|^2 of 2.  A vector whose largest value is below 2^-86 has the largest
+        // scale, 2^100: it loses 2^-113 per value.  2^-140: results below fp32's normal range.
         const double eps = 2.0 * (dim + 3) * 0x1p-24 * qb * qb +
-                           2.0 * 0x1p-13 * static_cast<double>(qscale[qi / NQ]) * sd * bm +
-                           2.0 * 0x1p-113 * sd * __builtin_sqrt(qn2) + 0x1p-140;
+                           2.0 * 0x1p-113 * __builtin_sqrt(static_cast<double>(dim)) * qb + 0x1p-140;
         ok = dk < ac + qn2 - eps;
     }
     if (lane == 0) {
@@ -782,7 +782,8 @@ __global__ void __launch_bounds__(64) dbg_products(const uint4* frag, const floa
                                                    uint32_t dim, float* out) {
     const uint32_t lane = lane_id(), half = lane >> 5, l32 = lane & 31u, t = blockIdx.x;
     f16x8 a[1][KC][NP];
-    const float qinv = load_queries<KC, 1>(queries, dim, 32, 0, a);
+    int qe[1];
+    load_queries<KC, 1>(queries, dim, 32, 0, a, qe);
     auto b = [&](int kc, int p) __attribute__((always_inline)) {
         return __builtin_bit_cast(f16x8, frag[((static_cast<uint64_t>(t) * KC + kc) * NP + p) * 64 + lane]);
     };
@@ -800,7 +801,8 @@ __global__ void __launch_bounds__(64) dbg_products(const uint4* frag, const floa
     for (int kc = 0; kc < KC; ++kc) mul(kc, 0, 0);
     const float binv = -0.5f * meta[t * 32u + l32].y;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) out[(static_cast<uint64_t>(acc_row(r, half)) * gridDim.x + t) * 32 + l32] = acc[r] * binv * qinv;
+    for (int r = 0; r < 16; ++r) out[(static_cast<uint64_t>(acc_row(r, half)) * gridDim.x + t) * 32 + l32] =
+        __builtin_amdgcn_ldexpf(acc[r] * binv, __builtin_amdgcn_ds_bpermute(static_cast<int>(acc_row(r, half) << 2), qe[0]));
 }
 
 // the same products from the fp32 instruction (lane half h: dimensions KC 8 h ..), one chain
@@ -845,13 +847,13 @@ int gfail(int code, const std::string& msg) {
 template <int KC, int QB>
 hipError_t launch_select(dim3 g, hipStream_t s, const uint4* frag, const float2* meta, uint64_t row0, uint64_t m,
                          const float* q, uint32_t dim, uint64_t nq, uint32_t nsplit, uint32_t split_tiles,
-                         uint64_t* topc, uint32_t* tshare, uint32_t* pub, float* qscale) {
+                         uint64_t* topc, uint32_t* tshare, uint32_t* pub) {
     constexpr int lds = 4 * bsg::lds_wave(QB);
     auto k = bsg::gt_select<KC, QB>;
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k, g, dim3(256), lds, s, frag, meta, row0, m, q, dim, nq, nsplit, split_tiles,
-                       row0 == 0 ? 1u : 0u, topc, tshare, pub, qscale);
+                       row0 == 0 ? 1u : 0u, topc, tshare, pub);
     return hipGetLastError();
 }
 
@@ -927,7 +929,7 @@ extern "C" int bs_index_groundtruth_device(bs_index idx, const float* d_queries,
     const uint64_t o_bn = al(chunk * tile_bytes), o_top = o_bn + al(chunk * 32 * 8),
                    o_share = o_top + al(nq * nsplit * bsg::C * 8),
                    o_pub = o_share + nq * 4,  // tshare and pub start as all ones together
-                   o_cnt = al(o_pub + std::min<uint64_t>(nsplit, bsg::PUB) * nq * 4), o_qs = o_cnt + 256, need = o_qs + nqb * 4;
+                   o_cnt = al(o_pub + std::min<uint64_t>(nsplit, bsg::PUB) * nq * 4), need = o_cnt + 256;
     char* ws = nullptr;
     if (hipMalloc(reinterpret_cast<void**>(&ws), need) != hipSuccess)
         return gfail(BS_ENOMEM, "hipMalloc of the ground-truth work buffers failed");
@@ -938,7 +940,6 @@ extern "C" int bs_index_groundtruth_device(bs_index idx, const float* d_queries,
     uint32_t* pub = reinterpret_cast<uint32_t*>(ws + o_pub);
     unsigned long long* nunc = reinterpret_cast<unsigned long long*>(ws + o_cnt);
     uint32_t* bmax = reinterpret_cast<uint32_t*>(ws + o_cnt + 8);
-    float* qscale = reinterpret_cast<float*>(ws + o_qs);
     hipError_t e = hipMemsetAsync(nunc, 0, 16, s);
     if (e == hipSuccess) e = hipMemsetAsync(tshare, 0xFF, o_cnt - o_share, s);  // no bound published yet
     const dim3 g(static_cast<uint32_t>((nqb * nsplit + 3) / 4));
@@ -952,7 +953,7 @@ extern "C" int bs_index_groundtruth_device(bs_index idx, const float* d_queries,
             if (le != hipSuccess) return le;
             return launch_select<K, decltype(qb)::value>(g, s, frag, meta, row0, m, d_queries, dim, nq,
                                                          static_cast<uint32_t>(nsplit),
-                                                         static_cast<uint32_t>(split_tiles), topc, tshare, pub, qscale);
+                                                         static_cast<uint32_t>(split_tiles), topc, tshare, pub);
         };
         e = with_steps(KC, go);
     }
@@ -960,12 +961,12 @@ extern "C" int bs_index_groundtruth_device(bs_index idx, const float* d_queries,
         // a wavefront merges a list in ~0.3 us: with many splits (few queries) 16 share them
         if (nsplit > 32)
             hipLaunchKernelGGL(bsg::gt_refine<16>, dim3(static_cast<uint32_t>(nq)), dim3(1024), 0, s, vecs, dstride,
-                               d_queries, dim, static_cast<uint32_t>(nsplit), topc, k, bmax, qscale,
-                               NQ, d_out, d_uncertified, nunc);
+                               d_queries, dim, static_cast<uint32_t>(nsplit), topc, k, bmax,
+                               d_out, d_uncertified, nunc);
         else
             hipLaunchKernelGGL(bsg::gt_refine<4>, dim3(static_cast<uint32_t>(nq)), dim3(256), 0, s, vecs, dstride,
-                               d_queries, dim, static_cast<uint32_t>(nsplit), topc, k, bmax, qscale,
-                               NQ, d_out, d_uncertified, nunc);
+                               d_queries, dim, static_cast<uint32_t>(nsplit), topc, k, bmax,
+                               d_out, d_uncertified, nunc);
         e = hipGetLastError();
     }
     unsigned long long nu = 0;

@@ -96,8 +96,8 @@ def test_groundtruth_rows_sorted_by_distance(gpu):
 
 @pytest.mark.parametrize("scale", [2.0 ** -60, 2.0 ** -20, 1.0, 2.0 ** 20, 2.0 ** 50])
 def test_groundtruth_scales(gpu, scale):
-    """fp16 operands are scaled per row: any magnitude, and queries of one block that differ by
-    2^12 from each other, stay certified"""
+    """fp16 operands are scaled per row and query: any magnitude stays certified, also beside queries
+    of the block that are 2^12 smaller"""
     base = (host.gen_normalized(9000, 100, 31) * np.float32(scale)).astype(np.float32)
     base[::7] *= np.float32(2.0 ** -9)
     q = (host.gen_normalized(96, 100, 32) * np.float32(scale)).astype(np.float32)
@@ -201,3 +201,23 @@ def test_groundtruth_products_precision(gpu, dim):
     q = (1 + rng.random((32, dim))).astype(np.float32)
     exact = q.astype(np.float64) @ b.astype(np.float64).T
     assert (np.abs(search.debug_gt_products(b, q) - exact) <= 2.0 ** -23 * np.abs(exact)).all()
+
+
+@pytest.mark.parametrize("dim", [24, 100, 128, 250])
+def test_groundtruth_query_beside_larger_ones(gpu, dim):
+    """a query's candidates and certificate are its own: queries 10^4 and 10^30 times larger in its
+    block of 64 change nothing"""
+    base = host.gen_mixture(6000, dim, 16, 0.0, 1.0, 0.1, 0.0, 61, 62)
+    q = host.gen_mixture(130, dim, 16, 0.0, 1.0, 0.1, 0.0, 61, 63)
+    g = search.GPUGraph(base, np.zeros((6000, 1), np.uint32))
+    alone = g.groundtruth(q, 20, exact_fallback=False)
+    assert (alone != -2).all(1).mean() >= 0.95
+    large = q.copy()
+    large[5] *= np.float32(1e4)
+    large[70] = np.float32(1e30)
+    large[129] *= np.float32(1e30)
+    raw = g.groundtruth(large, 20, exact_fallback=False)
+    rest = np.setdiff1d(np.arange(130), [5, 70, 129])
+    assert np.array_equal(raw[rest], alone[rest])
+    cert = (raw != -2).all(1)
+    assert np.array_equal(raw[cert], host.groundtruth(base, large, 20)[cert])
