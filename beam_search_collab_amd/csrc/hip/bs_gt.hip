@@ -198,10 +198,11 @@ __device__ __forceinline__ uint64_t sort_descending(uint64_t v) {
 
 // A operands of a wavefront: block b, lane (l32, half): query q0 + 32 b + l32, dimensions
 // 16 kc + 8 half + i, scaled by 2^-qe[b].  Each query has its own scale, as each row has, so what
-// a query loses below fp16's range does not depend on its neighbours.
+// a query loses below fp16's range does not depend on its neighbours.  Bit i of nanq[b]: query
+// 32 b + i has a NaN.
 template <int KC, int QB>
 __device__ __forceinline__ void load_queries(const float* queries, uint32_t dim, uint64_t nq, uint64_t q0,
-                                             f16x8 (&a)[QB][KC][NP], int (&qe)[QB]) {
+                                             f16x8 (&a)[QB][KC][NP], int (&qe)[QB], uint32_t (&nanq)[QB]) {
     const uint32_t lane = lane_id(), half = lane >> 5, l32 = lane & 31u;
     float x[QB][KC][8];
 #pragma unroll
@@ -216,6 +217,7 @@ __device__ __forceinline__ void load_queries(const float* queries, uint32_t dim,
                 x[b][kc][i] = qv[d < dim ? d : 0u];
             }
         float big = 0.0f;
+        bool nan = false;
 #pragma unroll
         for (int kc = 0; kc < KC; ++kc)
 #pragma unroll
@@ -223,9 +225,12 @@ __device__ __forceinline__ void load_queries(const float* queries, uint32_t dim,
                 const uint32_t d = 16u * kc + 8u * half + i;
                 const float v = qi < nq && d < dim ? x[b][kc][i] : 0.0f;
                 x[b][kc][i] = v;
+                nan = nan || v != v;
                 big = fabsf(v) > big || v != v ? (v != v ? __builtin_inff() : fabsf(v)) : big;
             }
         big = fmaxf(big, bsw::xor_lane_f<32>(big));
+        const uint64_t nm = ballot(nan);
+        nanq[b] = static_cast<uint32_t>(nm | (nm >> 32));
         const int e = scale_exp(big);
         const float sc = exp2i(e);
         qe[b] = -e;
@@ -294,7 +299,8 @@ gt_select(const uint4* frag, const float2* meta, uint64_t row0, uint64_t m, cons
 
     f16x8 a[QB][KC][NP];
     int qe[QB];
-    load_queries<KC, QB>(queries, dim, nq, qb * NQ, a, qe);
+    uint32_t nanq[QB];
+    load_queries<KC, QB>(queries, dim, nq, qb * NQ, a, qe, nanq);
     // the exponents by accumulator register, a byte each (a register each, 16 QB, does not fit: 10.3
     // ms for 10k queries, 500k x 128; in bytes 9.85; one scale for the wavefront's queries 9.5):
     // byte r % 4 of qep[b][r / 4] is that of query 32 b + acc_row(r, half)
@@ -309,9 +315,14 @@ gt_select(const uint4* frag, const float2* meta, uint64_t row0, uint64_t m, cons
     // i's.
     float tq = qb * NQ + lane < nq && lane < NQ ? __builtin_inff() : -__builtin_inff();
     float tau[QB][16];
-    uint32_t real = 0;  // the bits of `bits` (below) whose query exists
+    // the bits of `bits` (below) whose query exists and has no NaN: a query with one has no
+    // neighbours, and every row would survive for it
+    uint32_t real = 0;
 #pragma unroll
-    for (int e = 0; e < 16 * QB; ++e) real |= qb * NQ + 32u * (e / 16) + acc_row(e % 16, half) < nq ? 1u << e : 0u;
+    for (int e = 0; e < 16 * QB; ++e) {
+        const uint32_t i = acc_row(e % 16, half);
+        real |= qb * NQ + 32u * (e / 16) + i < nq && !((nanq[e / 16] >> i) & 1u) ? 1u << e : 0u;
+    }
     // queries whose list has been written to HBM (each lane re-reads only what it wrote)
     uint64_t written = fresh ? 0ull : ~0ull;
 
@@ -783,7 +794,8 @@ __global__ void __launch_bounds__(64) dbg_products(const uint4* frag, const floa
     const uint32_t lane = lane_id(), half = lane >> 5, l32 = lane & 31u, t = blockIdx.x;
     f16x8 a[1][KC][NP];
     int qe[1];
-    load_queries<KC, 1>(queries, dim, 32, 0, a, qe);
+    uint32_t nanq[1];
+    load_queries<KC, 1>(queries, dim, 32, 0, a, qe, nanq);
     auto b = [&](int kc, int p) __attribute__((always_inline)) {
         return __builtin_bit_cast(f16x8, frag[((static_cast<uint64_t>(t) * KC + kc) * NP + p) * 64 + lane]);
     };
