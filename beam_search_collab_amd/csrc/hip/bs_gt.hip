@@ -885,6 +885,8 @@ hipError_t with_steps(uint32_t KC, F&& f) {
     }
 }
 
+constexpr uint64_t REFINE_QUERIES = 1ull << 21;
+
 // Row splits per query block: nqb * nsplit wavefronts run 4 per CU (a SIMD holds one), so the
 // count is the one that fills whole rounds of them best, few rounds and few splits first (a
 // split costs its query another list of 128 to fill, publish and merge).  At least 8 tiles
@@ -969,16 +971,17 @@ extern "C" int bs_index_groundtruth_device(bs_index idx, const float* d_queries,
         };
         e = with_steps(KC, go);
     }
-    if (e == hipSuccess) {
-        // a wavefront merges a list in ~0.3 us: with many splits (few queries) 16 share them
-        if (nsplit > 32)
-            hipLaunchKernelGGL(bsg::gt_refine<16>, dim3(static_cast<uint32_t>(nq)), dim3(1024), 0, s, vecs, dstride,
-                               d_queries, dim, static_cast<uint32_t>(nsplit), topc, k, bmax,
-                               d_out, d_uncertified, nunc);
-        else
-            hipLaunchKernelGGL(bsg::gt_refine<4>, dim3(static_cast<uint32_t>(nq)), dim3(256), 0, s, vecs, dstride,
-                               d_queries, dim, static_cast<uint32_t>(nsplit), topc, k, bmax,
-                               d_out, d_uncertified, nunc);
+    // a wavefront merges a list in ~0.3 us: with many splits (few queries) 16 share them.  At most
+    // 2^21 queries per launch: a grid of 2^32 work-items is cut short without an error.
+    for (uint64_t q0 = 0; e == hipSuccess && q0 < nq; q0 += REFINE_QUERIES) {
+        const dim3 rg(static_cast<uint32_t>(std::min<uint64_t>(REFINE_QUERIES, nq - q0)));
+        auto go = [&](auto kernel, uint32_t threads) {
+            hipLaunchKernelGGL(kernel, rg, dim3(threads), 0, s, vecs, dstride, d_queries + q0 * dim, dim,
+                               static_cast<uint32_t>(nsplit), topc + q0 * nsplit * bsg::C, k, bmax, d_out + q0 * k,
+                               d_uncertified ? d_uncertified + q0 : nullptr, nunc);
+        };
+        if (nsplit > 32) go(bsg::gt_refine<16>, 1024);
+        else go(bsg::gt_refine<4>, 256);
         e = hipGetLastError();
     }
     unsigned long long nu = 0;

@@ -222,3 +222,19 @@ def test_groundtruth_query_beside_larger_ones(gpu, dim):
     assert np.array_equal(raw[rest], alone[rest])
     cert = (raw != -2).all(1)
     assert np.array_equal(raw[cert], host.groundtruth(base, large, 20)[cert])
+
+
+def test_groundtruth_many_queries(gpu):
+    """more queries than one launch takes with a workgroup for each (2^32 work-items)"""
+    rng = np.random.default_rng(71)
+    nq = (1 << 24) + 100
+    base = rng.random((200, 2), dtype=np.float32)
+    q = rng.random((nq, 2), dtype=np.float32)
+    g = search.GPUGraph(base, np.zeros((200, 1), np.uint32))
+    raw = g.groundtruth(q, 1, exact_fallback=False)
+    assert (raw != -2).mean() >= 0.95
+    step = 1 << 21  # the queries of one launch
+    at = np.unique(np.clip(np.arange(0, nq + step, step)[:, None] + np.arange(-40, 40), 0, nq - 1))
+    at = np.unique(np.concatenate([at, rng.integers(0, nq, 2000)]))
+    cert = raw[at, 0] != -2
+    assert np.array_equal(raw[at][cert], host.groundtruth(base, q[at], 1)[cert])
