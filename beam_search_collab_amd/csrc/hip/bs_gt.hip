@@ -906,11 +906,45 @@ uint64_t pick_splits(uint64_t nqb, uint64_t tiles, uint64_t slots) {
     return best;
 }
 
-}  // namespace
+// How a call is cut up, and its one work buffer: planes, norms, lists, published values, counters.
+struct Plan {
+    uint32_t KC;   // 16-dimension steps
+    uint64_t nqb;  // query blocks: 64 queries per wavefront while their operands fit beside a tile's, else 32
+    uint64_t tiles, chunk, nsplit, split_tiles;  // tiles of the base, held as planes at a time, per split
+    uint64_t tile_bytes, o_bn, o_top, o_share, o_pub, o_cnt, need;
+};
+Plan make_plan(uint64_t n, uint64_t nq, uint32_t dim, uint32_t cus, uint64_t plane_bytes) {
+    auto al = [](uint64_t v) { return (v + 255) & ~255ull; };
+    Plan p;
+    p.KC = steps_of(dim);
+    const uint32_t NQ = p.KC <= 8 ? 64 : 32;
+    p.nqb = (nq + NQ - 1) / NQ;
+    p.tile_bytes = static_cast<uint64_t>(p.KC) * bsg::NP * 1024;
+    p.tiles = (n + 31) / 32;
+    p.chunk = std::max<uint64_t>(1, std::min<uint64_t>(p.tiles, plane_bytes / p.tile_bytes));
+    p.nsplit = pick_splits(p.nqb, p.chunk, 4ull * cus);
+    p.split_tiles = (p.chunk + p.nsplit - 1) / p.nsplit;
+    p.o_bn = al(p.chunk * p.tile_bytes);
+    p.o_top = p.o_bn + al(p.chunk * 32 * 8);
+    p.o_share = p.o_top + al(nq * p.nsplit * bsg::C * 8);
+    p.o_pub = p.o_share + nq * 4;  // tshare and pub start as all ones together
+    p.o_cnt = al(p.o_pub + std::min<uint64_t>(p.nsplit, bsg::PUB) * nq * 4);
+    p.need = p.o_cnt + 256;
+    return p;
+}
+constexpr uint64_t PLANE_BYTES = 1ull << 30;  // of planes at a time, where there is room; the lists carry over
 
-extern "C" int bs_index_groundtruth_device(bs_index idx, const float* d_queries, uint64_t nq, uint32_t k,
-                                           int32_t* d_out, uint8_t* d_uncertified, void* stream,
-                                           uint64_t* n_uncertified) try {
+uint32_t device_cus() {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+        return 256;
+    return static_cast<uint32_t>(cus);
+}
+
+// ws_limit: the largest work buffer that may be allocated
+int groundtruth(bs_index idx, const float* d_queries, uint64_t nq, uint32_t k, int32_t* d_out, uint8_t* d_uncertified,
+                hipStream_t s, uint64_t* n_uncertified, uint64_t ws_limit) {
     const float* vecs = nullptr;
     uint32_t dstride = 0;
     int rc = bs_internal_vecs(idx, &vecs, &dstride);
@@ -923,42 +957,29 @@ extern "C" int bs_index_groundtruth_device(bs_index idx, const float* d_queries,
     if (dim > 256) return gfail(BS_EINVAL, "the device ground truth supports dim <= 256");
     if (nq == 0) return BS_OK;
     if (!d_queries || !d_out) return gfail(BS_EINVAL, "queries and output must be given");
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-        cus = 256;
-    // 16-dimension steps, and 64 queries per wavefront while their operands fit beside a tile's
-    const uint32_t KC = steps_of(dim);
-    const uint32_t NQ = KC <= 8 ? 64 : 32;
-    const uint64_t nqb = (nq + NQ - 1) / NQ;
-    // the fp16 planes are made for at most 1 GiB of rows at a time; the lists carry over
-    const uint64_t tile_bytes = static_cast<uint64_t>(KC) * bsg::NP * 1024;
-    const uint64_t tiles = (n + 31) / 32, chunk = std::min<uint64_t>(tiles, (1ull << 30) / tile_bytes);
-    const uint64_t nsplit = pick_splits(nqb, chunk, 4ull * static_cast<uint64_t>(cus));
-    const uint64_t split_tiles = (chunk + nsplit - 1) / nsplit;
-
-    // one allocation: planes, norms, lists, published values, counters
-    auto al = [](uint64_t v) { return (v + 255) & ~255ull; };
-    const uint64_t o_bn = al(chunk * tile_bytes), o_top = o_bn + al(chunk * 32 * 8),
-                   o_share = o_top + al(nq * nsplit * bsg::C * 8),
-                   o_pub = o_share + nq * 4,  // tshare and pub start as all ones together
-                   o_cnt = al(o_pub + std::min<uint64_t>(nsplit, bsg::PUB) * nq * 4), need = o_cnt + 256;
+    const uint32_t cus = device_cus();
+    // where the work buffer does not fit, planes of half as many rows at a time, down to 8 tiles
+    // (500k x 128, 10k queries: 9.7 ms with the 450 MB it takes, 9.6 with 200, 10.7 with 100, 51
+    // with 40)
+    Plan p = make_plan(n, nq, dim, cus, PLANE_BYTES);
     char* ws = nullptr;
-    if (hipMalloc(reinterpret_cast<void**>(&ws), need) != hipSuccess)
-        return gfail(BS_ENOMEM, "hipMalloc of the ground-truth work buffers failed");
+    while (p.need > ws_limit || hipMalloc(reinterpret_cast<void**>(&ws), p.need) != hipSuccess) {
+        (void)hipGetLastError();
+        if (p.chunk <= 8) return gfail(BS_ENOMEM, "hipMalloc of the ground-truth work buffers failed");
+        p = make_plan(n, nq, dim, cus, p.chunk / 2 * p.tile_bytes);
+    }
     uint4* frag = reinterpret_cast<uint4*>(ws);
-    float2* meta = reinterpret_cast<float2*>(ws + o_bn);
-    uint64_t* topc = reinterpret_cast<uint64_t*>(ws + o_top);
-    uint32_t* tshare = reinterpret_cast<uint32_t*>(ws + o_share);
-    uint32_t* pub = reinterpret_cast<uint32_t*>(ws + o_pub);
-    unsigned long long* nunc = reinterpret_cast<unsigned long long*>(ws + o_cnt);
-    uint32_t* bmax = reinterpret_cast<uint32_t*>(ws + o_cnt + 8);
+    float2* meta = reinterpret_cast<float2*>(ws + p.o_bn);
+    uint64_t* topc = reinterpret_cast<uint64_t*>(ws + p.o_top);
+    uint32_t* tshare = reinterpret_cast<uint32_t*>(ws + p.o_share);
+    uint32_t* pub = reinterpret_cast<uint32_t*>(ws + p.o_pub);
+    unsigned long long* nunc = reinterpret_cast<unsigned long long*>(ws + p.o_cnt);
+    uint32_t* bmax = reinterpret_cast<uint32_t*>(ws + p.o_cnt + 8);
     hipError_t e = hipMemsetAsync(nunc, 0, 16, s);
-    if (e == hipSuccess) e = hipMemsetAsync(tshare, 0xFF, o_cnt - o_share, s);  // no bound published yet
-    const dim3 g(static_cast<uint32_t>((nqb * nsplit + 3) / 4));
-    for (uint64_t c0 = 0; e == hipSuccess && c0 < tiles; c0 += chunk) {
-        const uint64_t row0 = c0 * 32, m = std::min(chunk * 32, n - row0), mt = (m + 31) / 32;
+    if (e == hipSuccess) e = hipMemsetAsync(tshare, 0xFF, p.o_cnt - p.o_share, s);  // no bound published yet
+    const dim3 g(static_cast<uint32_t>((p.nqb * p.nsplit + 3) / 4));
+    for (uint64_t c0 = 0; e == hipSuccess && c0 < p.tiles; c0 += p.chunk) {
+        const uint64_t row0 = c0 * 32, m = std::min(p.chunk * 32, n - row0), mt = (m + 31) / 32;
         const dim3 sg(static_cast<uint32_t>(std::min<uint64_t>((mt + 3) / 4, 8ull * cus)));
         auto go = [&](auto kc, auto qb) {
             constexpr int K = decltype(kc)::value;
@@ -966,10 +987,10 @@ extern "C" int bs_index_groundtruth_device(bs_index idx, const float* d_queries,
             const hipError_t le = hipGetLastError();
             if (le != hipSuccess) return le;
             return launch_select<K, decltype(qb)::value>(g, s, frag, meta, row0, m, d_queries, dim, nq,
-                                                         static_cast<uint32_t>(nsplit),
-                                                         static_cast<uint32_t>(split_tiles), topc, tshare, pub);
+                                                         static_cast<uint32_t>(p.nsplit),
+                                                         static_cast<uint32_t>(p.split_tiles), topc, tshare, pub);
         };
-        e = with_steps(KC, go);
+        e = with_steps(p.KC, go);
     }
     // a wavefront merges a list in ~0.3 us: with many splits (few queries) 16 share them.  At most
     // 2^21 queries per launch: a grid of 2^32 work-items is cut short without an error.
@@ -977,10 +998,10 @@ extern "C" int bs_index_groundtruth_device(bs_index idx, const float* d_queries,
         const dim3 rg(static_cast<uint32_t>(std::min<uint64_t>(REFINE_QUERIES, nq - q0)));
         auto go = [&](auto kernel, uint32_t threads) {
             hipLaunchKernelGGL(kernel, rg, dim3(threads), 0, s, vecs, dstride, d_queries + q0 * dim, dim,
-                               static_cast<uint32_t>(nsplit), topc + q0 * nsplit * bsg::C, k, bmax, d_out + q0 * k,
+                               static_cast<uint32_t>(p.nsplit), topc + q0 * p.nsplit * bsg::C, k, bmax, d_out + q0 * k,
                                d_uncertified ? d_uncertified + q0 : nullptr, nunc);
         };
-        if (nsplit > 32) go(bsg::gt_refine<16>, 1024);
+        if (p.nsplit > 32) go(bsg::gt_refine<16>, 1024);
         else go(bsg::gt_refine<4>, 256);
         e = hipGetLastError();
     }
@@ -991,12 +1012,11 @@ extern "C" int bs_index_groundtruth_device(bs_index idx, const float* d_queries,
     if (e != hipSuccess) return gfail(BS_EHIP, std::string("ground truth: ") + hipGetErrorString(e));
     if (n_uncertified) *n_uncertified = nu;
     return BS_OK;
-} catch (...) {
-    return bs_internal_exception();
 }
 
-extern "C" int bs_index_groundtruth(bs_index idx, const float* queries, uint64_t nq, uint32_t k, int32_t* out,
-                                    uint8_t* uncertified, uint64_t* n_uncertified) try {
+// the same on host buffers
+int groundtruth_host(bs_index idx, const float* queries, uint64_t nq, uint32_t k, int32_t* out, uint8_t* uncertified,
+                     uint64_t* n_uncertified, uint64_t ws_limit) {
     if (nq == 0) {
         if (n_uncertified) *n_uncertified = 0;
         return BS_OK;
@@ -1022,7 +1042,7 @@ extern "C" int bs_index_groundtruth(bs_index idx, const float* queries, uint64_t
         release();
         return gfail(BS_EHIP, "query upload failed");
     }
-    rc = bs_index_groundtruth_device(idx, dq, nq, k, dout, dunc, nullptr, n_uncertified);
+    rc = groundtruth(idx, dq, nq, k, dout, dunc, nullptr, n_uncertified, ws_limit);
     if (rc == BS_OK) {
         hipError_t e = hipMemcpy(out, dout, nq * k * 4, hipMemcpyDeviceToHost);
         if (e == hipSuccess && uncertified) e = hipMemcpy(uncertified, dunc, nq, hipMemcpyDeviceToHost);
@@ -1030,6 +1050,27 @@ extern "C" int bs_index_groundtruth(bs_index idx, const float* queries, uint64_t
     }
     release();
     return rc;
+}
+}  // namespace
+
+extern "C" int bs_index_groundtruth_device(bs_index idx, const float* d_queries, uint64_t nq, uint32_t k,
+                                           int32_t* d_out, uint8_t* d_uncertified, void* stream,
+                                           uint64_t* n_uncertified) try {
+    return groundtruth(idx, d_queries, nq, k, d_out, d_uncertified, static_cast<hipStream_t>(stream), n_uncertified, ~0ull);
+} catch (...) {
+    return bs_internal_exception();
+}
+
+extern "C" int bs_index_groundtruth(bs_index idx, const float* queries, uint64_t nq, uint32_t k, int32_t* out,
+                                    uint8_t* uncertified, uint64_t* n_uncertified) try {
+    return groundtruth_host(idx, queries, nq, k, out, uncertified, n_uncertified, ~0ull);
+} catch (...) {
+    return bs_internal_exception();
+}
+
+extern "C" int bs_debug_groundtruth(bs_index idx, const float* queries, uint64_t nq, uint32_t k, uint64_t ws_limit,
+                                    int32_t* out, uint8_t* uncertified) try {
+    return groundtruth_host(idx, queries, nq, k, out, uncertified, nullptr, ws_limit);
 } catch (...) {
     return bs_internal_exception();
 }

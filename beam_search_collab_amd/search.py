@@ -324,6 +324,17 @@ def debug_mfma32(A, B):
     return D
 
 
+def debug_groundtruth(graph, queries, k, ws_limit):
+    """GPUGraph.groundtruth with a work buffer of at most ws_limit bytes; -2 where uncertified"""
+    q = np.ascontiguousarray(queries, dtype=np.float32)
+    out = np.empty((q.shape[0], k), dtype=np.int32)
+    unc = np.zeros(q.shape[0], dtype=np.uint8)
+    _check(_lib.hip().bs_debug_groundtruth(graph._h, _ptr(q), q.shape[0], k, ws_limit, _ptr(out), _ptr(unc)),
+           "bs_debug_groundtruth")
+    out[unc != 0] = -2
+    return out
+
+
 def debug_gt_products(rows, queries, fp32=False):
     """q.b of 32 queries and n rows as the ground-truth candidates are selected by (bs_debug_gt_products)"""
     rows = np.ascontiguousarray(rows, dtype=np.float32)

@@ -274,6 +274,12 @@ int bs_debug_label_order(const uint32_t* labels, const float* lcost, uint64_t n,
  * one chain of v_mfma_f32_32x32x2f32 instead, to compare the rounding with. */
 int bs_debug_gt_products(const float* rows, uint32_t n, const float* queries, uint32_t dim, int fp32, float* out);
 
+/* bs_index_groundtruth with a work buffer of at most ws_limit bytes (a larger one counts as an
+ * allocation that failed: fewer rows are held as operands at a time, BS_ENOMEM when the lists alone
+ * do not fit). */
+int bs_debug_groundtruth(bs_index idx, const float* queries, uint64_t nq, uint32_t k, uint64_t ws_limit,
+                         int32_t* out, uint8_t* uncertified);
+
 /* One v_mfma_f32_32x32x2f32 product: A 32x2 and B 2x32 row-major in, D = A B 32x32
  * row-major out, read back through the accumulator layout the ground-truth kernel uses. */
 int bs_debug_mfma32(const float* A, const float* B, float* D);

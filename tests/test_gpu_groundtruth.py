@@ -238,3 +238,22 @@ def test_groundtruth_many_queries(gpu):
     at = np.unique(np.concatenate([at, rng.integers(0, nq, 2000)]))
     cert = raw[at, 0] != -2
     assert np.array_equal(raw[at][cert], host.groundtruth(base, q[at], 1)[cert])
+
+
+@pytest.mark.parametrize("n,nq,dim", [(20011, 70, 128), (9000, 300, 30), (15003, 33, 250)])
+def test_groundtruth_small_work_buffer(gpu, n, nq, dim):
+    """where the work buffer cannot be allocated, fewer rows are held as operands at a time, down to
+    8 tiles of 32: the same ids and certificates; an error only when the lists do not fit either"""
+    base = host.gen_mixture(n, dim, 16, 0.0, 128.0, 12.0, 0.0, 81, 82)
+    q = host.gen_mixture(nq, dim, 16, 0.0, 128.0, 12.0, 0.0, 81, 83)
+    g = search.GPUGraph(base, np.zeros((n, 1), np.uint32))
+    want = g.groundtruth(q, 50, exact_fallback=False)
+    cert = (want != -2).all(1)
+    assert cert.mean() >= 0.95
+    assert np.array_equal(want[cert], host.groundtruth(base, q, 50)[cert])
+    lists = nq * 1024  # one list of 128 keys per query
+    for limit in (8 << 20, 3 << 20, lists + (1 << 19)):
+        assert np.array_equal(search.debug_groundtruth(g, q, 50, limit), want)
+    with pytest.raises(search.BeamSearchError):
+        search.debug_groundtruth(g, q, 50, lists)
+    assert np.array_equal(g.groundtruth(q, 50, exact_fallback=False), want)
