@@ -183,8 +183,10 @@ int bs_internal_exception() {
     }
 }
 
-extern "C" int bs_index_create(const float* vecs, const uint32_t* edges, uint64_t n, uint32_t dim,
-                               uint32_t degree, bs_index* out) try {
+namespace {
+// calibrate false: as if the calibration had failed (the plain label order stays)
+int index_create(const float* vecs, const uint32_t* edges, uint64_t n, uint32_t dim, uint32_t degree, bs_index* out,
+                 bool calibrate) {
     if (!out) return fail(BS_EINVAL, "out is null");
     *out = nullptr;
     if (!vecs || !edges) return fail(BS_EINVAL, "vecs and edges must be given");
@@ -277,9 +279,29 @@ extern "C" int bs_index_create(const float* vecs, const uint32_t* edges, uint64_
         bs_index_destroy(ix);
         return fail(BS_EHIP, std::string("upload failed: ") + hipGetErrorString(e));
     }
-    calibrate_labels(ix);
+    if (calibrate) calibrate_labels(ix);
+    // The pivots and the cleared order workspace are done before any stream may search the index;
+    // the calibration has waited for them, unless it failed.
+    e = hipStreamSynchronize(nullptr);
+    if (e != hipSuccess) {
+        bs_index_destroy(ix);
+        return fail(BS_EHIP, std::string("upload failed: ") + hipGetErrorString(e));
+    }
     *out = ix;
     return BS_OK;
+}
+}  // namespace
+
+extern "C" int bs_index_create(const float* vecs, const uint32_t* edges, uint64_t n, uint32_t dim,
+                               uint32_t degree, bs_index* out) try {
+    return index_create(vecs, edges, n, dim, degree, out, true);
+} catch (...) {
+    return bs_internal_exception();
+}
+
+extern "C" int bs_debug_index_create_uncalibrated(const float* vecs, const uint32_t* edges, uint64_t n, uint32_t dim,
+                                                  uint32_t degree, bs_index* out) try {
+    return index_create(vecs, edges, n, dim, degree, out, false);
 } catch (...) {
     return bs_internal_exception();
 }

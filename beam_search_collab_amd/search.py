@@ -67,6 +67,9 @@ class GPUGraph:
     """Device-resident graph (vectors + fixed-degree adjacency) on the current GPU."""
 
     def __init__(self, vecs: np.ndarray, edges: np.ndarray):
+        self._open(vecs, edges, "bs_index_create")
+
+    def _open(self, vecs, edges, create):
         vecs = np.ascontiguousarray(vecs, dtype=np.float32)
         edges = np.ascontiguousarray(edges, dtype=np.uint32)
         if vecs.ndim != 2 or edges.ndim != 2 or vecs.shape[0] != edges.shape[0]:
@@ -76,8 +79,7 @@ class GPUGraph:
         self._vecs = vecs  # host rows, for the exact fallback of groundtruth()
         self.padded_dim = 0
         h = C.c_void_p()
-        _check(_lib.hip().bs_index_create(_ptr(vecs), _ptr(edges), self.n, self.dim, self.degree, C.byref(h)),
-               "bs_index_create")
+        _check(getattr(_lib.hip(), create)(_ptr(vecs), _ptr(edges), self.n, self.dim, self.degree, C.byref(h)), create)
         self._h = h
 
     def attach_rabitq(self, codes: np.ndarray, factors: np.ndarray, signs: np.ndarray):
@@ -322,6 +324,13 @@ def debug_mfma32(A, B):
     D = np.empty((32, 32), dtype=np.float32)
     _check(_lib.hip().bs_debug_mfma32(_ptr(A), _ptr(B), _ptr(D)), "bs_debug_mfma32")
     return D
+
+
+def debug_uncalibrated_graph(vecs, edges):
+    """a GPUGraph as a failed calibration of the query scheduling leaves it"""
+    g = GPUGraph.__new__(GPUGraph)
+    g._open(vecs, edges, "bs_debug_index_create_uncalibrated")
+    return g
 
 
 def debug_groundtruth(graph, queries, k, ws_limit):

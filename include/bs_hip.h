@@ -274,6 +274,11 @@ int bs_debug_label_order(const uint32_t* labels, const float* lcost, uint64_t n,
  * one chain of v_mfma_f32_32x32x2f32 instead, to compare the rounding with. */
 int bs_debug_gt_products(const float* rows, uint32_t n, const float* queries, uint32_t dim, int fp32, float* out);
 
+/* bs_index_create without the calibration of the query scheduling: the index that a failed
+ * calibration leaves. */
+int bs_debug_index_create_uncalibrated(const float* vecs, const uint32_t* edges, uint64_t n, uint32_t dim,
+                                       uint32_t degree, bs_index* out);
+
 /* bs_index_groundtruth with a work buffer of at most ws_limit bytes (a larger one counts as an
  * allocation that failed: fewer rows are held as operands at a time, BS_ENOMEM when the lists alone
  * do not fit). */

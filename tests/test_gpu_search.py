@@ -552,3 +552,25 @@ def test_beams_of_24_registers(gpu, topk, mode, degree):
     oids, od, _ = oi.search(q, 1000, omode, topk, 11, 900, 4096, 40)
     assert np.array_equal(ids, oids)
     assert d.tobytes() == od.tobytes()
+
+
+def test_index_is_complete_without_calibration(gpu):
+    """an index whose calibration failed has no device work pending when it is returned (a search on
+    another stream would read its pivots and order workspace), and searches by the plain label order"""
+    import torch
+    ds = dataset(4000, 128, 32, 64)
+    cfg = GPUBaseSearchCfg(64, 1024, ds["entry"], 1024, 16)
+    q = torch.from_numpy(ds["q"]).cuda()
+    ids = torch.empty(64, 10, dtype=torch.int32, device="cuda")
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    g = search.debug_uncalibrated_graph(ds["base"], ds["edges"])
+    assert torch.cuda.default_stream().query()
+    with pytest.raises(ValueError):
+        g.label_costs()
+    g.set_query_order(2)
+    g.search_device(q.data_ptr(), 64, ids.data_ptr(), 10, "base", cfg, stream=s.cuda_stream)
+    s.synchronize()
+    want = ds["g"].search(ds["q"], 10, "base", cfg)[0]
+    assert np.array_equal(ids.cpu().numpy().view(np.uint32), want)
+    g.close()
