@@ -170,6 +170,19 @@ def test_device_vamana_prune_sizes(gpu, n, dim, degree, beam, alpha):
     assert np.array_equal(search.build_vamana_device(base, degree, beam, alpha, 77), want)
 
 
+@pytest.mark.parametrize("n,dim,degree,beam,alpha", [(600, 130, 8, 24, 1.0), (600, 192, 8, 24, 2.0), (900, 333, 40, 150, 1.0),
+                                                     (700, 260, 64, 200, 1.5), (500, 960, 32, 128, 2.0)])
+def test_device_vamana_prune_long_rows(gpu, n, dim, degree, beam, alpha):
+    """rows too long for the registers: lanes stop reading once their candidate is dominated, in lists
+    of one block (whose distances serve both passes) and of several; repeated points, a hub"""
+    rng = np.random.default_rng(n + dim)
+    base = (rng.standard_normal((6, dim))[rng.integers(0, 6, n)] + 0.3 * rng.standard_normal((n, dim))).astype(np.float32)
+    base[3] = 0.0
+    base[10:14] = base[20]
+    want = host.build_vamana(base, degree, beam, alpha, 77, exact=True, threads=0)
+    assert np.array_equal(search.build_vamana_device(base, degree, beam, alpha, 77), want)
+
+
 def test_device_vamana_hub(gpu):
     """a point nearest to all others: its mirrored list passes what a wavefront sorts in LDS
     (1024 keys), so the lists of those batches are sorted in memory"""
