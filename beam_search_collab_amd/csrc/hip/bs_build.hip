@@ -803,19 +803,23 @@ extern "C" int bs_build_vamana_device(const float* vecs, uint64_t n, uint32_t di
     const uint64_t vis_words = (n + 31) / 32;
     const uint64_t slots = std::max<uint64_t>(1, std::min<uint64_t>(max_batch, (2ull << 30) / (vis_words * 4)));
 
-    DevBuf d_vecs, d_lid, d_ld, d_lcnt, d_order, d_vis, d_outk, d_outs, d_outn, d_rk, d_rks, d_heads, d_ctr, d_big, d_bigs,
-        d_bigjobs, d_beg, d_end, d_segb, d_sege, d_edges, d_tmp;
+    DevBuf d_vecs, d_lid, d_ld, d_lcnt, d_order, d_vis, d_outk, d_outn, d_rk, d_rks, d_heads, d_ctr, d_big, d_bigjobs, d_edges,
+        d_tmp;
+    // of the sorts in memory: the visit lists' (beams over 256) and the mirrored lists' (made when
+    // one first passes the LDS)
+    DevBuf d_outs, d_segb, d_sege, d_bigs, d_beg, d_end, d_bigtmp;
+    // visit lists short enough are sorted by the kernel that prunes them
+    const bool sort_here = outcap <= bvb::SORT_CAP;
     auto alloc = [&](DevBuf& b, size_t bytes) { return hipMalloc(&b.p, std::max<size_t>(bytes, 8)) == hipSuccess; };
     const uint64_t mrec = max_batch * degree;
     const uint64_t bigcap = mrec * (static_cast<uint64_t>(degree) + 1);
     if (!alloc(d_vecs, n * dstride * 4ull) || !alloc(d_lid, n * degree * 4ull) || !alloc(d_ld, n * degree * 4ull) ||
         !alloc(d_lcnt, n * 4ull) || !alloc(d_order, n * 4ull) || !alloc(d_vis, slots * vis_words * 4ull) ||
-        !alloc(d_outk, slots * outcap * 8ull) || !alloc(d_outs, slots * outcap * 8ull) || !alloc(d_outn, slots * 4ull) ||
+        !alloc(d_outk, slots * outcap * 8ull) || !alloc(d_outn, slots * 4ull) ||
         !alloc(d_rk, mrec * 8ull) || !alloc(d_rks, mrec * 8ull) || !alloc(d_heads, mrec * 16ull) ||
-        !alloc(d_ctr, sizeof(bvb::Counters)) || !alloc(d_big, bigcap * 8ull) || !alloc(d_bigs, bigcap * 8ull) ||
-        !alloc(d_bigjobs, mrec * 16ull) || !alloc(d_beg, mrec * 8ull) ||
-        !alloc(d_end, mrec * 8ull) || !alloc(d_segb, slots * 8ull) || !alloc(d_sege, slots * 8ull) ||
-        !alloc(d_edges, n * degree * 4ull))
+        !alloc(d_ctr, sizeof(bvb::Counters)) || !alloc(d_big, bigcap * 8ull) || !alloc(d_bigjobs, mrec * 16ull) ||
+        !alloc(d_edges, n * degree * 4ull) ||
+        (!sort_here && (!alloc(d_outs, slots * outcap * 8ull) || !alloc(d_segb, slots * 8ull) || !alloc(d_sege, slots * 8ull))))
         return vfail(BS_ENOMEM, "hipMalloc of the graph-construction buffers failed");
 
     hipError_t e = hipSuccess;
@@ -845,31 +849,25 @@ extern "C" int bs_build_vamana_device(const float* vecs, uint64_t n, uint32_t di
 
     if (slots * outcap > 0x7FFFFFFFull || bigcap > 0x7FFFFFFFull || mrec > 0xFFFFFFFFull)
         return vfail(BS_EINVAL, "batch too large for the device sorts (n or beam width too large)");
-    // hipCUB work space, sized for the largest of the three sorts
+    // hipCUB work space, sized for the larger of the two sorts
     size_t tmp_bytes = 0;
     {
-        size_t b1 = 0, b2 = 0, b3 = 0;
-        e = hipcub::DeviceSegmentedRadixSort::SortKeys(nullptr, b1, d_outk.as<uint64_t>(), d_outs.as<uint64_t>(),
-                                                   static_cast<int>(std::min<uint64_t>(slots * outcap, 0x7FFFFFFF)),
-                                                   static_cast<int>(slots), d_segb.as<uint64_t>(),
-                                                   d_sege.as<uint64_t>());
+        size_t b1 = 0, b2 = 0;
+        if (!sort_here)
+            e = hipcub::DeviceSegmentedRadixSort::SortKeys(nullptr, b1, d_outk.as<uint64_t>(), d_outs.as<uint64_t>(),
+                                                           static_cast<int>(slots * outcap), static_cast<int>(slots),
+                                                           d_segb.as<uint64_t>(), d_sege.as<uint64_t>());
         if (e == hipSuccess)
             e = hipcub::DeviceRadixSort::SortKeys(nullptr, b2, d_rk.as<uint64_t>(), d_rks.as<uint64_t>(),
                                                   static_cast<int>(mrec));
-        if (e == hipSuccess)
-            e = hipcub::DeviceSegmentedRadixSort::SortKeys(nullptr, b3, d_big.as<uint64_t>(), d_bigs.as<uint64_t>(),
-                                                   static_cast<int>(std::min<uint64_t>(bigcap, 0x7FFFFFFF)),
-                                                   static_cast<int>(mrec), d_beg.as<uint64_t>(),
-                                                   d_end.as<uint64_t>());
         if (e != hipSuccess) return vfail(BS_EHIP, std::string("sort sizing: ") + hipGetErrorString(e));
-        tmp_bytes = std::max({b1, b2, b3});
+        tmp_bytes = std::max(b1, b2);
         if (!alloc(d_tmp, tmp_bytes)) return vfail(BS_ENOMEM, "hipMalloc of the sort work space failed");
     }
+    size_t bigtmp_bytes = 0;
 
     uint64_t start = 1;
     double last_print = 0.0;
-    // visit lists short enough are sorted by the kernel that prunes them
-    const bool sort_here = outcap <= bvb::SORT_CAP;
     while (start < n) {
         const uint64_t end = std::min(std::min(start * 2, start + batch_bound), n);
         e = hipMemsetAsync(ctr, 0, sizeof(bvb::Counters), nullptr);
@@ -933,11 +931,21 @@ extern "C" int bs_build_vamana_device(const float* vecs, uint64_t n, uint32_t di
         if (e == hipSuccess && c.big) {
             const bool here = c.longest <= bvb::SORT_CAP;
             if (!here) {
+                if (!d_bigs.p) {
+                    e = hipcub::DeviceSegmentedRadixSort::SortKeys(nullptr, bigtmp_bytes, d_big.as<uint64_t>(),
+                                                                   d_bigs.as<uint64_t>(), static_cast<int>(bigcap),
+                                                                   static_cast<int>(mrec), d_beg.as<uint64_t>(),
+                                                                   d_end.as<uint64_t>());
+                    if (e != hipSuccess) break;
+                    if (!alloc(d_bigs, bigcap * 8ull) || !alloc(d_beg, mrec * 8ull) || !alloc(d_end, mrec * 8ull) ||
+                        !alloc(d_bigtmp, bigtmp_bytes))
+                        return vfail(BS_ENOMEM, "hipMalloc of the graph-construction buffers failed");
+                }
                 hipLaunchKernelGGL(bvb::vb_big_offsets, dim3((c.big + 255) / 256), dim3(256), 0, nullptr,
                                    d_bigjobs.as<uint4>(), c.big, d_beg.as<uint64_t>(), d_end.as<uint64_t>());
                 e = hipGetLastError();
                 if (e == hipSuccess)
-                    e = hipcub::DeviceSegmentedRadixSort::SortKeys(d_tmp.p, tmp_bytes, d_big.as<uint64_t>(),
+                    e = hipcub::DeviceSegmentedRadixSort::SortKeys(d_bigtmp.p, bigtmp_bytes, d_big.as<uint64_t>(),
                                                                    d_bigs.as<uint64_t>(), static_cast<int>(c.big_keys),
                                                                    static_cast<int>(c.big), d_beg.as<uint64_t>(),
                                                                    d_end.as<uint64_t>());
