@@ -775,11 +775,10 @@ struct DevBuf {
     }
 };
 
-}  // namespace
-
-extern "C" int bs_build_vamana_device(const float* vecs, uint64_t n, uint32_t dim, uint32_t degree,
-                                      uint32_t beam_width, float alpha, uint32_t seed, uint32_t* edges_out,
-                                      int verbose) try {
+// sort_cap: the most keys a list sorted in LDS may have, at most SORT_CAP; stats (may be null): the
+// longest mirrored list and the batches whose mirrored lists were sorted in memory
+int build_vamana(const float* vecs, uint64_t n, uint32_t dim, uint32_t degree, uint32_t beam_width, float alpha,
+                 uint32_t seed, uint32_t* edges_out, int verbose, uint32_t sort_cap, uint32_t* stats) {
     if (!vecs || !edges_out) return vfail(BS_EINVAL, "vecs and edges_out must be given");
     if (n == 0) return vfail(BS_EINVAL, "base dataset is empty");
     if (n > 0x7FFFFFFFull) return vfail(BS_EINVAL, "at most 2^31-1 points");
@@ -809,7 +808,7 @@ extern "C" int bs_build_vamana_device(const float* vecs, uint64_t n, uint32_t di
     // one first passes the LDS)
     DevBuf d_outs, d_segb, d_sege, d_bigs, d_beg, d_end, d_bigtmp;
     // visit lists short enough are sorted by the kernel that prunes them
-    const bool sort_here = outcap <= bvb::SORT_CAP;
+    const bool sort_here = outcap <= sort_cap;
     auto alloc = [&](DevBuf& b, size_t bytes) { return hipMalloc(&b.p, std::max<size_t>(bytes, 8)) == hipSuccess; };
     const uint64_t mrec = max_batch * degree;
     const uint64_t bigcap = mrec * (static_cast<uint64_t>(degree) + 1);
@@ -929,7 +928,11 @@ extern "C" int bs_build_vamana_device(const float* vecs, uint64_t n, uint32_t di
             e = hipGetLastError();
         }
         if (e == hipSuccess && c.big) {
-            const bool here = c.longest <= bvb::SORT_CAP;
+            const bool here = c.longest <= sort_cap;
+            if (stats) {
+                stats[0] = std::max(stats[0], c.longest);
+                stats[1] += here ? 0u : 1u;
+            }
             if (!here) {
                 if (!d_bigs.p) {
                     e = hipcub::DeviceSegmentedRadixSort::SortKeys(nullptr, bigtmp_bytes, d_big.as<uint64_t>(),
@@ -983,6 +986,24 @@ extern "C" int bs_build_vamana_device(const float* vecs, uint64_t n, uint32_t di
     if (e == hipSuccess) e = hipMemcpy(edges_out, d_edges.p, n * degree * 4ull, hipMemcpyDeviceToHost);
     if (e != hipSuccess) return vfail(BS_EHIP, std::string("graph construction: ") + hipGetErrorString(e));
     return BS_OK;
+}
+}  // namespace
+
+extern "C" int bs_build_vamana_device(const float* vecs, uint64_t n, uint32_t dim, uint32_t degree,
+                                      uint32_t beam_width, float alpha, uint32_t seed, uint32_t* edges_out,
+                                      int verbose) try {
+    return build_vamana(vecs, n, dim, degree, beam_width, alpha, seed, edges_out, verbose, bvb::SORT_CAP, nullptr);
+} catch (...) {
+    return bs_internal_exception();
+}
+
+extern "C" int bs_debug_build_vamana(const float* vecs, uint64_t n, uint32_t dim, uint32_t degree, uint32_t beam_width,
+                                     float alpha, uint32_t seed, uint32_t sort_cap, uint32_t* edges_out,
+                                     uint32_t* stats) try {
+    if (sort_cap < 64 || sort_cap > bvb::SORT_CAP) return vfail(BS_EINVAL, "sort_cap must be in 64..1024");
+    if (!stats) return vfail(BS_EINVAL, "stats must be given");
+    stats[0] = stats[1] = 0;
+    return build_vamana(vecs, n, dim, degree, beam_width, alpha, seed, edges_out, 0, sort_cap, stats);
 } catch (...) {
     return bs_internal_exception();
 }

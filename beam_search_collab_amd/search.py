@@ -326,6 +326,17 @@ def debug_mfma32(A, B):
     return D
 
 
+def debug_build_vamana(vecs, degree, beam_width, alpha, seed, sort_cap):
+    """build_vamana_device with lists of more than sort_cap keys sorted in memory: (edges, the longest
+    mirrored list, the batches whose mirrored lists were sorted in memory)"""
+    vecs = np.ascontiguousarray(vecs, dtype=np.float32)
+    out = np.empty((vecs.shape[0], degree), dtype=np.uint32)
+    stats = np.zeros(2, np.uint32)
+    _check(_lib.hip().bs_debug_build_vamana(_ptr(vecs), vecs.shape[0], vecs.shape[1], degree, beam_width, alpha, seed,
+                                            sort_cap, _ptr(out), _ptr(stats)), "bs_debug_build_vamana")
+    return out, int(stats[0]), int(stats[1])
+
+
 def debug_uncalibrated_graph(vecs, edges):
     """a GPUGraph as a failed calibration of the query scheduling leaves it"""
     g = GPUGraph.__new__(GPUGraph)

@@ -274,6 +274,12 @@ int bs_debug_label_order(const uint32_t* labels, const float* lcost, uint64_t n,
  * one chain of v_mfma_f32_32x32x2f32 instead, to compare the rounding with. */
 int bs_debug_gt_products(const float* rows, uint32_t n, const float* queries, uint32_t dim, int fp32, float* out);
 
+/* bs_build_vamana_device where a wavefront sorts lists of at most sort_cap keys (64..1024) in LDS, longer
+ * ones in memory (bs_build_vamana_device: 1024).  stats: the longest mirrored list that was pruned
+ * (0 if none passed 64 keys) and the number of batches whose mirrored lists were sorted in memory. */
+int bs_debug_build_vamana(const float* vecs, uint64_t n, uint32_t dim, uint32_t degree, uint32_t beam_width,
+                          float alpha, uint32_t seed, uint32_t sort_cap, uint32_t* edges_out, uint32_t stats[2]);
+
 /* bs_index_create without the calibration of the query scheduling: the index that a failed
  * calibration leaves. */
 int bs_debug_index_create_uncalibrated(const float* vecs, const uint32_t* edges, uint64_t n, uint32_t dim,

@@ -183,15 +183,33 @@ def test_device_vamana_prune_long_rows(gpu, n, dim, degree, beam, alpha):
     assert np.array_equal(search.build_vamana_device(base, degree, beam, alpha, 77), want)
 
 
-def test_device_vamana_hub(gpu):
-    """a point nearest to all others: its mirrored list passes what a wavefront sorts in LDS
-    (1024 keys), so the lists of those batches are sorted in memory"""
+@pytest.mark.parametrize("n,dim,degree,beam,cap", [(60000, 96, 4, 8, 1024), (56000, 40, 8, 16, 512)])
+def test_device_vamana_hub(gpu, n, dim, degree, beam, cap):
+    """a point nearest to all others: its mirrored list passes what a wavefront sorts in LDS (1024
+    keys, or the given cap), so the lists of those batches are sorted in memory"""
     rng = np.random.default_rng(9)
-    base = rng.standard_normal((56000, 40)).astype(np.float32)
+    base = rng.standard_normal((n, dim)).astype(np.float32)
     base /= np.linalg.norm(base, axis=1, keepdims=True)
     base[17] = 0.0
-    want = host.build_vamana(base, 8, 16, 1.2, 3, exact=True, threads=0)
-    assert np.array_equal(search.build_vamana_device(base, 8, 16, 1.2, 3), want)
+    want = host.build_vamana(base, degree, beam, 1.2, 3, exact=True, threads=0)
+    got, longest, in_memory = search.debug_build_vamana(base, degree, beam, 1.2, 3, cap)
+    assert longest > cap and in_memory >= 1, (longest, in_memory)
+    assert np.array_equal(got, want)
+    assert np.array_equal(search.build_vamana_device(base, degree, beam, 1.2, 3), want)
+
+
+@pytest.mark.parametrize("n,dim,degree,beam,alpha", [(700, 16, 64, 200, 2.0), (900, 47, 100, 150, 1.5), (1500, 200, 64, 256, 2.0),
+                                                     (1200, 17, 128, 128, 1.2), (800, 97, 64, 1024, 1.1)])
+def test_device_vamana_lists_sorted_in_memory(gpu, n, dim, degree, beam, alpha):
+    """every list over 64 keys sorted in memory, visit lists among them: the same graph"""
+    rng = np.random.default_rng(n + dim)
+    base = rng.standard_normal((n, dim)).astype(np.float32)
+    base[3] = 0.0
+    base[10:14] = base[20]
+    want = host.build_vamana(base, degree, beam, alpha, 77, exact=True, threads=0)
+    got, longest, in_memory = search.debug_build_vamana(base, degree, beam, alpha, 77, 64)
+    assert longest > 64 and in_memory >= 1, (longest, in_memory)
+    assert np.array_equal(got, want)
 
 
 @pytest.mark.parametrize("n,dim,degree", [(65, 17, 1), (300, 32, 3), (257, 33, 33), (130, 64, 64), (200, 96, 20),
