@@ -78,6 +78,7 @@ HIP_API = {
     "bs_debug_build_vamana": (C.c_int, [vp, u64, u32, u32, u32, f32, u32, u32, vp, vp]),
     "bs_debug_index_create_uncalibrated": (C.c_int, [vp, vp, u64, u32, u32, P(vp)]),
     "bs_debug_groundtruth": (C.c_int, [vp, vp, u64, u32, u64, vp, vp]),
+    "bs_debug_gt_plan": (C.c_int, [u64, u64, u32, vp]),
     "bs_debug_gt_products": (C.c_int, [vp, u32, vp, u32, C.c_int, vp]),
 }
 

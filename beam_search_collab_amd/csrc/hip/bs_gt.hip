@@ -48,6 +48,16 @@ constexpr uint32_t REFRESH = 16;      // tiles between two reads of the publishe
 
 constexpr uint32_t TS = 36;           // floats per lane of the values staged for an append (16-byte aligned)
 
+// the place in a split's list of the value it publishes, of G = min(splits, PUB) that do
+__host__ __device__ constexpr uint32_t pub_place(uint32_t nsplit) {
+    const uint32_t G = nsplit < PUB ? nsplit : PUB;
+    return (C + G - 1) / G;
+}
+// tiles of a split's priming pass (0: none)
+__host__ __device__ constexpr uint32_t prime_tiles(uint32_t nsplit, uint32_t tiles) {
+    return nsplit > 1 && pub_place(nsplit) <= 32u ? (tiles / 16u < 64u ? tiles / 16u : 64u) : 0u;
+}
+
 // LDS of a gt_select wavefront of QB x 32 queries: append buffers, 32 lanes' values, key counts
 constexpr uint32_t lds_wave(int qb) { return static_cast<uint32_t>(qb) * 32 * (BUF * 8 + 4) + 32 * TS * 4; }
 
@@ -290,7 +300,7 @@ gt_select(const uint4* frag, const float2* meta, uint64_t row0, uint64_t m, cons
     const uint32_t s = static_cast<uint32_t>(w / nqb);
     const uint32_t ntile = static_cast<uint32_t>((m + 31) / 32);
     const uint32_t t0 = s * split_tiles, t1 = std::min(ntile, t0 + split_tiles);
-    const uint32_t G = std::min(nsplit, PUB), mth = (C + G - 1) / G;
+    const uint32_t G = std::min(nsplit, PUB), mth = pub_place(nsplit);
 
     char* my = smem + static_cast<size_t>(wave) * lds_wave(QB);
     uint64_t* buf = reinterpret_cast<uint64_t*>(my);
@@ -534,7 +544,7 @@ gt_select(const uint4* frag, const float2* meta, uint64_t row0, uint64_t m, cons
     // smallest value of those rows, so it can be published as this split's mth value before any
     // list exists, and the lists then start at a threshold that admits about one row in 50
     // instead of every row.
-    const uint32_t prime = fresh && nsplit > 1 && mth <= 32u && t1 > t0 ? std::min(64u, (t1 - t0) / 16u) : 0u;
+    const uint32_t prime = fresh && t1 > t0 ? prime_tiles(nsplit, t1 - t0) : 0u;
     auto publish_minima = [&]() __attribute__((always_inline)) {
         float* st = reinterpret_cast<float*>(buf);  // no keys yet: NQ queries x TS floats
 #pragma unroll
@@ -1064,6 +1074,19 @@ extern "C" int bs_index_groundtruth_device(bs_index idx, const float* d_queries,
 extern "C" int bs_index_groundtruth(bs_index idx, const float* queries, uint64_t nq, uint32_t k, int32_t* out,
                                     uint8_t* uncertified, uint64_t* n_uncertified) try {
     return groundtruth_host(idx, queries, nq, k, out, uncertified, n_uncertified, ~0ull);
+} catch (...) {
+    return bs_internal_exception();
+}
+
+extern "C" int bs_debug_gt_plan(uint64_t n, uint64_t nq, uint32_t dim, uint32_t out[4]) try {
+    if (!out) return gfail(BS_EINVAL, "null argument");
+    if (n == 0 || n > 0x7FFFFFFFull || nq == 0 || dim == 0 || dim > 256) return gfail(BS_EINVAL, "n, nq or dim out of range");
+    const Plan p = make_plan(n, nq, dim, device_cus(), PLANE_BYTES);
+    out[0] = static_cast<uint32_t>(p.nsplit);
+    out[1] = static_cast<uint32_t>(p.split_tiles);
+    out[2] = bsg::prime_tiles(out[0], out[1]);
+    out[3] = p.KC <= 8 ? 2 : 1;
+    return BS_OK;
 } catch (...) {
     return bs_internal_exception();
 }

@@ -355,6 +355,13 @@ def debug_groundtruth(graph, queries, k, ws_limit):
     return out
 
 
+def debug_gt_plan(n, nq, dim):
+    """(row splits, tiles of 32 rows per split, tiles of the priming pass, query blocks per wavefront)"""
+    out = np.zeros(4, np.uint32)
+    _check(_lib.hip().bs_debug_gt_plan(n, nq, dim, _ptr(out)), "bs_debug_gt_plan")
+    return tuple(int(x) for x in out)
+
+
 def debug_gt_products(rows, queries, fp32=False):
     """q.b of 32 queries and n rows as the ground-truth candidates are selected by (bs_debug_gt_products)"""
     rows = np.ascontiguousarray(rows, dtype=np.float32)

@@ -66,8 +66,8 @@ def test_groundtruth_at_scale(gpu):
                                         (40000, 129, 128, 100), (30000, 31, 129, 10), (20001, 65, 192, 100),
                                         (50000, 1, 193, 128), (40003, 70, 256, 100)])
 def test_groundtruth_operand_sizes(gpu, n, nq, dim, k):
-    """the edges of the row tiles, query blocks, 16-dimension steps and operand instances; enough
-    rows per split to prime the thresholds in the larger ones"""
+    """the edges of the row tiles, query blocks, 16-dimension steps and operand instances (splits of
+    few tiles: no priming)"""
     base = host.gen_mixture(n, dim, 16, 0.0, 128.0, 12.0, 0.0, 21, 22)
     q = host.gen_mixture(nq, dim, 16, 0.0, 128.0, 12.0, 0.0, 21, 23)
     g = search.GPUGraph(base, np.zeros((n, 1), np.uint32))
@@ -257,3 +257,22 @@ def test_groundtruth_small_work_buffer(gpu, n, nq, dim):
     with pytest.raises(search.BeamSearchError):
         search.debug_groundtruth(g, q, 50, lists)
     assert np.array_equal(g.groundtruth(q, 50, exact_fallback=False), want)
+
+
+@pytest.mark.parametrize("n,nq,dim,primes", [(40000, 4160, 128, True), (100003, 2000, 100, True), (120000, 4001, 32, True),
+                                             (100000, 1000, 60, True), (60001, 4100, 200, True), (40000, 20000, 24, False)])
+def test_groundtruth_long_splits(gpu, n, nq, dim, primes):
+    """many query blocks, so few splits of many tiles: thresholds primed by the first tiles' minima
+    (with four splits and more) and refreshed from the other splits on the way, lists merged from all"""
+    nsplit, tiles, prime, qb = search.debug_gt_plan(n, nq, dim)
+    assert nsplit > 1 and (prime > 0) == primes and tiles > prime + 17, (nsplit, tiles, prime)  # refresh: from step 17
+    assert qb == (2 if dim <= 128 else 1)
+    base = host.gen_mixture(n, dim, 16, 0.0, 128.0, 12.0, 0.0, 91, 92)
+    q = host.gen_mixture(nq, dim, 16, 0.0, 128.0, 12.0, 0.0, 91, 93)
+    g = search.GPUGraph(base, np.zeros((n, 1), np.uint32))
+    raw = g.groundtruth(q, 100, exact_fallback=False)
+    cert = (raw != -2).all(1)
+    assert cert.mean() >= 0.95
+    at = np.unique(np.concatenate([np.random.default_rng(nq).integers(0, nq, 150), np.arange(20), np.arange(nq - 20, nq)]))
+    at = at[cert[at]]
+    assert np.array_equal(raw[at], host.groundtruth(base, q[at], 100))
