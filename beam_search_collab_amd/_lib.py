@@ -75,6 +75,7 @@ HIP_API = {
     "bs_index_groundtruth": (C.c_int, [vp, vp, u64, u32, vp, vp, P(u64)]),
     "bs_index_groundtruth_device": (C.c_int, [vp, vp, u64, u32, vp, vp, vp, P(u64)]),
     "bs_debug_mfma32": (C.c_int, [vp, vp, vp]),
+    "bs_debug_mfma32_f16": (C.c_int, [vp, vp, vp]),
     "bs_debug_build_vamana": (C.c_int, [vp, u64, u32, u32, u32, f32, u32, u32, vp, vp]),
     "bs_debug_index_create_uncalibrated": (C.c_int, [vp, vp, u64, u32, u32, P(vp)]),
     "bs_debug_groundtruth": (C.c_int, [vp, vp, u64, u32, u64, vp, vp]),

@@ -163,7 +163,7 @@ __global__ void __launch_bounds__(256) gt_split(const float* vecs, uint64_t row0
 
 // D (32 x 32) element of accumulator register r in this lane: row (query) 8(r/4) + 4(lane/32)
 // + r%4, column (base row) lane % 32 -- the 32 x 32 output layout of the f32 and f16
-// instructions alike, checked by bs_debug_mfma32.
+// instructions alike, checked by bs_debug_mfma32_f16 and bs_debug_mfma32.
 __device__ __forceinline__ uint32_t acc_row(int r, uint32_t half) {
     return 8u * static_cast<uint32_t>(r / 4) + 4u * half + static_cast<uint32_t>(r % 4);
 }
@@ -852,6 +852,22 @@ __global__ void __launch_bounds__(64) dbg_mfma32(const float* A, const float* B,
     for (int r = 0; r < 16; ++r) D[acc_row(r, half) * 32 + l32] = acc[r];
 }
 
+// the same for v_mfma_f32_32x32x16_f16 with the operand rule of gt_split and load_queries: A 32x16,
+// B 16x32
+__global__ void __launch_bounds__(64) dbg_mfma32_f16(const float* A, const float* B, float* D) {
+    const uint32_t lane = lane_id(), half = lane >> 5, l32 = lane & 31u;
+    f16x8 a, b;
+#pragma unroll
+    for (uint32_t i = 0; i < 8; ++i) {
+        a[i] = static_cast<_Float16>(A[l32 * 16 + 8 * half + i]);
+        b[i] = static_cast<_Float16>(B[(8 * half + i) * 32 + l32]);
+    }
+    f32x16 acc = {};
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, acc, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) D[acc_row(r, half) * 32 + l32] = acc[r];
+}
+
 }  // namespace bsg
 
 namespace {
@@ -1142,28 +1158,42 @@ extern "C" int bs_debug_gt_products(const float* rows, uint32_t n, const float* 
     return bs_internal_exception();
 }
 
-extern "C" int bs_debug_mfma32(const float* A, const float* B, float* D) try {
+namespace {
+// one 32 x 32 product, K values per row of A and column of B
+int mfma_check(void (*kernel)(const float*, const float*, float*), uint32_t K, const float* A, const float* B, float* D) {
     float *dA = nullptr, *dB = nullptr, *dD = nullptr;
     auto release = [&]() {
         if (dA) (void)hipFree(dA);
         if (dB) (void)hipFree(dB);
         if (dD) (void)hipFree(dD);
     };
-    if (hipMalloc(&dA, 64 * 4) != hipSuccess || hipMalloc(&dB, 64 * 4) != hipSuccess ||
-        hipMalloc(&dD, 1024 * 4) != hipSuccess) {
+    const size_t bytes = 32ull * K * 4;
+    if (hipMalloc(&dA, bytes) != hipSuccess || hipMalloc(&dB, bytes) != hipSuccess || hipMalloc(&dD, 1024 * 4) != hipSuccess) {
         release();
         return gfail(BS_ENOMEM, "hipMalloc failed");
     }
-    hipError_t e = hipMemcpy(dA, A, 64 * 4, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(dB, B, 64 * 4, hipMemcpyHostToDevice);
+    hipError_t e = hipMemcpy(dA, A, bytes, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(dB, B, bytes, hipMemcpyHostToDevice);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(bsg::dbg_mfma32, dim3(1), dim3(64), 0, nullptr, dA, dB, dD);
+        hipLaunchKernelGGL(kernel, dim3(1), dim3(64), 0, nullptr, dA, dB, dD);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpy(D, dD, 1024 * 4, hipMemcpyDeviceToHost);
     release();
     if (e != hipSuccess) return gfail(BS_EHIP, std::string("mfma check: ") + hipGetErrorString(e));
     return BS_OK;
+}
+}  // namespace
+
+extern "C" int bs_debug_mfma32(const float* A, const float* B, float* D) try {
+    return mfma_check(bsg::dbg_mfma32, 2, A, B, D);
+} catch (...) {
+    return bs_internal_exception();
+}
+
+extern "C" int bs_debug_mfma32_f16(const float* A, const float* B, float* D) try {
+    if (!A || !B || !D) return gfail(BS_EINVAL, "null argument");
+    return mfma_check(bsg::dbg_mfma32_f16, 16, A, B, D);
 } catch (...) {
     return bs_internal_exception();
 }

@@ -326,6 +326,14 @@ def debug_mfma32(A, B):
     return D
 
 
+def debug_mfma32_f16(A, B):
+    A = np.ascontiguousarray(A, dtype=np.float32).reshape(32, 16)
+    B = np.ascontiguousarray(B, dtype=np.float32).reshape(16, 32)
+    D = np.empty((32, 32), dtype=np.float32)
+    _check(_lib.hip().bs_debug_mfma32_f16(_ptr(A), _ptr(B), _ptr(D)), "bs_debug_mfma32_f16")
+    return D
+
+
 def debug_build_vamana(vecs, degree, beam_width, alpha, seed, sort_cap):
     """build_vamana_device with lists of more than sort_cap keys sorted in memory: (edges, the longest
     mirrored list, the batches whose mirrored lists were sorted in memory)"""

@@ -296,8 +296,12 @@ int bs_debug_groundtruth(bs_index idx, const float* queries, uint64_t nq, uint32
                          int32_t* out, uint8_t* uncertified);
 
 /* One v_mfma_f32_32x32x2f32 product: A 32x2 and B 2x32 row-major in, D = A B 32x32
- * row-major out, read back through the accumulator layout the ground-truth kernel uses. */
+ * row-major out, read back through the 32x32 accumulator layout. */
 int bs_debug_mfma32(const float* A, const float* B, float* D);
+
+/* One v_mfma_f32_32x32x16_f16 product: A 32x16 and B 16x32 row-major in (rounded to fp16), D 32x32
+ * out, through the operand and accumulator layouts the ground-truth kernel uses. */
+int bs_debug_mfma32_f16(const float* A, const float* B, float* D);
 
 /* Visit filters: nbatch lane-parallel batches of bsize (<= 64) inserts (0xFFFFFFFF =
  * idle lane), then nquery contains().  bloom = 0: HashFilter (filter_hash.cuh),

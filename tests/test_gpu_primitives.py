@@ -175,10 +175,19 @@ def test_host_tools_do_not_need_the_gpu_but_index_does(gpu):
 
 
 def test_mfma32_layout(gpu):
-    """the accumulator layout the ground-truth kernel reads back (row 8(r/4)+4(lane/32)+r%4,
-    column lane%32 for register r) gives D = A B for one v_mfma_f32_32x32x2f32"""
+    """the 32x32 accumulator layout (row 8(r/4)+4(lane/32)+r%4, column lane%32 for register r)
+    gives D = A B for one v_mfma_f32_32x32x2f32"""
     rng = np.random.default_rng(3)
     A = rng.integers(-8, 8, (32, 2)).astype(np.float32)
     B = rng.integers(-8, 8, (2, 32)).astype(np.float32)
     D = search.debug_mfma32(A, B)
     assert np.array_equal(D, A @ B)
+
+
+def test_mfma32_f16_layout(gpu):
+    """the operand and accumulator layouts of the ground-truth kernel give D = A B for one
+    v_mfma_f32_32x32x16_f16 (small whole numbers: exact in fp16 and in the sums)"""
+    rng = np.random.default_rng(4)
+    A = rng.integers(-8, 8, (32, 16)).astype(np.float32)
+    B = rng.integers(-8, 8, (16, 32)).astype(np.float32)
+    assert np.array_equal(search.debug_mfma32_f16(A, B), A @ B)
