@@ -478,6 +478,13 @@ int make_plan(bs_index ix, const bs_search_cfg* cfg, uint64_t nq, Plan& pl) {
     // them all (32 registers took 100k x 75, 777 queries, topk 1500 9.73 ms against 8.36; 50k x
     // 64 bwarp1, 2000 queries, topk 1100 4.80 against 3.94; 100k x 128, 10k queries, topk 1100 58.4
     // against 51.3).
+    // The steps between the powers of two above 1024 keys end there.  RaBitQ beams of that size stay at
+    // 32, since their final sort takes a power of two of keys (bsd::sort_beam): padded to one in
+    // 16 KB of LDS, 24 registers measured 8.75 -> 7.81 ms (100k x 128, 2000 queries, topk 1100) and
+    // 11.29 -> 10.00 (1536).  Base beams of 1537..1792 keys with 28 registers measured 9.93 -> 9.41 ms
+    // and 12.11 -> 11.10 (100k x 75, 777 queries, topk 1600 and 1792), of 2049..3072 with 48 27.6 -> 20.2
+    // and 45.7 -> 32.8 (topk 2100 and 3072).  None of the three is built: each is a set of instances
+    // of its own (9 per filter, 3 or 6 for RaBitQ), not yet tested over degrees and filters.
     // RaBitQ beams of 513..640 and 641..768 keys get 10 and 12 registers (the recall@10 0.95
     // point of config C is topk 640: 1M x 128, 10k queries, 6.31 ms with 12 registers)
     pl.TR = T <= 64 ? 1 : T <= 128 ? 2 : T <= 256 ? 4 : T <= 512 ? 8
