@@ -51,6 +51,10 @@ int check_device() {
 
 }  // namespace
 
+// staging of the large copies to the host: threads, slots of each and bytes of a slot
+constexpr uint32_t COPY_T = 4, COPY_SLOTS = 3;
+constexpr size_t COPY_SLOT = 2u << 20;
+
 struct bs_index_s {
     int device = 0;
     uint64_t n = 0;
@@ -75,9 +79,10 @@ struct bs_index_s {
     hipEvent_t ws_free = nullptr;
     // expected cost per label for the base-family label order (calibrate_labels), or null
     float* d_lcost = nullptr;
-    // streams of the large copies to the host (download), made by the first of them; one copy of
-    // an index uses them at a time
-    hipStream_t copy[4] = {nullptr, nullptr, nullptr, nullptr};
+    // pinned staging of the large copies to the host (download), made by the first of them; one copy
+    // of an index uses it at a time
+    char* pin = nullptr;
+    hipEvent_t pin_done[COPY_T * COPY_SLOTS] = {};
     std::mutex copy_mutex;
     // device staging of bs_search (host buffers): grows to the largest call, reused after
     void* d_stage = nullptr;
@@ -93,44 +98,69 @@ constexpr uint32_t LDS_GRANULE = 512;
 
 // A copy from the device to pageable host memory.  One such copy runs at the speed of the
 // runtime's single thread through its pinned staging (17 GB/s, 10 into memory touched for the
-// first time); four threads on streams of their own reach 46 and 30 (200 MB).  Synchronous; the
-// null stream's earlier work is waited for first.  Smaller copies, and any case where streams
-// cannot be made, take the one copy.  (Uploads gain nothing: 28 GB/s by one copy, and a new
-// index's streams start slower: opening 200k x 128 16.2 -> 20.8 ms.)
+// first time); COPY_T threads that each take a part through slots of pinned memory of their own, the
+// next slots filled while one is copied out, take a codebook of 200k x 128 (179 MB to the host) from
+// 20.7 to 8.6 ms, 12 the first time (1 or 4 MB slots 9.5 and 8.8, 8 threads 8.4).  All on the null
+// stream: a stream of the library's own would be one more hardware queue of the process, and with a
+// second queue every synchronous call takes 8 us longer for good (a search of 3 queries from host
+// buffers 142 -> 151 us), also after the stream is destroyed.  (Four threads on streams of their
+// own: 11.5 ms, 20 the first time.)  Synchronous.  Smaller copies, and any case where the staging
+// cannot be made, take the one copy.  (Uploads gain nothing: 28 GB/s by one copy.)
 hipError_t download(bs_index ix, void* dst, const void* src, size_t bytes) {
-    constexpr int T = 4;
     const hipMemcpyKind kind = hipMemcpyDeviceToHost;
     if (bytes < (16u << 20)) return hipMemcpy(dst, src, bytes, kind);
     const std::lock_guard<std::mutex> lock(ix->copy_mutex);  // callers on several threads
-    for (hipStream_t& s : ix->copy)
-        if (!s && hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) {
-            s = nullptr;
+    if (!ix->pin) {
+        hipError_t e = hipSuccess;
+        for (hipEvent_t& v : ix->pin_done)
+            if (e == hipSuccess && !v) e = hipEventCreateWithFlags(&v, hipEventDisableTiming);
+        if (e == hipSuccess)
+            e = hipHostMalloc(reinterpret_cast<void**>(&ix->pin), COPY_T * COPY_SLOTS * COPY_SLOT, hipHostMallocDefault);
+        if (e != hipSuccess) {
+            ix->pin = nullptr;
             (void)hipGetLastError();
             return hipMemcpy(dst, src, bytes, kind);
         }
-    hipError_t e = hipStreamSynchronize(nullptr);
-    if (e != hipSuccess) return e;
-    hipError_t err[T] = {hipSuccess, hipSuccess, hipSuccess, hipSuccess};
-    auto piece = [&](int t, bool own_thread) {
-        const size_t a = bytes * t / T & ~static_cast<size_t>(4095);
-        const size_t b = t + 1 == T ? bytes : bytes * (t + 1) / T & ~static_cast<size_t>(4095);
-        hipError_t r = own_thread ? hipSetDevice(ix->device) : hipSuccess;
-        if (r == hipSuccess)
-            r = hipMemcpyWithStream(static_cast<char*>(dst) + a, static_cast<const char*>(src) + a, b - a, kind, ix->copy[t]);
-        err[t] = r;
+    }
+    hipError_t err[COPY_T];
+    auto part = [&](uint32_t t, bool own_thread) {
+        const size_t a = bytes * t / COPY_T & ~static_cast<size_t>(4095);
+        const size_t b = t + 1 == COPY_T ? bytes : bytes * (t + 1) / COPY_T & ~static_cast<size_t>(4095);
+        char* slots = ix->pin + t * COPY_SLOTS * COPY_SLOT;
+        hipEvent_t* done = ix->pin_done + t * COPY_SLOTS;
+        const size_t pieces = (b - a + COPY_SLOT - 1) / COPY_SLOT;
+        auto size_of = [&](size_t i) { return std::min(COPY_SLOT, b - a - i * COPY_SLOT); };
+        hipError_t e = own_thread ? hipSetDevice(ix->device) : hipSuccess;
+        auto fetch = [&](size_t i) {
+            if (e == hipSuccess)
+                e = hipMemcpyAsync(slots + i % COPY_SLOTS * COPY_SLOT, static_cast<const char*>(src) + a + i * COPY_SLOT,
+                                   size_of(i), kind, nullptr);
+            if (e == hipSuccess) e = hipEventRecord(done[i % COPY_SLOTS], nullptr);
+        };
+        for (size_t i = 0; i < std::min<size_t>(COPY_SLOTS, pieces); ++i) fetch(i);
+        for (size_t i = 0; e == hipSuccess && i < pieces; ++i) {
+            e = hipEventSynchronize(done[i % COPY_SLOTS]);
+            if (e != hipSuccess) break;
+            std::memcpy(static_cast<char*>(dst) + a + i * COPY_SLOT, slots + i % COPY_SLOTS * COPY_SLOT, size_of(i));
+            if (i + COPY_SLOTS < pieces) fetch(i + COPY_SLOTS);
+        }
+        err[t] = e;
     };
-    std::thread th[T];
-    int started = 1;
+    std::thread th[COPY_T];
+    uint32_t started = 1;
     try {
-        for (; started < T; ++started) th[started] = std::thread(piece, started, true);
+        for (; started < COPY_T; ++started) th[started] = std::thread(part, started, true);
     } catch (...) {  // no thread to be had: this one copies the rest
     }
-    piece(0, false);
-    for (int t = started; t < T; ++t) piece(t, false);
+    part(0, false);
+    for (uint32_t t = started; t < COPY_T; ++t) part(t, false);
     for (std::thread& x : th)
         if (x.joinable()) x.join();
-    for (int t = 0; t < T; ++t)
-        if (err[t] != hipSuccess) return err[t];
+    for (hipError_t e : err)
+        if (e != hipSuccess) {
+            (void)hipStreamSynchronize(nullptr);  // nothing may still write to the staging
+            return e;
+        }
     return hipSuccess;
 }
 
@@ -419,8 +449,9 @@ extern "C" void bs_index_destroy(bs_index ix) {
     if (ix->d_ows) (void)hipFree(ix->d_ows);
     if (ix->d_lcost) (void)hipFree(ix->d_lcost);
     if (ix->d_stage) (void)hipFree(ix->d_stage);
-    for (hipStream_t s : ix->copy)
-        if (s) (void)hipStreamDestroy(s);
+    for (hipEvent_t v : ix->pin_done)
+        if (v) (void)hipEventDestroy(v);
+    if (ix->pin) (void)hipHostFree(ix->pin);
     delete ix;
 }
 

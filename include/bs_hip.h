@@ -177,7 +177,8 @@ int bs_index_entry_point(bs_index idx, uint32_t* entry);
  * outputs: codes n*degree*(pdim/32) u32, factors n*3*degree f32, signs pdim f32, entry.
  * The factor products the reference forms in long double are made on the device in integers
  * with the same roundings (edges of infinite or NaN vectors: on the host, in long double).
- * Synchronous; allocates work buffers (rotations n*pdim f32, codes, 12 B per edge).  dim > 16. */
+ * Synchronous; allocates work buffers (rotations n*pdim f32, codes, 12 B per edge) and, where codes or
+ * factors pass 16 MB, 24 MB of pinned host memory that the index keeps.  dim > 16. */
 int bs_index_build_rabitq(bs_index idx, uint32_t seed, uint32_t* codes, float* factors, float* signs,
                           uint32_t* entry);
 

@@ -29,6 +29,14 @@ def test_exports(header, path):
     assert set(names) == set(api), set(names) ^ set(api)
 
 
+def test_library_creates_no_stream():
+    """every stream is one more hardware queue of the process, and a second queue makes each
+    synchronous call of the program slower for good: the library works on the caller's streams"""
+    import subprocess
+    out = subprocess.run(["nm", "-D", "--undefined-only", _lib.HIP_LIB_PATH], capture_output=True, text=True, check=True).stdout
+    assert "hipMemcpy" in out and "hipStreamCreate" not in out
+
+
 def test_oracle_is_not_linked_by_the_product():
     import subprocess
     for path in (_lib.HIP_LIB_PATH, _lib.HOST_LIB_PATH):

@@ -248,8 +248,8 @@ def test_device_codebook_infinite_rows(gpu):
 
 
 def test_codebook_from_two_threads(gpu):
-    """two threads ask one index for its codebook (20 MB of codes: the copies to the host go by
-    several streams, made by whichever comes first): each gets the result of a single call"""
+    """two threads ask one index for its codebook (20 MB of codes: the copies to the host go through
+    the index's pinned staging, made by whichever comes first): each gets the result of a single call"""
     from concurrent.futures import ThreadPoolExecutor
     n, dim, degree = 40_000, 100, 32
     base = host.gen_mixture(n, dim, 8, 0.0, 128.0, 12.0, 0.0, 3, 4)
@@ -265,3 +265,20 @@ def test_codebook_from_two_threads(gpu):
                 assert x.tobytes() == y.tobytes()
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("n,dim,degree", [(70001, 40, 33), (52429, 100, 20), (140007, 33, 17)])
+def test_codebook_downloads_in_pieces(gpu, n, dim, degree):
+    """codes and factors over 16 MB come to the host in pieces by several threads: sizes that end
+    inside a page and inside a piece, a few pieces per thread and more than its slots"""
+    rng = np.random.default_rng(n)
+    base = rng.standard_normal((n, dim)).astype(np.float32)
+    edges = rng.integers(0, n, (n, degree)).astype(np.uint32)
+    g = search.GPUGraph(base, edges)
+    want = host.build_rabitq(base, edges, 7)
+    for _ in range(2):
+        got = g.build_rabitq(7)
+        assert got[0] == want[0]
+        for a, b in zip(got[1:], want[1:]):
+            assert a.tobytes() == b.tobytes()
+    g.close()
