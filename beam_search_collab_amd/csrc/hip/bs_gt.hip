@@ -264,8 +264,9 @@ __device__ __forceinline__ void load_queries(const float* queries, uint32_t dim,
 // Against fp64 the rms error of q.b is 0.36-0.56 of the fp32 instructions' over mixture and
 // unit-sphere data of 16..256 dimensions and 0.12-0.79 over wide-ranged data of 32 and more and
 // values that differ in their last 12 bits, because the chain rounds 8 times less often; where one or
-// two products are most of the sum and both round once, 1.0-1.27 (the matrix unit's rounding).  Two planes and three products
-// hold 22 to 24 of the 24 bits: 1.9-2.9 there and up to 1.27 on wide-ranged data.
+// two products are most of the sum and both round once, 1.0-1.27 (the matrix unit's rounding).
+// Two planes and three products hold 22 to 24 of the 24 bits: 1.9-2.9 there and up to 1.27 on
+// wide-ranged data.
 // Six fp16 products of 16 dimensions take 192 matrix cycles, eight v_mfma_f32_32x32x2f32 512.
 // 500k x 128, 10k queries: 17.1 -> 8.7 ms with the filtering below.
 // Two query blocks per wavefront (dim <= 128) halve the base bytes per product.
