@@ -53,7 +53,8 @@ __host__ __device__ constexpr uint32_t pub_place(uint32_t nsplit) {
     const uint32_t G = nsplit < PUB ? nsplit : PUB;
     return (C + G - 1) / G;
 }
-// tiles of a split's priming pass (0: none)
+// tiles of a split's priming pass (0: none), the same for all splits: one that publishes later holds
+// the others up
 __host__ __device__ constexpr uint32_t prime_tiles(uint32_t nsplit, uint32_t tiles) {
     return nsplit > 1 && pub_place(nsplit) <= 32u ? (tiles / 16u < 64u ? tiles / 16u : 64u) : 0u;
 }
@@ -287,7 +288,7 @@ __device__ __forceinline__ void load_queries(const float* queries, uint32_t dim,
 template <int KC, int QB>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 gt_select(const uint4* frag, const float2* meta, uint64_t row0, uint64_t m, const float* queries, uint32_t dim,
-          uint64_t nq, uint32_t nsplit, uint32_t split_tiles, uint32_t fresh, uint64_t* topc, uint32_t* tshare,
+          uint64_t nq, uint32_t nsplit, uint32_t prime, uint32_t fresh, uint64_t* topc, uint32_t* tshare,
           uint32_t* pub) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const uint32_t lane = lane_id(), wave = bsw::uniform(threadIdx.x >> 6), half = lane >> 5, l32 = lane & 31u;
@@ -300,7 +301,10 @@ gt_select(const uint4* frag, const float2* meta, uint64_t row0, uint64_t m, cons
     const uint64_t qb = w % nqb;
     const uint32_t s = static_cast<uint32_t>(w / nqb);
     const uint32_t ntile = static_cast<uint32_t>((m + 31) / 32);
-    const uint32_t t0 = s * split_tiles, t1 = std::min(ntile, t0 + split_tiles);
+    // the splits share the tiles evenly: with equal shares rounded up the last ones can come out
+    // empty, and a split that publishes nothing leaves the shared bound below (G values) without effect
+    const uint32_t t0 = static_cast<uint32_t>(static_cast<uint64_t>(s) * ntile / nsplit);
+    const uint32_t t1 = static_cast<uint32_t>((static_cast<uint64_t>(s) + 1) * ntile / nsplit);
     const uint32_t G = std::min(nsplit, PUB), mth = pub_place(nsplit);
 
     char* my = smem + static_cast<size_t>(wave) * lds_wave(QB);
@@ -324,7 +328,8 @@ gt_select(const uint4* frag, const float2* meta, uint64_t row0, uint64_t m, cons
     // tau: per accumulator register, the threshold of its query (a float compare passes a
     // superset of the list's key order; none passes for a query past nq).  Lane i's tq is query
     // i's.
-    float tq = qb * NQ + lane < nq && lane < NQ ? __builtin_inff() : -__builtin_inff();
+    const uint64_t nan2 = (static_cast<uint64_t>(nanq[QB - 1]) << 32) | nanq[0];
+    float tq = qb * NQ + lane < nq && lane < NQ && !bsw::lane_in(nan2) ? __builtin_inff() : -__builtin_inff();
     float tau[QB][16];
     // the bits of `bits` (below) whose query exists and has no NaN: a query with one has no
     // neighbours, and every row would survive for it
@@ -545,7 +550,6 @@ gt_select(const uint4* frag, const float2* meta, uint64_t row0, uint64_t m, cons
     // smallest value of those rows, so it can be published as this split's mth value before any
     // list exists, and the lists then start at a threshold that admits about one row in 50
     // instead of every row.
-    const uint32_t prime = fresh && t1 > t0 ? prime_tiles(nsplit, t1 - t0) : 0u;
     auto publish_minima = [&]() __attribute__((always_inline)) {
         float* st = reinterpret_cast<float*>(buf);  // no keys yet: NQ queries x TS floats
 #pragma unroll
@@ -581,9 +585,10 @@ gt_select(const uint4* frag, const float2* meta, uint64_t row0, uint64_t m, cons
             __hip_atomic_store(&pub[static_cast<uint64_t>(s) * nq + qb * NQ + lane], static_cast<uint32_t>(orderable(v)),
                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         // the other splits reach this point at about the same time: read until all have
-        // published, at most 32 times (about 30 us; a split that is not resident yet never will)
+        // published, at most 32 times (a read is 8 us for 64 splits; a split that is not resident yet
+        // never will).  Measured: one read and 20 us with every split resident.
         for (int i = 0; i < 32; ++i)
-            if (ballot(!refresh()) == 0) break;
+            if (ballot(!refresh() && tq != -__builtin_inff()) == 0) break;
         spread_tau();
     };
     if (t0 < t1) {
@@ -885,13 +890,13 @@ int gfail(int code, const std::string& msg) {
 // one workgroup of the select: KC steps of 16 dimensions, QB query blocks of 32 per wavefront
 template <int KC, int QB>
 hipError_t launch_select(dim3 g, hipStream_t s, const uint4* frag, const float2* meta, uint64_t row0, uint64_t m,
-                         const float* q, uint32_t dim, uint64_t nq, uint32_t nsplit, uint32_t split_tiles,
+                         const float* q, uint32_t dim, uint64_t nq, uint32_t nsplit, uint32_t prime,
                          uint64_t* topc, uint32_t* tshare, uint32_t* pub) {
     constexpr int lds = 4 * bsg::lds_wave(QB);
     auto k = bsg::gt_select<KC, QB>;
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k, g, dim3(256), lds, s, frag, meta, row0, m, q, dim, nq, nsplit, split_tiles,
+    hipLaunchKernelGGL(k, g, dim3(256), lds, s, frag, meta, row0, m, q, dim, nq, nsplit, prime,
                        row0 == 0 ? 1u : 0u, topc, tshare, pub);
     return hipGetLastError();
 }
@@ -940,7 +945,8 @@ uint64_t pick_splits(uint64_t nqb, uint64_t tiles, uint64_t slots) {
 struct Plan {
     uint32_t KC;   // 16-dimension steps
     uint64_t nqb;  // query blocks: 64 queries per wavefront while their operands fit beside a tile's, else 32
-    uint64_t tiles, chunk, nsplit, split_tiles;  // tiles of the base, held as planes at a time, per split
+    uint64_t tiles, chunk, nsplit;  // tiles of the base, held as planes at a time; row splits
+    uint32_t split_tiles, prime;    // tiles of the smallest split (the others have one more at most), primed ones
     uint64_t tile_bytes, o_bn, o_top, o_share, o_pub, o_cnt, need;
 };
 Plan make_plan(uint64_t n, uint64_t nq, uint32_t dim, uint32_t cus, uint64_t plane_bytes) {
@@ -953,7 +959,8 @@ Plan make_plan(uint64_t n, uint64_t nq, uint32_t dim, uint32_t cus, uint64_t pla
     p.tiles = (n + 31) / 32;
     p.chunk = std::max<uint64_t>(1, std::min<uint64_t>(p.tiles, plane_bytes / p.tile_bytes));
     p.nsplit = pick_splits(p.nqb, p.chunk, 4ull * cus);
-    p.split_tiles = (p.chunk + p.nsplit - 1) / p.nsplit;
+    p.split_tiles = static_cast<uint32_t>(p.chunk / p.nsplit);
+    p.prime = bsg::prime_tiles(static_cast<uint32_t>(p.nsplit), p.split_tiles);
     p.o_bn = al(p.chunk * p.tile_bytes);
     p.o_top = p.o_bn + al(p.chunk * 32 * 8);
     p.o_share = p.o_top + al(nq * p.nsplit * bsg::C * 8);
@@ -1018,7 +1025,7 @@ int groundtruth(bs_index idx, const float* d_queries, uint64_t nq, uint32_t k, i
             if (le != hipSuccess) return le;
             return launch_select<K, decltype(qb)::value>(g, s, frag, meta, row0, m, d_queries, dim, nq,
                                                          static_cast<uint32_t>(p.nsplit),
-                                                         static_cast<uint32_t>(p.split_tiles), topc, tshare, pub);
+                                                         row0 == 0 ? p.prime : 0u, topc, tshare, pub);
         };
         e = with_steps(p.KC, go);
     }
@@ -1103,8 +1110,8 @@ extern "C" int bs_debug_gt_plan(uint64_t n, uint64_t nq, uint32_t dim, uint32_t 
     if (n == 0 || n > 0x7FFFFFFFull || nq == 0 || dim == 0 || dim > 256) return gfail(BS_EINVAL, "n, nq or dim out of range");
     const Plan p = make_plan(n, nq, dim, device_cus(), PLANE_BYTES);
     out[0] = static_cast<uint32_t>(p.nsplit);
-    out[1] = static_cast<uint32_t>(p.split_tiles);
-    out[2] = bsg::prime_tiles(out[0], out[1]);
+    out[1] = p.split_tiles;
+    out[2] = p.prime;
     out[3] = p.KC <= 8 ? 2 : 1;
     return BS_OK;
 } catch (...) {

@@ -364,7 +364,7 @@ def debug_groundtruth(graph, queries, k, ws_limit):
 
 
 def debug_gt_plan(n, nq, dim):
-    """(row splits, tiles of 32 rows per split, tiles of the priming pass, query blocks per wavefront)"""
+    """(row splits, tiles of 32 rows in the smallest, tiles of the priming pass, query blocks per wavefront)"""
     out = np.zeros(4, np.uint32)
     _check(_lib.hip().bs_debug_gt_plan(n, nq, dim, _ptr(out)), "bs_debug_gt_plan")
     return tuple(int(x) for x in out)

@@ -270,8 +270,8 @@ int bs_debug_cost_order(const float* signal, uint64_t n, uint32_t* qmap, uint32_
 int bs_debug_label_order(const uint32_t* labels, const float* lcost, uint64_t n, uint32_t g, uint32_t X,
                          uint32_t* qmap);
 
-/* How bs_index_groundtruth cuts a call up: out = {row splits, tiles of 32 rows per split, tiles of a
- * split's priming pass, query blocks of 32 per wavefront}. */
+/* How bs_index_groundtruth cuts a call up: out = {row splits, tiles of 32 rows in the smallest split,
+ * tiles of a split's priming pass, query blocks of 32 per wavefront}. */
 int bs_debug_gt_plan(uint64_t n, uint64_t nq, uint32_t dim, uint32_t out[4]);
 
 /* The dot products q.b that select ground-truth candidates, 32 queries against n rows (a

@@ -110,3 +110,14 @@ def test_debug_entry_points_refuse_null_buffers_before_any_device_call():
     assert lib.bs_debug_filter(0, 64, None, 1, 4, lab, None, 0, None) == -1
     assert lib.bs_debug_fastscan(None, sig, 32, 1, None, None, 0, 32, 0.0, None, None, None, None, None) == -1
     assert b"null" in lib.bs_last_error() or b"must be given" in lib.bs_last_error()
+
+
+def test_groundtruth_splits_hold_rows():
+    """no row split of a ground-truth call is empty: one that publishes no value leaves the bound that
+    all splits share without effect, and the others waiting for it"""
+    from beam_search_collab_amd import search
+    for nq in (1, 4, 64, 136, 300, 500, 1000, 1500, 3000, 10000):
+        for n in list(range(1, 400, 37)) + [1000, 12000, 18812, 30000, 50000, 99999, 200000, 500000]:
+            for dim in (16, 40, 100, 128, 250):
+                nsplit, tiles, prime, _ = search.debug_gt_plan(n, nq, dim)
+                assert tiles >= 1 and (nsplit - 1) * tiles < (n + 31) // 32 and prime <= tiles, (n, nq, dim)
