@@ -66,8 +66,8 @@ def test_groundtruth_at_scale(gpu):
                                         (40000, 129, 128, 100), (30000, 31, 129, 10), (20001, 65, 192, 100),
                                         (50000, 1, 193, 128), (40003, 70, 256, 100)])
 def test_groundtruth_operand_sizes(gpu, n, nq, dim, k):
-    """the edges of the row tiles, query blocks, 16-dimension steps and operand instances (splits of
-    few tiles: no priming)"""
+    """the edges of the row tiles, query blocks, 16-dimension steps and operand instances, in splits of
+    few tiles"""
     base = host.gen_mixture(n, dim, 16, 0.0, 128.0, 12.0, 0.0, 21, 22)
     q = host.gen_mixture(nq, dim, 16, 0.0, 128.0, 12.0, 0.0, 21, 23)
     g = search.GPUGraph(base, np.zeros((n, 1), np.uint32))
@@ -276,3 +276,21 @@ def test_groundtruth_long_splits(gpu, n, nq, dim, primes):
     at = np.unique(np.concatenate([np.random.default_rng(nq).integers(0, nq, 150), np.arange(20), np.arange(nq - 20, nq)]))
     at = at[cert[at]]
     assert np.array_equal(raw[at], host.groundtruth(base, q[at], 100))
+
+
+@pytest.mark.parametrize("n,nq,dim", [(600, 3, 24), (1030, 100, 70), (2100, 500, 128), (12001, 500, 16), (9999, 70, 250),
+                                      (50000, 1000, 128)])
+def test_groundtruth_short_splits(gpu, n, nq, dim):
+    """splits of a few tiles prime their thresholds too, from up to half of their rows; also where the
+    query count leaves the last block nearly empty and a query has a NaN"""
+    nsplit, tiles, prime, _ = search.debug_gt_plan(n, nq, dim)
+    assert prime == max(min(tiles // 16, 64), min(tiles // 2, 4)) if nsplit >= 4 else prime == 0
+    base = host.gen_mixture(n, dim, 16, 0.0, 128.0, 12.0, 0.0, 95, 96)
+    q = host.gen_mixture(nq, dim, 16, 0.0, 128.0, 12.0, 0.0, 95, 97)
+    q[nq // 2, dim - 1] = np.nan
+    g = search.GPUGraph(base, np.zeros((n, 1), np.uint32))
+    raw = g.groundtruth(q, 60, exact_fallback=False)
+    assert (raw[nq // 2] == -1).all()
+    cert = (raw != -2).all(1) & (np.arange(nq) != nq // 2)
+    assert cert.sum() >= 0.95 * (nq - 1)
+    assert np.array_equal(raw[cert], host.groundtruth(base, q[cert], 60))
