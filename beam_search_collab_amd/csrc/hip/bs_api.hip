@@ -84,6 +84,11 @@ struct bs_index_s {
     char* pin = nullptr;
     hipEvent_t pin_done[COPY_T * COPY_SLOTS] = {};
     std::mutex copy_mutex;
+    // work buffer of the ground truth, kept between calls (bs_internal_gt_workspace); whoever holds
+    // the mutex uses it
+    char* gt_ws = nullptr;
+    size_t gt_bytes = 0;
+    std::mutex gt_mutex;
     // device staging of bs_search (host buffers): grows to the largest call, reused after
     void* d_stage = nullptr;
     size_t stage_bytes = 0;
@@ -196,6 +201,24 @@ int bs_internal_edges(bs_index ix, const uint32_t** edges) {
     return BS_OK;
 }
 void bs_internal_set_error(const std::string& msg) { g_err = msg; }
+std::mutex& bs_internal_gt_mutex(bs_index ix) { return ix->gt_mutex; }
+// The kept work buffer with at least `bytes`, under the mutex; bytes = 0 gives it back.
+hipError_t bs_internal_gt_workspace(bs_index ix, size_t bytes, char** ws) {
+    if (bytes == 0 || ix->gt_bytes < bytes) {
+        if (ix->gt_ws) (void)hipFree(ix->gt_ws);
+        ix->gt_ws = nullptr;
+        ix->gt_bytes = 0;
+        if (bytes == 0) return hipSuccess;
+        const hipError_t e = hipMalloc(reinterpret_cast<void**>(&ix->gt_ws), bytes);
+        if (e != hipSuccess) {
+            ix->gt_ws = nullptr;
+            return e;
+        }
+        ix->gt_bytes = bytes;
+    }
+    *ws = ix->gt_ws;
+    return hipSuccess;
+}
 hipError_t bs_internal_download(bs_index ix, void* dst, const void* src, size_t bytes) {
     return download(ix, dst, src, bytes);
 }
@@ -380,6 +403,11 @@ extern "C" int bs_index_attach_rabitq(bs_index ix, const uint32_t* codes, const 
         (void)hipFree(ix->d_signs);
         ix->d_signs = nullptr;
     }
+    {
+        // room for the records: the ground truth's kept work buffer goes first
+        const std::lock_guard<std::mutex> lock(ix->gt_mutex);
+        (void)bs_internal_gt_workspace(ix, 0, nullptr);
+    }
     if (hipMalloc(&ix->d_recs, ix->n * static_cast<size_t>(rw) * 4) != hipSuccess)
         return fail(BS_ENOMEM, "hipMalloc of the rabitq records failed");
     HIP_TRY(hipMalloc(&ix->d_signs, padded_dim * sizeof(float)));
@@ -452,6 +480,7 @@ extern "C" void bs_index_destroy(bs_index ix) {
     for (hipEvent_t v : ix->pin_done)
         if (v) (void)hipEventDestroy(v);
     if (ix->pin) (void)hipHostFree(ix->pin);
+    if (ix->gt_ws) (void)hipFree(ix->gt_ws);
     delete ix;
 }
 

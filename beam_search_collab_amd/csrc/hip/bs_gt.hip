@@ -22,11 +22,14 @@
 
 #include <algorithm>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <type_traits>
 #include <vector>
 
 int bs_internal_vecs(bs_index idx, const float** vecs, uint32_t* dstride);
+std::mutex& bs_internal_gt_mutex(bs_index idx);
+hipError_t bs_internal_gt_workspace(bs_index idx, size_t bytes, char** ws);
 void bs_internal_set_error(const std::string& msg);
 int bs_internal_exception();
 
@@ -975,6 +978,7 @@ Plan make_plan(uint64_t n, uint64_t nq, uint32_t dim, uint32_t cus, uint64_t pla
     return p;
 }
 constexpr uint64_t PLANE_BYTES = 1ull << 30;  // of planes at a time, where there is room; the lists carry over
+constexpr uint64_t KEEP_BYTES = 5ull << 28;   // the largest work buffer that an index keeps
 
 uint32_t device_cus() {
     int dev = 0, cus = 0;
@@ -1000,12 +1004,17 @@ int groundtruth(bs_index idx, const float* d_queries, uint64_t nq, uint32_t k, i
     if (nq == 0) return BS_OK;
     if (!d_queries || !d_out) return gfail(BS_EINVAL, "queries and output must be given");
     const uint32_t cus = device_cus();
-    // where the work buffer does not fit, planes of half as many rows at a time, down to 8 tiles
-    // (500k x 128, 10k queries: 9.7 ms with the 450 MB it takes, 9.6 with 200, 10.7 with 100, 51
-    // with 40)
+    // The work buffer is the index's, kept for its next call, where it is free and not over KEEP_BYTES;
+    // else this call's own.  (Memory given back is wiped by the driver at some 40 GB/s: one query on
+    // 500k x 128 took 0.75 ms, but 11.0 when repeated with 450 MB allocated and freed each time.)
+    // Where it does not fit, planes of half as many rows at a time, down to 8 tiles (500k x 128, 10k
+    // queries: 9.7 ms with the 450 MB it takes, 9.6 with 200, 10.7 with 100, 51 with 40).
+    std::unique_lock<std::mutex> lock(bs_internal_gt_mutex(idx), std::try_to_lock);
     Plan p = make_plan(n, nq, dim, cus, PLANE_BYTES);
     char* ws = nullptr;
-    while (p.need > ws_limit || hipMalloc(reinterpret_cast<void**>(&ws), p.need) != hipSuccess) {
+    auto keep = [&]() { return lock.owns_lock() && p.need <= KEEP_BYTES; };
+    while (p.need > ws_limit || (keep() ? bs_internal_gt_workspace(idx, p.need, &ws)
+                                        : hipMalloc(reinterpret_cast<void**>(&ws), p.need)) != hipSuccess) {
         (void)hipGetLastError();
         if (p.chunk <= 8) return gfail(BS_ENOMEM, "hipMalloc of the ground-truth work buffers failed");
         p = make_plan(n, nq, dim, cus, p.chunk / 2 * p.tile_bytes);
@@ -1050,7 +1059,8 @@ int groundtruth(bs_index idx, const float* d_queries, uint64_t nq, uint32_t k, i
     unsigned long long nu = 0;
     if (e == hipSuccess) e = hipMemcpyAsync(&nu, nunc, 8, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
-    (void)hipFree(ws);
+    if (e != hipSuccess) (void)hipStreamSynchronize(s);  // nothing may still write to the buffer
+    if (!keep()) (void)hipFree(ws);
     if (e != hipSuccess) return gfail(BS_EHIP, std::string("ground truth: ") + hipGetErrorString(e));
     if (n_uncertified) *n_uncertified = nu;
     return BS_OK;

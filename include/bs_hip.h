@@ -210,7 +210,9 @@ const char* bs_last_error(void);
  * certificate that no row outside its candidates can be among the k nearest.
  * out: nq*k int32 (-1 where fewer than k rows exist).  uncertified: nq bytes (1 = no
  * certificate: recompute that query, e.g. with bs_groundtruth) or NULL; n_uncertified
- * (nullable) gets their number.  Synchronous; allocates device work buffers. */
+ * (nullable) gets their number.  Synchronous; the index keeps its device work buffer (up to 1.25
+ * GiB) until it is destroyed or bs_index_attach_rabitq makes its records; a call that finds the
+ * buffer in use, by another thread, or needs more allocates its own. */
 int bs_index_groundtruth(bs_index idx, const float* queries, uint64_t nq, uint32_t k, int32_t* out,
                          uint8_t* uncertified, uint64_t* n_uncertified);
 /* The same on device buffers (queries nq*dim f32, out nq*k int32, uncertified nq u8 or

@@ -294,3 +294,42 @@ def test_groundtruth_short_splits(gpu, n, nq, dim):
     cert = (raw != -2).all(1) & (np.arange(nq) != nq // 2)
     assert cert.sum() >= 0.95 * (nq - 1)
     assert np.array_equal(raw[cert], host.groundtruth(base, q[cert], 60))
+
+
+def test_groundtruth_work_buffer_is_kept(gpu):
+    """repeated calls reuse the index's work buffer (allocated and freed each time it costs up to ten
+    times the call), for calls of any size, two threads at a time and on several streams; it is given
+    back with the index"""
+    import torch
+    from concurrent.futures import ThreadPoolExecutor
+    n, dim = 150_000, 128
+    base = host.gen_mixture(n, dim, 16, 0.0, 128.0, 12.0, 0.0, 98, 99)
+    q = host.gen_mixture(900, dim, 16, 0.0, 128.0, 12.0, 0.0, 98, 100)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    g = search.GPUGraph(base, np.zeros((n, 1), np.uint32))
+    before = torch.cuda.mem_get_info()[0]
+    parts = [q[:1], q[:70], q, q[5:6], q[100:400]]
+    want = [search.GPUGraph(base, np.zeros((n, 1), np.uint32)).groundtruth(x, 40, exact_fallback=False) for x in parts]
+    for x, w in zip(parts, want):
+        assert np.array_equal(g.groundtruth(x, 40, exact_fallback=False), w)
+    kept = before - torch.cuda.mem_get_info()[0]
+    assert kept >= 100 << 20, kept  # the operands of 150k x 128 in three planes
+    with ThreadPoolExecutor(2) as ex:
+        for got in (list(ex.map(lambda x: g.groundtruth(x, 40, exact_fallback=False), parts)) for _ in range(3)):
+            for r, w in zip(got, want):
+                assert np.array_equal(r, w)
+    s = torch.cuda.Stream()
+    dq = torch.from_numpy(q).cuda()
+    out = torch.empty(900, 40, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    import ctypes as C
+    from beam_search_collab_amd import _lib
+    nu = C.c_uint64(0)
+    assert _lib.hip().bs_index_groundtruth_device(g.handle, dq.data_ptr(), 900, 40, out.data_ptr(), None, s.cuda_stream,
+                                                  C.byref(nu)) == 0
+    cert = (want[2] != -2).all(1)
+    assert np.array_equal(out.cpu().numpy()[cert], want[2][cert])
+    assert np.array_equal(g.groundtruth(q, 40, exact_fallback=False), want[2])
+    g.close()
+    assert torch.cuda.mem_get_info()[0] >= before  # the rows are given back too (77 MB)
